@@ -28,6 +28,8 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <type_traits>
+
 #include "../../include/pfh.h"
 #include "pfh_device.h"
 #include "pfh_host.h"
@@ -58,8 +60,11 @@ struct Slot {
 };
 
 struct Smem {
-    pfh2d_step_args args;        // LDS copy for the out-of-line class paths
-    double red[kWaves * 8];
+    // LDS copy of the step arguments: the cell bodies make the few they use
+    // per row wave-uniform; held in scalar registers all 54 words would spill
+    pfh2d_step_args args;
+    double vel[kWaves * 8];      // wave sums before the velocity
+    double red[kWaves * 4];      // wave sums of the commit
     int ired[kWaves * 8];
     Slot slot[2];
     uint32_t csraw[2][48];       // CellState (192 B) of the next cell
@@ -68,20 +73,12 @@ struct Smem {
     int fm;                      // full-moment step (one in full_moment_every)
 };
 
-// The staged window, an LDS object of its own: the global-to-LDS window
-// copies write only here, so the compiler does not hold other LDS reads
-// (slots, partials) until those copies land.
-static __shared__ __attribute__((aligned(16))) float s_window[kPhiLdsFloats];
+// The scalars of the next cell run on lane 0 of wave 1 (wave 0 fetches and
+// commits).
+constexpr int kScalarsThread = kWave;
+constexpr int kFetchLanes = 48;                       // dwords of a CellState
 
-// Control lanes: the first 16 lanes of the workgroup (kControlLanes). No
-// LDS-path class gives them pixels (7x144, 5x176, 7x144 and 6x160 pixel
-// threads are at most 1008), so they fetch the next cell while the other
-// lanes compute. They sit in wave 0, which the SIMD issues first and which
-// therefore finishes its pixels first: the fetch's serial latency (the next
-// cell's scalars) then stays off the barrier's critical path, where it lay
-// in the last wave.
-constexpr int kLeaderLane = 0;                        // lane 0 of wave 0
-constexpr int kScalarsThread = kWave;                 // lane 0 of wave 1
+#define PFH_LDS __attribute__((address_space(3)))
 
 // threadIdx.x made opaque inside the persistent loop: without this, LICM
 // hoists every per-thread index and address of the cell body out of the loop
@@ -247,9 +244,10 @@ __device__ __noinline__ void cell_scalars(const ScalarArgs A, const pfh_cell_sta
 
 // Zero every tile pixel outside the destination window (class change). The
 // window itself is fully rewritten by the update, so no ordering is needed.
+template <int NT>
 __device__ void zero_outside_window(float* tile, int dwx, int dwy, int dtx0,
                                     int dty0) {
-    for (int i = opaque_tid(); i < kTileArea; i += kNT) {
+    for (int i = opaque_tid(); i < kTileArea; i += NT) {
         const int x = i % kTilePitch, y = i / kTilePitch;
         if (!((unsigned)(x - dtx0) < (unsigned)dwx &&
               (unsigned)(y - dty0) < (unsigned)dwy))
@@ -366,124 +364,124 @@ __device__ void record_observers(const pfh2d_step_args& A, int n, const Ctl& c, 
     }
 }
 
-// Velocity from the interaction integral (src/kernels.cu:300-342): wave
-// trees, then thread 0 adds the 16 wave sums in order and commits; with an
-// observer, the observer's sums ride in the same reduction.
-template <int kObs = 0>
-__device__ void reduce_velocity(const pfh2d_step_args& A, int n, Smem& sm,
-                                Ctl& c, double aIx, double aIy, ObsSums ob = ObsSums()) {
-    const int tid = opaque_tid();
-    const int lane = tid & (kWave - 1);
-    const int wave = tid / kWave;
-    aIx = wave_sum(aIx);
-    aIy = wave_sum(aIy);
-    if constexpr (kObs == 2) {
-        ob.bx = wave_sum(ob.bx);
-        ob.by = wave_sum(ob.by);
-        ob.gx = wave_sum(ob.gx);
-        ob.gy = wave_sum(ob.gy);
-        ob.kx = wave_sum(ob.kx);
-        ob.ky = wave_sum(ob.ky);
-    }
-    if (lane == 0) {
-        sm.red[wave * 8 + 0] = aIx;
-        sm.red[wave * 8 + 1] = aIy;
-        if constexpr (kObs == 2) {
-            double* r = sm.red + wave * 8;
-            r[2] = ob.bx; r[3] = ob.by;
-            r[4] = ob.gx; r[5] = ob.gy; r[6] = ob.kx; r[7] = ob.ky;
-        }
-    }
-    lds_barrier();
-    if (threadIdx.x == 0) {
-        double sIx = 0.0, sIy = 0.0;
-        for (int w = 0; w < kWaves; ++w) {
-            sIx += sm.red[w * 8 + 0];
-            sIy += sm.red[w * 8 + 1];
-        }
-        const double vxd = (double)c.vA * (double)c.cosp
-                         + (double)A.mot_coeff * sIx;
-        const double vyd = (double)c.vA * (double)c.sinp
-                         + (double)A.mot_coeff * sIy;
-        c.vx = (float)vxd;
-        c.vy = (float)vyd;
-        pfh_cell_state* cs = &A.cell[n];
-        cs->vx = (float)vxd;
-        cs->vy = (float)vyd;
-        cs->Ix = sIx;
-        cs->Iy = sIy;
-        if constexpr (kObs != 0) record_observers<kObs>(A, n, c, sIx, sIy, sm.red);
-    }
-    lds_barrier();
-}
-
-// Moments/support reduction and CellState commit (src/kernels.cu:542-591).
-struct NoHook {
-    __device__ void operator()() const {}
-};
-
-// after_partials runs on every thread once the wave partials are published
-// (every wave has finished the cell's pixel phases).
 __device__ __forceinline__ double readlane_f64(double v, int l) {
     const int lo = __builtin_amdgcn_readlane(__double2loint(v), l);
     const int hi = __builtin_amdgcn_readlane(__double2hiint(v), l);
     return __hiloint2double(hi, lo);
 }
 
+// The spatial observer's wave sums (slots 2-7 of a logical wave's row).
+__device__ __forceinline__ void publish_observer(Smem& sm, int lw, const ObsSums& ob) {
+    const double v[2] = {wave_sum4(ob.bx, ob.by, ob.gx, ob.gy),
+                         wave_sum4(ob.kx, ob.ky, ob.kx, ob.ky)};
+    const int lane = (int)threadIdx.x & (kWave - 1);
+    const int j = 2 * ((lane >> 4) & 1) + (lane >> 5);   // lanes 0, 32, 16, 48: 0..3
+    if ((lane & 15) == 0) {
+        sm.vel[lw * 8 + 2 + j] = v[0];
+        if (j < 2) sm.vel[lw * 8 + 6 + j] = v[1];
+    }
+}
+
+// The wave sums of the interaction integral of a wave's VW logical waves.
+template <int NW, int VW>
+__device__ __forceinline__ void publish_velocity(Smem& sm, int wave, const double (&aIx)[VW],
+                                                 const double (&aIy)[VW]) {
+    const double v = wave_sum4(aIx[0], aIy[0], aIx[VW - 1], aIy[VW - 1]);
+    const int lane = (int)threadIdx.x & (kWave - 1);
+    const int lw = wave + NW * (VW > 1 ? (lane >> 4) & 1 : 0);
+    if ((lane & 15) == 0 && (VW > 1 || (lane & 16) == 0)) sm.vel[lw * 8 + (lane >> 5)] = v;
+}
+
+// Velocity from the interaction integral (src/kernels.cu:300-342), after the
+// barrier that orders the wave sums: every wave adds the 16 wave sums in order
+// itself, x on its even lanes and y on its odd ones (no second barrier to hand
+// the result out); thread 0 and 1 store them, thread 0 runs the observer.
+template <int kObs = 0>
+__device__ __forceinline__ void finish_velocity(const pfh2d_step_args& A, int n, Smem& sm,
+                                                Ctl& c, float& vx, float& vy) {
+    const int lane = (int)threadIdx.x & (kWave - 1);
+    const int xy = lane & 1;
+    double s = 0.0;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) s += sm.vel[w * 8 + xy];
+    const double vd = (double)c.vA * (double)(xy ? c.sinp : c.cosp)
+                    + (double)A.mot_coeff * s;
+    const uint32_t v = __float_as_uint((float)vd);
+    vx = __uint_as_float(__builtin_amdgcn_readlane(v, 0));
+    vy = __uint_as_float(__builtin_amdgcn_readlane(v, 1));
+    if (threadIdx.x < 2) {
+        pfh_cell_state* cs = &A.cell[n];
+        (xy ? cs->vy : cs->vx) = __uint_as_float(v);
+        (xy ? cs->Iy : cs->Ix) = s;
+    }
+    if constexpr (kObs != 0) {
+        const double sIy = readlane_f64(s, 1);
+        if (threadIdx.x == 0) {
+            c.vx = vx;
+            c.vy = vy;
+            record_observers<kObs>(A, n, c, s, sIy, sm.vel);
+        }
+    }
+}
+
+// One logical wave's part of the commit: a lane's moments, support rows and
+// phi_max, and the wave's support columns.
+struct Part {
+    double V = 0.0, Cx = 0.0, Cy = 0.0;
+    int blox, bhix;                  // uniform
+    int bloy, bhiy, pmaxb;
+};
+__device__ __forceinline__ void publish_part(Smem& sm, int lw, const Part& p) {
+    const double m = wave_sum4(p.V, p.Cx, p.Cy, 0.0);
+    const int b = wave_tree4(-p.bloy, p.bhiy, p.pmaxb, 0,
+                             [](int x, int y) { return max(x, y); });
+    const int lane = (int)threadIdx.x & (kWave - 1);
+    const int j = 2 * ((lane >> 4) & 1) + (lane >> 5);   // lanes 0, 32, 16: 0..2
+    if ((lane & 15) == 0 && lane != 48) {
+        sm.red[lw * 4 + j] = m;
+        sm.ired[lw * 8 + 2 + j] = j == 0 ? -b : b;       // lo_y, hi_y, pmax
+    }
+    if (lane == 0) {
+        sm.ired[lw * 8 + 0] = p.blox;
+        sm.ired[lw * 8 + 1] = p.bhix;
+    }
+}
+
+// The CellState commit (src/kernels.cu:542-591), on wave 0 after the barrier
+// that orders publish_part: lanes 0-3 add the 16 wave partials of V, Cx, Cy
+// and the perimeter, lanes 4-8 reduce the support box and phi_max, each in
+// wave order from the same initial value. The other waves go on: the next
+// cell's first barrier lies between this and the next publish_part.
 // old_raw: the cell's CellState as fetched at the start of its turn (LDS),
 // for the counters that the commit advances.
-template <int CLS, class Hook = NoHook>
-__device__ void reduce_commit(const pfh2d_step_args& A, int n, Smem& sm,
-                              const Ctl& c, const uint32_t* old_raw,
-                              double aV, double aCx, double aCy, double aPer,
-                              int blox, int bhix, int bloy, int bhiy,
-                              int pmaxb, Hook after_partials = Hook()) {
-    const int tid = opaque_tid();
-    const int lane = tid & (kWave - 1);
-    const int wave = tid / kWave;
-    aV = wave_sum(aV);
-    aCx = wave_sum(aCx);
-    aCy = wave_sum(aCy);
-    aPer = wave_sum(aPer);
-    blox = wave_min(blox);
-    bhix = wave_max(bhix);
-    bloy = wave_min(bloy);
-    bhiy = wave_max(bhiy);
-    pmaxb = wave_max(pmaxb);
-    if (lane == 0) {
-        double* rw = sm.red + wave * 8;
-        rw[0] = aV; rw[1] = aCx; rw[2] = aCy; rw[3] = aPer;
-        int* iw = sm.ired + wave * 8;
-        iw[0] = blox; iw[1] = bhix; iw[2] = bloy; iw[3] = bhiy; iw[4] = pmaxb;
-    }
-    lds_barrier();
-    after_partials();
-    if (__builtin_amdgcn_readfirstlane(wave) == 0) {
-        // Lanes 0-3 add the 16 wave partials of V, Cx, Cy and the perimeter,
-        // lanes 4-8 reduce the support box and phi_max, each in wave order
-        // from the same initial value: the sums of one thread doing all nine.
-        double sl = 0.0;
-        int ml = 0;
-        if (lane < 4) {
-            for (int w = 0; w < kWaves; ++w) sl += sm.red[w * 8 + lane];
-        } else if (lane < 9) {
-            const int j = lane - 4;                  // 0 lo_x, 1 hi_x, 2 lo_y, 3 hi_y, 4 pmax
-            const bool is_max = (j & 1) != 0 || j == 4;
-            ml = j == 0 ? c.dwx : j == 2 ? c.dwy : j == 4 ? 0 : -1;
-            for (int w = 0; w < kWaves; ++w) {
-                const int v = sm.ired[w * 8 + j];
-                ml = is_max ? max(ml, v) : min(ml, v);
-            }
+template <int CLS>
+__device__ __forceinline__ void commit_cell(const pfh2d_step_args& A, int n, const Smem& sm,
+                                            const Ctl& c, const uint32_t* old_raw) {
+    const int lane = opaque_tid();
+    double sl = 0.0;
+    int ml = 0;
+    if (lane < 4) {
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) sl += sm.red[w * 4 + lane];
+    } else if (lane < 9) {
+        const int j = lane - 4;                  // 0 lo_x, 1 hi_x, 2 lo_y, 3 hi_y, 4 pmax
+        const bool is_max = (j & 1) != 0 || j == 4;
+        ml = j == 0 ? c.dwx : j == 2 ? c.dwy : j == 4 ? 0 : -1;
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) {
+            const int v = sm.ired[w * 8 + j];
+            ml = is_max ? max(ml, v) : min(ml, v);
         }
-        const double sV = readlane_f64(sl, 0), sCx = readlane_f64(sl, 1);
-        const double sCy = readlane_f64(sl, 2), sPer = readlane_f64(sl, 3);
-        const int Blox = __builtin_amdgcn_readlane(ml, 4);
-        const int Bhix = __builtin_amdgcn_readlane(ml, 5);
-        const int Bloy = __builtin_amdgcn_readlane(ml, 6);
-        const int Bhiy = __builtin_amdgcn_readlane(ml, 7);
-        const int Pmax = __builtin_amdgcn_readlane(ml, 8);
-        const pfh_cell_state* old = reinterpret_cast<const pfh_cell_state*>(old_raw);
-        if (lane == 0) {
+    }
+    const double sV = readlane_f64(sl, 0), sCx = readlane_f64(sl, 1);
+    const double sCy = readlane_f64(sl, 2), sPer = readlane_f64(sl, 3);
+    const int Blox = __builtin_amdgcn_readlane(ml, 4);
+    const int Bhix = __builtin_amdgcn_readlane(ml, 5);
+    const int Bloy = __builtin_amdgcn_readlane(ml, 6);
+    const int Bhiy = __builtin_amdgcn_readlane(ml, 7);
+    const int Pmax = __builtin_amdgcn_readlane(ml, 8);
+    const pfh_cell_state* old = reinterpret_cast<const pfh_cell_state*>(old_raw);
+    if (lane == 0) {
         pfh_cell_state* cs = &A.cell[n];
         cs->gx0 = c.gx0n;
         cs->gy0 = c.gy0n;
@@ -510,18 +508,12 @@ __device__ void reduce_commit(const pfh2d_step_args& A, int n, Smem& sm,
             if (c.no_margin || (c.dcls == kClassFallback && edge))
                 cs->reserved[1] = old->reserved[1] + 1u;
         }
-        }
     }
-    lds_barrier();
 }
 
 // The check step's commit: the cell's new window position and class (all its
-// consumer reads), between the same two barriers as reduce_commit.
-template <class Hook>
-__device__ void commit_position(const pfh2d_step_args& A, int n, Smem& sm, const Ctl& c,
-                                Hook after_partials) {
-    lds_barrier();
-    after_partials();
+// consumer reads).
+__device__ __forceinline__ void commit_position(const pfh2d_step_args& A, int n, const Ctl& c) {
     if (threadIdx.x == 0) {
         pfh_cell_state* cs = &A.cell[n];
         cs->gx0 = c.gx0n;
@@ -530,57 +522,53 @@ __device__ void commit_position(const pfh2d_step_args& A, int n, Smem& sm, const
         cs->cls_written[A.parity_out] = (uint8_t)c.dcls;
         A.cell_cls[n] = (uint8_t)c.dcls;
     }
-    lds_barrier();
 }
 
 // -------------------------------------------------------------------------
-// Next-cell fetch by the control lanes, in four stages so that each stage
-// only waits on a load issued one phase earlier:
+// Next-cell fetch by wave 0, in four stages so that each stage only waits on
+// a load issued one phase earlier:
 //   1 the queue ticket (atomic on the cursor);
 //   2 the cell id perm[ticket];
-//   3 its class and its 192-byte CellState (3 dwords per control lane);
+//   3 its class and its 192-byte CellState (a dword on each of 48 lanes);
 //   4 the CellState copy into LDS, the slot, and the per-cell scalars.
-// An unsupported class id is flagged here (reference dispatch default,
-// src/kernels.cu:1017-1021) and skipped by the dispatch.
+// A workgroup's first cell is its own index; the cursor hands out the cells
+// from gridDim.x on. An unsupported class id is flagged here (reference
+// dispatch default, src/kernels.cu:1017-1021) and skipped by the dispatch.
 // -------------------------------------------------------------------------
 struct Fetch {
     unsigned long long tk;
     int nn, cls;
-    uint32_t w0, w1, w2;
+    uint32_t w;
 };
 
 __device__ __forceinline__ void fetch1(const pfh2d_step_args& A, Fetch& f) {
-    if (((int)threadIdx.x & (kWave - 1)) == kLeaderLane)
-        f.tk = atomicAdd(A.cursor_use, 1ull);
+    if (threadIdx.x == 0) f.tk = atomicAdd(A.cursor_use, 1ull);
 }
 
 __device__ __forceinline__ void fetch2(const pfh2d_step_args& A, Fetch& f) {
-    const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)f.tk, kLeaderLane);
-    const uint32_t hi = __builtin_amdgcn_readlane((uint32_t)(f.tk >> 32), kLeaderLane);
-    const unsigned long long k = ((unsigned long long)hi << 32) | lo;
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)f.tk);
+    const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(f.tk >> 32));
+    const unsigned long long k =
+        (((unsigned long long)hi << 32) | lo) + (unsigned long long)gridDim.x;
     f.nn = k < (unsigned long long)A.N ? (int)A.perm[k] : -1;
 }
 
 __device__ __forceinline__ void fetch3(const pfh2d_step_args& A, Fetch& f) {
-    if (f.nn >= 0) {
-        const int j = ((int)threadIdx.x & (kWave - 1)) - kLeaderLane;
-        const uint32_t* w = reinterpret_cast<const uint32_t*>(A.cell + f.nn);
-        f.cls = (int)A.cell_cls[f.nn];
-        f.w0 = w[j];
-        f.w1 = w[j + 16];
-        f.w2 = w[j + 32];
+    const int nn = __builtin_amdgcn_readfirstlane(f.nn);
+    if (nn >= 0) {
+        const uint32_t* w = reinterpret_cast<const uint32_t*>(A.cell + nn);
+        f.cls = (int)A.cell_cls[nn];
+        f.w = w[min((int)threadIdx.x, kFetchLanes - 1)];
     }
 }
 
-// 4a (control lanes): the CellState copy, the id and the class into LDS.
+// 4a (wave 0): the CellState copy, the id and the class into LDS.
 __device__ __forceinline__ void fetch4a(const pfh2d_step_args& A, Smem& sm, Fetch& f,
                                         int which) {
-    const int j = ((int)threadIdx.x & (kWave - 1)) - kLeaderLane;
+    const int j = (int)threadIdx.x;
     int cls = -1;
     if (f.nn >= 0) {
-        sm.csraw[which][j] = f.w0;
-        sm.csraw[which][j + 16] = f.w1;
-        sm.csraw[which][j + 32] = f.w2;
+        if (j < kFetchLanes) sm.csraw[which][j] = f.w;
         cls = f.cls < kNumClasses ? f.cls : kNumClasses;
     }
     if (j == 0) {
@@ -613,44 +601,77 @@ __device__ __forceinline__ void fetch4b(const pfh2d_step_args& A, Smem& sm, int 
     }
 }
 
+// Stages 2-4 at once (wave 0), where nothing is there to hide them behind.
 template <bool kBatch>
-__device__ __forceinline__ void fetch4(const pfh2d_step_args& A, Smem& sm, Fetch& f,
-                                       int which, unsigned long long step) {
+__device__ __forceinline__ void fetch_rest(const pfh2d_step_args& A, Smem& sm, Fetch& f,
+                                           int which, unsigned long long step) {
+    fetch3(A, f);
     fetch4a(A, sm, f, which);
-    if (((int)threadIdx.x & (kWave - 1)) == kLeaderLane) fetch4b<kBatch>(A, sm, which, step);
+    if (threadIdx.x == 0) fetch4b<kBatch>(A, sm, which, step);
 }
-
 template <bool kBatch = false>
 __device__ __forceinline__ void fetch_all(const pfh2d_step_args& A, Smem& sm, int which,
                                           unsigned long long step) {
     Fetch f;
     fetch1(A, f);
     fetch2(A, f);
-    fetch3(A, f);
-    fetch4<kBatch>(A, sm, f, which, step);
+    fetch_rest<kBatch>(A, sm, f, which, step);
+}
+// The workgroup's first cell.
+template <bool kBatch = false>
+__device__ __forceinline__ void fetch_first(const pfh2d_step_args& A, Smem& sm,
+                                            unsigned long long step) {
+    Fetch f;
+    f.nn = (int)blockIdx.x < A.N ? (int)A.perm[blockIdx.x] : -1;
+    fetch_rest<kBatch>(A, sm, f, 0, step);
 }
 
 // -------------------------------------------------------------------------
-// LDS path: classes 0-3.
+// Column-walk path: classes 0-3.
 //
-// LDS holds the window with a one-pixel zero ring: row r (= y + 1, y in
-// [-1, WY]) starts at r*PX with four pad floats (the last one is column -1)
-// and column WX falls on the next row's first pad, so the stencil never needs
-// an edge test. Thread (band, x) walks rows y0..y0+RB-1 of column x with a
-// rolling 3x3 neighbourhood: three LDS reads per row.
+// Work split. A cell's pixels belong to 1024 logical threads (16 logical
+// waves): thread t owns rows y0..y0+RB-1 of one column, x = (t - 16) % WX,
+// band = (t - 16) / WX; the order of every fp64 sum follows that split. A
+// workgroup has NW = 8 or 16 waves, and each wave walks 16 / NW logical
+// waves one after the other. With NW = 8 two workgroups, two independent
+// cells, share a compute unit, so that one cell's loads, reductions, scalars
+// and barriers run under the other's arithmetic.
+//
+// Data path. A wave reads only the 64 columns of its logical wave (at most
+// two runs of columns, in adjacent bands) and one halo column on each side:
+// three rows are 57 groups of 16 B, one buffer load per lane, that goes
+// through registers into rows private to the wave in LDS. No barrier is
+// needed between staging and stencil. Groups outside the window (the halo of
+// an edge column, rows past the window, the gap group between the two runs,
+// columns of logical threads that own nothing) are past the descriptor's
+// end, for which the buffer load returns zeros: the stencil has no edge test
+// and a lane that owns nothing computes exact zeros. The rows of the last
+// logical wave stay in LDS for the update; those of the other are read again
+// (from L2).
+//
+// The S word of a pixel is requested at the start of the cell into the
+// register that later holds the pixel's passive right-hand side, and the
+// scatter's returned word replaces that right-hand side in the update.
 //
 // Exact shortcuts (phi never takes the value -0, so adding or subtracting a
 // signed zero changes no sum or right-hand side):
 //   - a wave-row where no lane overlaps another cell (S_other == 0) skips the
-//     repulsion term and the fp64 interaction-integral terms, all zero;
-//   - a wave-row where every lane has c == passive == gx == gy == 0 has
-//     phi_next == +0 exactly and only stores the zeros.
+//     repulsion term and the fp64 interaction-integral terms, all zero.
 // -------------------------------------------------------------------------
+constexpr int kRowGroupsW = 19;                        // 16 groups, two halos, one gap
+constexpr int kRowFloats = 4 * kRowGroupsW;
+constexpr int kChunkRows = 3;                          // rows per buffer load
+constexpr int kChunkFloats = kChunkRows * kRowFloats;
+constexpr int kChunkLanes = kChunkRows * kRowGroupsW;  // 57 of 64
+constexpr int kChunkSlots = 10;                        // chunks a wave holds in LDS
+constexpr int kChunkDepth = 3;                         // chunk loads in flight
+template <int NW> constexpr int kWindowFloats = NW * kChunkSlots * kChunkFloats;
+
 struct Roll {
     float sW, sC, sE, cW, cC, cE, nW, nC, nE;
 };
 
-__device__ __forceinline__ void load_row(const float* p, float& w, float& c, float& e) {
+__device__ __forceinline__ void load_row(const PFH_LDS float* p, float& w, float& c, float& e) {
     w = p[-1];
     c = p[0];
     e = p[1];
@@ -696,15 +717,8 @@ __device__ __forceinline__ float euler_update(float cC, float gxv, float gyv, fl
     return fmaf(dt, fmaf(mrel, pas, -adv), cC);
 }
 
-__device__ __forceinline__ float s_other_of(uint32_t qS, float c, uint32_t& negc) {
-    const uint32_t qc = q_of(c);
-    const bool neg = qS < qc;
-    negc += neg ? 2u : 0u;          // the reference evaluates S_other once per pass
-    return neg ? 0.0f : (float)(qS - qc) * kQInv;
-}
-
-// The same, counting this lane's negative differences once each (the
-// subtraction's borrow is added in with carry).
+// S_other, counting this lane's negative differences (the subtraction's
+// borrow is added in with carry).
 __device__ __forceinline__ float s_other_lane(uint32_t qS, float c, uint32_t& neg1) {
     const uint32_t qc = q_of(c);
     const bool neg = qS < qc;
@@ -712,34 +726,13 @@ __device__ __forceinline__ float s_other_lane(uint32_t qS, float c, uint32_t& ne
     return neg ? 0.0f : (float)(qS - qc) * kQInv;
 }
 
-// Class-0 window prefetch: rows [r0, r1) of cell nn's class-0 window,
-// copied from HBM straight into LDS (global-to-LDS loads, no registers), row
-// r to dst0 + (r - r0) * PX. Waves W0..W0+NW-1 take rows r0 + (w - W0) + NW j;
-// one instruction moves one 576 B row with 36 lanes of 16 B. Wave 0 (thread
-// 0 commits the cell, the control lanes fetch) is never among them, so that
-// none of its own memory waits has to wait for the copies. A wave's copies
-// are complete when its vmcnt has passed them; LDS release fences (and so
-// every barrier here) wait for them too.
-template <int W0 = 1, int NW = kWaves - 1>
-__device__ __forceinline__ void copy_rows0(const pfh2d_step_args& A, int nn, float* dst0,
-                                           int r0, int r1) {
-    using G = Staged<0>;
-    const int lane = (int)threadIdx.x & (kWave - 1);
-    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);
-    const PFH_GLOBAL float* src = gptr(A.phi_in) + (size_t)nn * kTileArea
-                                + (size_t)G::TY0 * kTilePitch + G::TX0 + 4 * lane;
-    if (wave >= W0 && wave < W0 + NW && lane < G::NCH) {
-        for (int r = r0 + wave - W0; r < r1; r += NW)
-            __builtin_amdgcn_global_load_lds(
-                (const PFH_GLOBAL void*)(src + (size_t)r * kTilePitch),
-                (__attribute__((address_space(3))) void*)(dst0 + (r - r0) * G::PX),
-                16, 0, 0);
-    }
+// mask = 2 mask + (v > kSupportEps): the support rows of a column, one bit a
+// row, the compare's bit shifted in by the add's carry.
+__device__ __forceinline__ void push_support(uint32_t& mask, float v) {
+    asm("v_cmp_gt_f32_e32 vcc, %1, %2\n\tv_addc_co_u32_e32 %0, vcc, %0, %0, vcc"
+        : "+v"(mask) : "v"(v), "v"(kSupportEps) : "vcc");
 }
 
-// kCheck: a check step (the surrogate's acceptance field), which needs the
-// new field and the cell's window position only: no scatter, moments,
-// support, flags or perimeter, and a commit of the position alone.
 // The cell's domain: the launch's own population or, in a batched step,
 // its replica's side, S pitch and S offset, made wave-uniform.
 struct Dom {
@@ -754,439 +747,536 @@ __device__ __forceinline__ Dom cell_dom(const pfh2d_step_args& A, const Slot& c)
         return {__builtin_amdgcn_readfirstlane(c.L), __builtin_amdgcn_readfirstlane(c.P),
                 ((unsigned long long)hi << 32) | lo};
     } else {
-        return {A.L, A.P, 0ull};
+        return {__builtin_amdgcn_readfirstlane(A.L), __builtin_amdgcn_readfirstlane(A.P), 0ull};
     }
 }
 
-template <int CLS, bool kCheck = false, bool kBatch = false, int kObs = 0>
-__device__ void cell_staged(const pfh2d_step_args& A, int n,
-                            unsigned long long step, Smem& sm, Ctl& c, int nxt,
-                            int& pre, int& pslot, int* ring = nullptr) {
+// Wave-uniform copies of values read from LDS (the out-of-line paths' arguments,
+// the cell's scalars): they then live in scalar registers.
+template <class T>
+__device__ __forceinline__ T* uni_ptr(T* p) {
+    const uint64_t v = (uint64_t)p;
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
+    const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+    return (T*)(((uint64_t)hi << 32) | lo);
+}
+__device__ __forceinline__ float uni(float v) {
+    return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(v)));
+}
+
+// Raw buffer descriptors: a byte offset at or past the end reads zeros and
+// stores nothing. One covers the rows of a tile that a window occupies, so
+// rows above and below the window need no test; kOffNone is past every one.
+constexpr uint32_t kOffNone = 0x80000000u;
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc_of(const void* base, uint32_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, (int)bytes, 0x00020000);
+}
+constexpr uint32_t kTileRow = 4u * kTilePitch;         // bytes of a tile row
+
+// phi_next of one source pixel from global memory, bit for bit as the walk
+// computes it (the perimeter of a recentred cell needs values that the
+// destination window does not hold).
+struct NextArgs {
+    const float* win;            // window origin in the input tile
+    const uint32_t* S;
+    int WX, WY, L, P, gx0, gy0;
+    float gam, dwC, volC, repC, vx, vy, mrel, dt;
+};
+__device__ __noinline__ float next_at(const NextArgs a, int x, int y) {
+    auto f = [&](int xx, int yy) -> float {
+        return (unsigned)xx < (unsigned)a.WX && (unsigned)yy < (unsigned)a.WY
+                   ? a.win[(size_t)yy * kTilePitch + xx] : 0.0f;
+    };
+    const float cC = f(x, y), cE = f(x + 1, y), cW = f(x - 1, y);
+    const float nC = f(x, y + 1), sC = f(x, y - 1);
+    uint32_t neg = 0u;
+    const float So = s_other_lane(
+        a.S[(size_t)wrapi(a.gy0 + y, a.L) * a.P + wrapi(a.gx0 + x, a.L)], cC, neg);
+    const float pas = with_repulsion(
+        passive_head_of(nC, sC, cE, cW, f(x + 1, y + 1), f(x - 1, y + 1), f(x + 1, y - 1),
+                        f(x - 1, y - 1), cC, a.gam, a.dwC, a.volC), a.repC, cC, So);
+    return euler_update(cC, 0.5f * (cE - cW), 0.5f * (nC - sC), pas, a.vx, a.vy, a.mrel, a.dt);
+}
+
+// One lane's share of logical wave lw: its column as a pixel, and the 16 B
+// group it stages as a loader. Recomputed per pass (a few instructions on the
+// lane index and scalars) rather than held.
+template <int CLS>
+struct Share {
     using G = Staged<CLS>;
-    constexpr int WX = G::WX, WY = G::WY, TX0 = G::TX0, TY0 = G::TY0;
-    constexpr int PX = G::PX;
-    constexpr int RB = G::RB, NCH = G::NCH, NCHUNK = G::NCHUNK, KCH = G::KCH;
-    constexpr bool kExact = G::NB * RB == WY;   // no partial band
+    int lane, x0, split, band0;            // all but lane are uniform
+    __device__ __forceinline__ explicit Share(int lw) {
+        asm volatile("" : "+s"(lw));
+        lane = opaque_tid() & (kWave - 1);
+        const int pv = lw * kWave - kControlLanes + G::WX;   // >= 0
+        const int row = pv / G::WX;
+        band0 = row - 1;
+        x0 = pv - row * G::WX;                               // first run's first column
+        split = min(kWave, G::WX - x0);                      // lanes of the first run
+    }
+    __device__ __forceinline__ bool second() const { return lane >= split; }
+    __device__ __forceinline__ int x() const { return lane + (second() ? -split : x0); }
+    __device__ __forceinline__ int band() const { return band0 + (second() ? 1 : 0); }
+    __device__ __forceinline__ bool active() const { return (unsigned)band() < (unsigned)G::NB; }
+    // first row; band 0's or the last one's where the lane owns nothing
+    __device__ __forceinline__ int y0() const {
+        return min(max(band(), 0), G::NB - 1) * G::RB;
+    }
+    // the lane's column in a staged row (floats)
+    __device__ __forceinline__ int col() const { return 4 + lane + (second() ? 4 : 0); }
+    // byte offset, from the window's first row, of the lane's group in the
+    // first chunk (rows -1, 0, 1 of the band)
+    __device__ __forceinline__ uint32_t group() const {
+        const int r = lane / kRowGroupsW, q = lane - r * kRowGroupsW;
+        const int n1 = split / 4;
+        const bool two = q > n1 + 1;
+        const int xg = 4 * (q - 1) + (two ? -4 * (n1 + 1) : x0);
+        const int bg = band0 + (two ? 1 : 0);
+        const bool ok = lane < kChunkLanes && (unsigned)xg < (unsigned)G::WX &&
+                        (unsigned)bg < (unsigned)G::NB && !(two && split == kWave);
+        const int off = (bg * G::RB + r - 1) * (int)kTileRow + 4 * (G::TX0 + xg);
+        return ok ? (uint32_t)off : kOffNone;
+    }
+};
+
+// kCheck: a check step (the surrogate's acceptance field), which needs the
+// new field and the cell's window position only: no scatter, moments,
+// support, flags or perimeter, and a commit of the position alone.
+template <int CLS, int NW, bool kCheck = false, bool kBatch = false, int kObs = 0>
+__device__ void cell_walk(const pfh2d_step_args& A, int n, unsigned long long step, Smem& sm,
+                          PFH_LDS float* win, Ctl& c, int nxt) {
+    using G = Staged<CLS>;
+    constexpr int WX = G::WX, WY = G::WY, TX0 = G::TX0, TY0 = G::TY0, RB = G::RB;
+    constexpr int NT = NW * kWave, VW = kWaves / NW;
+    constexpr int NCK = (RB + 2 + kChunkRows - 1) / kChunkRows;
+    constexpr bool kKeep = NCK <= kChunkSlots;   // the last pass's rows stay for the update
+    // chunk loads in order: the passes of phase A, then those of phase B that
+    // find their rows gone
+    constexpr int kLoads = (VW + (kKeep ? VW - 1 : VW)) * NCK;
     const int tid = opaque_tid();
-    const int pix = tid - kControlLanes;                 // pixel thread index
-    const bool control = pix < 0;
-    const int x = control ? 0 : pix % WX;
-    const int band = control ? 0 : pix / WX;
-    const bool active = !control && band < G::NB;
-    const int y0 = band * RB;
+    const int lane = tid & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
     Fetch nf;
-    if (control) fetch1(A, nf);
+    if (wave == 0) fetch1(A, nf);
     const Dom dm = cell_dom<kBatch>(A, sm.slot[nxt ^ 1]);
     const int L = dm.L, P = dm.P;
-    // the origin from the LDS copy of the CellState: a global load here would
-    // make the S loads wait for every load issued before it
-    const int gx0 = c.gx0;
-    const int gy0 = c.gy0;
-    float* phi_s = s_window;
-    // The window in LDS: class 0 in its two pieces (piece 1 in slot pslot),
-    // the other classes whole. rowp(r) is the start of row r's data; cbw is
-    // this thread's column at row y0 - 1 (a band's rows are all in one piece).
-    float* base1 = phi_s;
-    float* base2 = phi_s;
-    if constexpr (CLS == 0) {
-        base1 = phi_s + pslot * Split0::P1_FLOATS;
-        base2 = phi_s + 2 * Split0::P1_FLOATS;
-    }
-    auto rowp = [&](int r) -> float* {
-        if constexpr (CLS == 0)
-            return r <= Split0::P2_R0 ? base1 + (r + 1) * PX + 4
-                                      : base2 + (r - Split0::P2_R0) * PX + 4;
-        else
-            return phi_s + (r + 1) * PX + 4;
-    };
-    float* cbw = base1 + y0 * PX + 4 + x;
-    if constexpr (CLS == 0) {
-        if (band >= Split0::KB) cbw = base2 + (y0 - 1 - Split0::P2_R0) * PX + 4 + x;
-    }
-    const int gx = (gx0 + x < L) ? gx0 + x : gx0 + x - L;
-    // k is a compile-time row index: rows below RFULL exist in every band, so
-    // only the last band's tail rows are tested at run time.
-    auto row_ok = [&](int k) { return kExact || k < G::RFULL || y0 + k < WY; };
-
-    // Window rows of phi in flight (16 B each) ...
-    const PFH_GLOBAL float* tin = gptr(A.phi_in) + (size_t)n * kTileArea;
-    const PFH_GLOBAL uint32_t* S_rd = gptr(A.S_rd + dm.off);
-    const bool have = CLS == 0 && pre != 0;     // window already copied into LDS
-    f32x4 ph[KCH];
-    if (!have) {
-#pragma unroll
-        for (int k = 0; k < KCH; ++k) {
-            const int u = tid + k * kNT;
-            if (u < NCHUNK) {
-                const int r = u / NCH, c4 = u - (u / NCH) * NCH;
-                ph[k] = *reinterpret_cast<const PFH_GLOBAL f32x4*>(
-                    tin + (size_t)(TY0 + r) * kTilePitch + TX0 + 4 * c4);
-            }
-        }
-    }
-    // ... and this thread's column of the S window. S is addressed by a
-    // 32-bit byte offset (4 P L < 2^32, checked at launch) that advances one
-    // row pitch per row and wraps once at the domain edge.
+    const int gx0 = __builtin_amdgcn_readfirstlane(c.gx0);
+    const int gy0 = __builtin_amdgcn_readfirstlane(c.gy0);
+    PFH_LDS float* const rows = win + wave * (kChunkSlots * kChunkFloats);
+    const __amdgpu_buffer_rsrc_t tin =
+        rsrc_of(uni_ptr(A.phi_in) + (size_t)n * kTileArea + (size_t)TY0 * kTilePitch,
+                WY * kTileRow);
     const uint32_t s_pitch = 4u * (uint32_t)P, s_wrap = s_pitch * (uint32_t)L;
-    uint32_t s_off0;
-    {
-        int gy = gy0 + y0;
+    const __amdgpu_buffer_rsrc_t s_in = rsrc_of(uni_ptr(A.S_rd) + dm.off, s_wrap);
+    // no row of the walk wraps around the domain (rows past the window included)
+    const bool flat = gy0 + G::NB * RB <= L;
+
+    auto lw_of = [&](int v) { return wave + NW * v; };
+    // S byte offset of a lane's first row: 32 bits (4 P L < 2^32, checked at
+    // launch); a wrapping column advances it row by row
+    auto s_off_of = [&](int x, int y0) -> uint32_t {
+        int gx = gx0 + x, gy = gy0 + y0;
+        if (gx >= L) gx -= L;
         if (gy >= L) gy -= L;
-        s_off0 = (uint32_t)gy * s_pitch + 4u * (uint32_t)gx;
-    }
-    // Every lane issues all RB loads (control lanes and rows past the window
-    // read in-bounds S words that no row uses): with no branch around a load,
-    // each row of phase A waits only for its own word.
-    auto load_qs = [&](uint32_t (&qS)[RB]) {
-        uint32_t off = s_off0;
-#pragma unroll
-        for (int k = 0; k < RB; ++k) {
-            qS[k] = *reinterpret_cast<const PFH_GLOBAL uint32_t*>(
-                reinterpret_cast<const PFH_GLOBAL char*>(S_rd) + off);
-            off += s_pitch;
-            if (off >= s_wrap) off -= s_wrap;
-            asm volatile("" : "+v"(off));   // one live offset, not one per row
-        }
+        return (uint32_t)gy * s_pitch + 4u * (uint32_t)gx;
     };
-    uint32_t qS[RB];
-    load_qs(qS);
-    if (have) {
-        // This wave's global-to-LDS copies, issued during the previous cell,
-        // are older than the RB loads just issued: retire all but those.
-        static_assert(RB <= 63, "vmcnt is 6 bits");
-        asm volatile("s_waitcnt vmcnt(%0)" :: "n"(RB) : "memory");
-    } else {
+    auto s_next = [&](uint32_t off) -> uint32_t {
+        const uint32_t o = off + s_pitch;
+        return min(o, o - s_wrap);               // o - s_wrap is huge below the wrap
+    };
+
+    // ---- chunk pipeline ----
+    u32x4 pf[kChunkDepth];
+    uint32_t group[VW];                          // the lane's group in each pass
 #pragma unroll
-        for (int k = 0; k < KCH; ++k) {
-            const int u = tid + k * kNT;
-            if (u < NCHUNK) {
-                const int r = u / NCH, c4 = u - (u / NCH) * NCH;
-                if constexpr (CLS == 0) {             // rows P2_R0, R1 go to both pieces
-                    if (r <= Split0::R1)
-                        *reinterpret_cast<f32x4*>(base1 + (r + 1) * PX + 4 + 4 * c4) = ph[k];
-                    if (r >= Split0::P2_R0)
-                        *reinterpret_cast<f32x4*>(base2 + (r - Split0::P2_R0) * PX + 4 + 4 * c4) = ph[k];
-                } else {
-                    *reinterpret_cast<f32x4*>(phi_s + (r + 1) * PX + 4 + 4 * c4) = ph[k];
-                }
+    for (int v = 0; v < VW; ++v) group[v] = Share<CLS>(lw_of(v)).group();
+    // logical wave of chunk load j
+    auto v_of = [&](int j) {
+        const int p = j / NCK;
+        return p < VW ? p : (kKeep ? VW - 2 : VW - 1) - (p - VW);
+    };
+    auto issue = [&](int j) {                    // chunk j of the load order
+        pf[j % kChunkDepth] = __builtin_amdgcn_raw_buffer_load_b128(
+            tin, (int)(group[v_of(j)] + (uint32_t)(j % NCK) * (kChunkRows * kTileRow)), 0, 0);
+    };
+    auto chunk_at = [&](int j) -> PFH_LDS float* {
+        return rows + (j % kChunkSlots) * kChunkFloats;
+    };
+    auto advance = [&](int j) {                  // chunk j into LDS, j + depth requested
+        if (lane < kChunkLanes)
+            *reinterpret_cast<PFH_LDS u32x4*>(chunk_at(j) + 4 * lane) = pf[j % kChunkDepth];
+        __builtin_amdgcn_wave_barrier();
+        if (j + kChunkDepth < kLoads) issue(j + kChunkDepth);
+    };
+
+#pragma unroll
+    for (int j = 0; j < kChunkDepth; ++j) issue(j);
+    uint32_t qS[VW][RB];
+#pragma unroll
+    for (int v = 0; v < VW; ++v) {
+        const Share<CLS> g(lw_of(v));
+        uint32_t off = s_off_of(g.x(), g.y0());
+        if (flat) {
+            uint32_t so = 0u;
+#pragma unroll
+            for (int k = 0; k < RB; ++k) {
+                qS[v][k] = __builtin_amdgcn_raw_buffer_load_b32(s_in, (int)off, (int)so, 0);
+                so += s_pitch;
+                asm volatile("" : "+s"(so));     // one live offset, not one per row
+            }
+        } else {
+#pragma unroll
+            for (int k = 0; k < RB; ++k) {
+                qS[v][k] = __builtin_amdgcn_raw_buffer_load_b32(s_in, (int)off, 0, 0);
+                off = s_next(off);
             }
         }
-    }
-    // zero ring: the pads of every row (column -1 and column WX) and rows -1, WY
-    if constexpr (CLS == 0) {
-        // The class-0 layout's ring is written by nothing but this set-up
-        // (copies, staging and the perimeter pass write data columns only):
-        // both piece-1 slots and piece 2 are set up once, and again after a
-        // cell of another class has used the LDS.
-        if (*ring == 0) {
-            constexpr int n1 = (Split0::P1_ROWS + 1) * 4, n2 = (Split0::P2_ROWS + 1) * 4;
-            float* const b2 = phi_s + 2 * Split0::P1_FLOATS;
-            for (int i = tid; i < 2 * n1 + n2 + 3 * WX; i += kNT) {
-                if (i < 2 * n1) {
-                    const int sl = i >= n1 ? 1 : 0, j = i - sl * n1;
-                    phi_s[sl * Split0::P1_FLOATS + (j >> 2) * PX + (j & 3)] = 0.0f;
-                } else if (i < 2 * n1 + n2) {
-                    const int j = i - 2 * n1;
-                    b2[(j >> 2) * PX + (j & 3)] = 0.0f;
-                } else {
-                    const int j = i - 2 * n1 - n2;
-                    if (j < 2 * WX) {
-                        const int sl = j >= WX ? 1 : 0;
-                        phi_s[sl * Split0::P1_FLOATS + 4 + (j - sl * WX)] = 0.0f;
-                    } else {
-                        b2[(WY - Split0::P2_R0) * PX + 4 + (j - 2 * WX)] = 0.0f;
-                    }
-                }
-            }
-            *ring = 1;
-        }
-    } else {
-        for (int i = tid; i < (WY + 3) * 4 + 2 * WX; i += kNT) {
-            if (i < (WY + 3) * 4) phi_s[(i >> 2) * PX + (i & 3)] = 0.0f;
-            else {
-                const int j = i - (WY + 3) * 4;
-                phi_s[(j < WX ? 0 : (WY + 1) * PX - WX) + 4 + j] = 0.0f;
-            }
-        }
-    }
-    lds_barrier();
-    // The id and then the CellState of the next cell: wave 0 waits for them
-    // here, while the other waves of its SIMD start phase A.
-    if (control) {
-        fetch2(A, nf);
-        fetch3(A, nf);
     }
 
-    const float gam = c.gam, dwC = c.dwC, volC = c.volC;
-    const float repC = A.rep_coeff;
+    const float gam = uni(c.gam), dwC = uni(c.dwC), volC = uni(c.volC);
+    const float repC = uni(A.rep_coeff);
     if (c.zero_tile)
-        zero_outside_window(A.phi_out + (size_t)n * kTileArea, c.dwx, c.dwy,
-                            c.dtx0, c.dty0);
+        zero_outside_window<NT>(A.phi_out + (size_t)n * kTileArea, c.dwx, c.dwy,
+                                c.dtx0, c.dty0);
 
     // ---- phase A: interaction integral and the held passive RHS ----
-    float pas[RB];
-    double aIx = 0.0, aIy = 0.0;
-    ObsSums ob;
-    if (active) {
-        uint32_t neg1 = 0u;
+    float pas[VW][RB];
+    double aIx[VW], aIy[VW];
+    uint32_t neg1 = 0u;
+#pragma unroll
+    for (int v = 0; v < VW; ++v) {
+        const int q0 = v * NCK;
+        const Share<CLS> g(lw_of(v));
+        const int col = g.col();
+        auto row = [&](int kk) -> const PFH_LDS float* {
+            return chunk_at(q0 + kk / kChunkRows) + (kk % kChunkRows) * kRowFloats + col;
+        };
+        aIx[v] = aIy[v] = 0.0;
+        ObsSums ob;
+        advance(q0);
+        if (NCK > 1) advance(q0 + 1);
         Roll q;
-        load_row(cbw, q.sW, q.sC, q.sE);
-        load_row(cbw + PX, q.cW, q.cC, q.cE);
+        float fW, fC, fE;                        // the row after the next, on its way
+        load_row(row(0), q.sW, q.sC, q.sE);
+        load_row(row(1), q.cW, q.cC, q.cE);
+        load_row(row(2), fW, fC, fE);
 #pragma unroll
         for (int k = 0; k < RB; ++k) {
-            pas[k] = 0.0f;
-            if (row_ok(k)) {
-                load_row(cbw + (k + 2) * PX, q.nW, q.nC, q.nE);
-                const float head = passive_head(q, gam, dwC, volC);
-                const float So = s_other_lane(qS[k], q.cC, neg1);
-                if constexpr (kObs == 2)
-                    observe_pixel(ob, x, y0 + k, q.cC, q.cE, q.cW, q.nC, q.sC, q.nE, q.nW,
-                                  q.sE, q.sW, So, gam, dwC, repC, c.og2iv, c.ocx, c.ocy);
-                if (wave_any(So != 0.0f)) {
-                    pas[k] = with_repulsion(head, repC, q.cC, So);
-                    const float gxv = 0.5f * (q.cE - q.cW);
-                    const float gyv = 0.5f * (q.nC - q.sC);
-                    aIx += (double)(q.cC * gxv * So);
-                    aIy += (double)(q.cC * gyv * So);
-                } else {
-                    pas[k] = head;
-                }
-                q.sW = q.cW; q.sC = q.cC; q.sE = q.cE;
-                q.cW = q.nW; q.cC = q.nC; q.cE = q.nE;
+            q.nW = fW; q.nC = fC; q.nE = fE;
+            if (k + 1 < RB) load_row(row(k + 3), fW, fC, fE);
+            const float head = passive_head(q, gam, dwC, volC);
+            const float So = s_other_lane(qS[v][k], q.cC, neg1);
+            if constexpr (kObs == 2)
+                observe_pixel(ob, g.x(), g.y0() + k, q.cC, q.cE, q.cW, q.nC, q.sC, q.nE, q.nW,
+                              q.sE, q.sW, So, gam, dwC, repC, c.og2iv, c.ocx, c.ocy);
+            if (wave_any(So != 0.0f)) {
+                pas[v][k] = with_repulsion(head, repC, q.cC, So);
+                const float gxv = 0.5f * (q.cE - q.cW);
+                const float gyv = 0.5f * (q.nC - q.sC);
+                aIx[v] += (double)(q.cC * gxv * So);
+                aIy[v] += (double)(q.cC * gyv * So);
+            } else {
+                pas[v][k] = head;
             }
+            q.sW = q.cW; q.sC = q.cC; q.sE = q.cE;
+            q.cW = q.nW; q.cC = q.nC; q.cE = q.nE;
+            if (k % kChunkRows == kChunkRows - 1 && (k + 4) / kChunkRows < NCK)
+                advance(q0 + (k + 4) / kChunkRows);
+            if (v == 0 && k == RB / 3 && wave == 0) fetch2(A, nf);
+            if (v == 0 && k == 2 * RB / 3 && wave == 0) fetch3(A, nf);
             // One row per scheduling region keeps the walk's register
             // footprint at one row instead of the whole column.
             __builtin_amdgcn_sched_barrier(0);
         }
-        // two events per negative pixel (the reference evaluates S_other once
-        // per pass)
-        if (neg1) flag_add(A.flags, PFH_FLAG_S_NEGATIVE, 2u * neg1);
+        if constexpr (kObs == 2) publish_observer(sm, lw_of(v), ob);
     }
-
-    if (control) fetch4a(A, sm, nf, nxt);       // visible after the next barrier
-    reduce_velocity<kObs>(A, n, sm, c, aIx, aIy, ob);
-    // A class-0 cell next in the queue gets its window copied in ahead:
-    // piece 1 into the other slot (its last reader was the previous cell) as
-    // soon as the first waves finish phase B, piece 2 once every wave has.
-    int next_nn = -1;
-    if constexpr (CLS == 0) {
-        const int ncls = __builtin_amdgcn_readfirstlane(sm.slot[nxt].cls);
-        const int nn = __builtin_amdgcn_readfirstlane(sm.slot[nxt].n);
-        if (ncls == 0 && nn >= 0) next_nn = nn;
-    }
+    publish_velocity<NW, VW>(sm, wave, aIx, aIy);
+    // two events per negative pixel (the reference evaluates S_other once
+    // per pass)
+    if (neg1) flag_add(A.flags, PFH_FLAG_S_NEGATIVE, 2u * neg1);
+    if (wave == 0) fetch4a(A, sm, nf, nxt);     // visible after the barrier
+    lds_barrier();
+    float vx, vy;
+    finish_velocity<kObs>(A, n, sm, c, vx, vy);
 
     // ---- phase B: Euler update, shifted store, scatter, moments ----
-    const float vx = c.vx, vy = c.vy, mrel = c.mrel, dt = A.dt;
-    const int sx = c.sx, sy = c.sy, dwx = c.dwx, dwy = c.dwy;
-    const int dtx0 = c.dtx0, dty0 = c.dty0;
-    PFH_GLOBAL float* tout = gptr(A.phi_out) + (size_t)n * kTileArea;
-    double aV = 0.0, aCx = 0.0, aCy = 0.0, aPer = 0.0;
-    int blox = dwx, bhix = -1, bloy = dwy, bhiy = -1, pmaxb = 0;
+    const float mrel = uni(c.mrel), dt = uni(A.dt);
+    const int sx = __builtin_amdgcn_readfirstlane(c.sx);
+    const int sy = __builtin_amdgcn_readfirstlane(c.sy);
+    const int dwx = __builtin_amdgcn_readfirstlane(c.dwx);
+    const int dwy = __builtin_amdgcn_readfirstlane(c.dwy);
+    const int dtx0 = __builtin_amdgcn_readfirstlane(c.dtx0);
+    const int dty0 = __builtin_amdgcn_readfirstlane(c.dty0);
+    const int dcls = __builtin_amdgcn_readfirstlane(c.dcls);
+    const bool moved = (sx | sy) != 0 || dcls != CLS;
+    float* const tout_p = uni_ptr(A.phi_out) + (size_t)n * kTileArea;
+    PFH_GLOBAL float* const tout = gptr(tout_p);
+    const __amdgpu_buffer_rsrc_t tst =
+        rsrc_of(tout_p + (size_t)dty0 * kTilePitch, (uint32_t)dwy * kTileRow);
+    // a step without a scatter (S_sc NULL) has an empty aggregate
+    uint32_t* const S_sc_p = uni_ptr(A.S_sc);
+    const __amdgpu_buffer_rsrc_t s_out = rsrc_of(S_sc_p + dm.off, S_sc_p ? s_wrap : 0u);
+    uint32_t olds[VW][RB];
     bool nonfin = false, clampf = false, ovf = false;
-    auto update = [&](float cC, float gxv, float gyv, float pas_k) -> float {
-        return euler_update(cC, gxv, gyv, pas_k, vx, vy, mrel, dt);
-    };
-    const int a = x - sx;
-    if (active) {
-        const bool ain = (unsigned)a < (unsigned)dwx;
-        uint32_t olds[RB];
-        int rlo = dwy, rhi = -1;
-        const float* cb = cbw;
-        float sC = cb[0];
-        float cW, cC, cE;
-        load_row(cb + PX, cW, cC, cE);
-        PFH_GLOBAL float* orow = tout + (ptrdiff_t)(dty0 + y0 - sy) * kTilePitch + dtx0 + a;
-        // the aggregate's base in a VGPR pair: the per-row atomic then needs
-        // neither the argument block nor a scalar wait
-        const bool scatter = A.S_sc != nullptr;   // NULL: a step that scatters nothing
-        PFH_GLOBAL char* S_sc = reinterpret_cast<PFH_GLOBAL char*>(
-            gptr(scatter ? A.S_sc + dm.off : A.S_sc));
-        asm volatile("" : "+v"(S_sc));
-        uint32_t s_off = s_off0;
+
+    // One pass: kGen handles recentred cells, class changes, columns that wrap
+    // around the domain and lanes that own nothing; without it a destination
+    // pixel is its source.
+    auto pass_b = [&](auto gen, int v) {
+        constexpr bool kGen = decltype(gen)::value;
+        const bool loads = !(kKeep && v == VW - 1);
+        // first chunk of this pass in the ring
+        const int q0 = !loads ? v * NCK
+                              : (VW + (kKeep ? VW - 2 - v : VW - 1 - v)) * NCK;
+        const Share<CLS> g(lw_of(v));
+        const int col = g.col();
+        auto row = [&](int kk) -> const PFH_LDS float* {
+            return chunk_at(q0 + kk / kChunkRows) + (kk % kChunkRows) * kRowFloats + col;
+        };
+        const int y0 = g.y0();
+        const int a = kGen ? g.x() - sx : g.x();
+        const bool ain = !kGen || (g.active() && (unsigned)a < (unsigned)dwx);
+        const int b0 = kGen ? y0 - sy : y0;
+        uint32_t st = (uint32_t)(b0 * (int)kTileRow + 4 * ((kGen ? dtx0 : TX0) + a));
+        if (kGen && !ain) st = kOffNone;
+        uint32_t s_off = s_off_of(g.x(), y0), so = 0u;
+        Part p;
+        p.blox = dwx; p.bhix = -1; p.bloy = dwy; p.bhiy = -1; p.pmaxb = 0;
+        uint32_t sup = 0u, pmax = 0u;
+        double bd = (double)b0;
         const double ad = (double)a;
+        if (loads) {
+            advance(q0);
+            if (NCK > 1) advance(q0 + 1);
+        }
+        float sC = row(0)[0];
+        float cW, cC, cE, fW, fC, fE;
+        load_row(row(1), cW, cC, cE);
+        load_row(row(2), fW, fC, fE);
 #pragma unroll
         for (int k = 0; k < RB; ++k) {
-            const int y = y0 + k;
-            olds[k] = 0u;
-            if (row_ok(k)) {
-                float nW, nC, nE;
-                load_row(cb + (k + 2) * PX, nW, nC, nE);
-                const float gxv = 0.5f * (cE - cW);
-                const float gyv = 0.5f * (nC - sC);
-                const int b = y - sy;
-                const bool valid = ain && (unsigned)b < (unsigned)dwy;
-                const float pn = update(cC, gxv, gyv, pas[k]);
-                if (valid) *orow = pn;
-                if constexpr (!kCheck) {
-                // A lane whose destination is outside the window contributes
-                // an exact zero to every sum below.
-                const float pv = valid ? pn : 0.0f;
-                const float sq = pv * pv;
-                nonfin |= !isfinite(pv);
-                clampf |= (sq > kQClampPhiSq);
-                pmaxb = max(pmaxb, (int)__float_as_uint(fabsf(pv)));
-                const uint32_t qv = __float2uint_rn(fminf(sq, kQClampPhiSq) * kQScale);
-                if (qv && scatter)
-                    olds[k] = __hip_atomic_fetch_add(
-                        reinterpret_cast<PFH_GLOBAL uint32_t*>(S_sc + s_off), qv,
-                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                const double d = (double)pv * (double)pv;
-                aV += d;
-                aCy += d * (double)b;
-                if (pv > kSupportEps) { rlo = min(rlo, b); rhi = max(rhi, b); }
-                }
-                sC = cC;
-                cW = nW; cC = nC; cE = nE;
-                orow += kTilePitch;
-                asm volatile("" : "+v"(orow));   // a pointer increment, not a multiply
-                s_off += s_pitch;
-                if (s_off >= s_wrap) s_off -= s_wrap;
-                asm volatile("" : "+v"(s_off));
+            const float nW = fW, nC = fC, nE = fE;
+            if (k + 2 < RB) load_row(row(k + 3), fW, fC, fE);
+            else if (k + 1 < RB) fC = row(k + 3)[0];
+            const float gxv = 0.5f * (cE - cW);
+            const float gyv = 0.5f * (nC - sC);
+            const float pn = euler_update(cC, gxv, gyv, pas[v][k], vx, vy, mrel, dt);
+            // rows past the destination window are past the descriptor's end;
+            // rows past the source window hold no pixel of the cell (shifted,
+            // they could land inside)
+            if constexpr (kGen) {
+                uint32_t o = st + (uint32_t)k * kTileRow;
+                if (k >= G::RFULL) o = y0 + k < WY ? o : kOffNone;
+                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(pn), tst, (int)o, 0, 0);
+            } else {
+                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(pn), tst, (int)st,
+                                                      (int)(k * kTileRow), 0);
             }
+            if constexpr (!kCheck) {
+                // A lane whose destination is outside the window contributes
+                // an exact zero to every sum below. Rows below RFULL exist in
+                // every band, so only the last band's tail rows are tested
+                // without a shift.
+                float pv = pn;
+                if (kGen)
+                    pv = ain && y0 + k < WY && (unsigned)(b0 + k) < (unsigned)dwy ? pn : 0.0f;
+                else if (k >= G::RFULL)
+                    pv = y0 + k < WY ? pn : 0.0f;
+                const float sq = pv * pv;
+                pmax = max(pmax, __float_as_uint(fabsf(pv)));
+                uint32_t w = __float2uint_rn(fminf(sq, kQClampPhiSq) * kQScale);
+                const bool add = w != 0u;
+                asm volatile("" : "+v"(w));  // the old word takes the addend's register
+                if (add)
+                    w = (uint32_t)__builtin_amdgcn_raw_ptr_buffer_atomic_add_i32(
+                        (int)w, s_out, (int)s_off, (int)so, 0);
+                olds[v][k] = w;
+                const double d = (double)pv * (double)pv;
+                p.V += d;
+                p.Cy += d * bd;
+                bd += 1.0;
+                push_support(sup, pv);
+                // added up here: sunk to the end of the pass, the sums would
+                // keep every row's value live
+                asm volatile("" : "+v"(p.V), "+v"(p.Cy), "+v"(pmax));
+                if (kGen) {
+                    s_off = s_next(s_off);
+                } else {
+                    so += s_pitch;
+                    asm volatile("" : "+s"(so));
+                }
+            }
+            sC = cC;
+            cW = nW; cC = nC; cE = nE;
+            if (loads && k % kChunkRows == kChunkRows - 1 && (k + 4) / kChunkRows < NCK)
+                advance(q0 + (k + 4) / kChunkRows);
             __builtin_amdgcn_sched_barrier(0);
         }
-        aCx = aV * ad;                 // every pixel of this thread has column a
-        if (rhi >= 0) { blox = a; bhix = a; bloy = rlo; bhiy = rhi; }
-        // Exact S_overflow test with one register per pixel: every addend is
-        // at most 2^29, so a wrap needs old >= 2^32 - 2^29; only such
-        // candidates recompute q from this thread's own stored value.
+        if constexpr (!kCheck) {
+            p.Cx = p.V * ad;               // every pixel of this lane has column a
+            if (sup) {                     // bit RB - 1 - k: row k
+                p.bloy = b0 + (RB - 32) + __clz((int)sup);
+                p.bhiy = b0 + RB - __ffs((int)sup);
+            }
+            // columns of the two runs: the second run's lie left of the first's
+            const uint64_t m = __builtin_amdgcn_ballot_w64(sup != 0u);
+            const uint64_t m2 = g.split < kWave ? m >> g.split : 0ull;
+            const uint64_t m1 = g.split < kWave ? m & ((1ull << g.split) - 1ull) : m;
+            if (m) {
+                const int sh = kGen ? sx : 0;
+                p.blox = (m2 ? __builtin_ctzll(m2) : g.x0 + __builtin_ctzll(m1)) - sh;
+                p.bhix = (m1 ? g.x0 + 63 - __builtin_clzll(m1) : 63 - __builtin_clzll(m2)) - sh;
+            }
+            p.pmaxb = (int)pmax;
+            nonfin |= pmax >= 0x7F800000u;
+            // sq grows with |phi|; a NaN hides the lane's other values, which
+            // are then read back
+            const float pm = __uint_as_float(pmax);
+            clampf |= pm * pm > kQClampPhiSq;
+            if (pmax > 0x7F800000u) {
+                for (int k = 0; k < RB; ++k) {
+                    const int b = b0 + k;
+                    if (ain && y0 + k < WY && (unsigned)b < (unsigned)dwy) {
+                        const float t = tout[(size_t)(dty0 + b) * kTilePitch + dtx0 + a];
+                        clampf |= t * t > kQClampPhiSq;
+                    }
+                }
+            }
+            publish_part(sm, lw_of(v), p);
+        }
+    };
+    // a logical wave with lanes that own nothing takes the general pass too
+    auto whole = [&](int lw) {
+        return lw > 0 && (lw + 1) * kWave - kControlLanes <= G::NB * WX;
+    };
 #pragma unroll
-        for (int k = 0; k < (kCheck ? 0 : RB); ++k) {
-            if (olds[k] >= 0xE0000000u) {
-                const int b = y0 + k - sy;
-                const uint32_t qv = q_of(tout[(size_t)(dty0 + b) * kTilePitch + dtx0 + a]);
-                ovf |= olds[k] > 0xFFFFFFFFu - qv;
+    for (int v = VW - 1; v >= 0; --v) {
+        if (moved || !flat || !whole(lw_of(v))) pass_b(std::true_type{}, v);
+        else pass_b(std::false_type{}, v);
+    }
+    if constexpr (!kCheck) {
+        // Exact S_overflow test: every addend is at most 2^29, so a wrap needs
+        // old >= 2^32 - 2^29; only such candidates recompute q from this
+        // thread's own stored value.
+        uint32_t big = 0u;
+#pragma unroll
+        for (int v = 0; v < VW; ++v)
+#pragma unroll
+            for (int k = 0; k < RB; ++k) big = max(big, olds[v][k]);
+        if (big >= 0xE0000000u) {
+#pragma unroll
+            for (int v = 0; v < VW; ++v) {
+                const Share<CLS> g(lw_of(v));
+                const PFH_GLOBAL float* mine =
+                    tout + (ptrdiff_t)(dty0 + g.y0() - sy) * kTilePitch + dtx0 + g.x() - sx;
+#pragma unroll
+                for (int k = 0; k < RB; ++k) {
+                    if (olds[v][k] >= 0xE0000000u) {
+                        const uint32_t qv = q_of(mine[k * kTilePitch]);
+                        ovf |= olds[v][k] > 0xFFFFFFFFu - qv;
+                    }
+                }
             }
         }
+        if (nonfin) flag_or(A.flags, PFH_FLAG_NONFINITE);
+        if (clampf) flag_or(A.flags, PFH_FLAG_Q_CLAMP);
+        if (ovf) flag_or(A.flags, PFH_FLAG_S_OVERFLOW);
     }
-    if (nonfin) flag_or(A.flags, PFH_FLAG_NONFINITE);
-    if (clampf) flag_or(A.flags, PFH_FLAG_Q_CLAMP);
-    if (ovf) flag_or(A.flags, PFH_FLAG_S_OVERFLOW);
 
     // Destination pixels whose source lies outside the window are zero.
-    if (c.dcls == CLS) {
-        const int ny = sy > 0 ? sy : -sy, nx = sx > 0 ? sx : -sx;
-        const int rows = ny * dwx, total = rows + nx * dwy;
-        for (int i = tid; i < total; i += kNT) {
-            int aa, b;
-            if (i < rows) {
-                const int rr = i / dwx;
-                aa = i - rr * dwx;
-                b = sy > 0 ? dwy - sy + rr : rr;
-            } else {
-                const int j = i - rows, cc = j / dwy;
-                b = j - cc * dwy;
-                aa = sx > 0 ? dwx - sx + cc : cc;
-            }
-            tout[(size_t)(dty0 + b) * kTilePitch + dtx0 + aa] = 0.0f;
-        }
-    } else {
-        for (int i = tid; i < dwx * dwy; i += kNT) {
-            const int b = i / dwx, aa = i - (i / dwx) * dwx;
-            const int ii = aa + sx, jj = b + sy;
-            if (!((unsigned)ii < (unsigned)WX && (unsigned)jj < (unsigned)WY))
+    if (moved) {
+        if (dcls == CLS) {
+            const int ny = sy > 0 ? sy : -sy, nx = sx > 0 ? sx : -sx;
+            const int nrow = ny * dwx, total = nrow + nx * dwy;
+            for (int i = tid; i < total; i += NT) {
+                int aa, b;
+                if (i < nrow) {
+                    const int rr = i / dwx;
+                    aa = i - rr * dwx;
+                    b = sy > 0 ? dwy - sy + rr : rr;
+                } else {
+                    const int j = i - nrow, cc = j / dwy;
+                    b = j - cc * dwy;
+                    aa = sx > 0 ? dwx - sx + cc : cc;
+                }
                 tout[(size_t)(dty0 + b) * kTilePitch + dtx0 + aa] = 0.0f;
+            }
+        } else {
+            for (int i = tid; i < dwx * dwy; i += NT) {
+                const int b = i / dwx, aa = i - (i / dwx) * dwx;
+                const int ii = aa + sx, jj = b + sy;
+                if (!((unsigned)ii < (unsigned)WX && (unsigned)jj < (unsigned)WY))
+                    tout[(size_t)(dty0 + b) * kTilePitch + dtx0 + aa] = 0.0f;
+            }
         }
     }
 
     // Perimeter on full-moment steps (one step in full_moment_every) from the
     // new field in the source layout with source-window zeros (the staged
-    // semantics, src/kernels.cu:512-538). phi_next is recomputed here, bit for
-    // bit as above, instead of being held through the update.
+    // semantics, src/kernels.cu:512-538): read back from the stored tile, or
+    // recomputed where a recentred window does not hold it.
     if (!kCheck && c.fm) {
-        float pns[RB];
-        if (active) {
-            uint32_t qS2[RB];
-            load_qs(qS2);
-            uint32_t negc2 = 0u;
-            Roll q;
-            load_row(cbw, q.sW, q.sC, q.sE);
-            load_row(cbw + PX, q.cW, q.cC, q.cE);
-#pragma unroll
-            for (int k = 0; k < RB; ++k) {
-                pns[k] = 0.0f;
-                if (row_ok(k)) {
-                    load_row(cbw + (k + 2) * PX, q.nW, q.nC, q.nE);
-                    const float So = s_other_of(qS2[k], q.cC, negc2);
-                    const float pk = with_repulsion(passive_head(q, gam, dwC, volC), repC,
-                                                    q.cC, So);
-                    pns[k] = update(q.cC, 0.5f * (q.cE - q.cW), 0.5f * (q.nC - q.sC), pk);
-                    q.sW = q.cW; q.sC = q.cC; q.sE = q.cE;
-                    q.cW = q.nW; q.cC = q.nC; q.cE = q.nE;
+        __threadfence();          // stores reach L2; L1 lines are invalidated
+        __syncthreads();
+        const NextArgs na{A.phi_in + (size_t)n * kTileArea + (size_t)TY0 * kTilePitch + TX0,
+                          A.S_rd + dm.off, WX, WY, L, P, c.gx0, c.gy0, c.gam, c.dwC, c.volC,
+                          A.rep_coeff, vx, vy, mrel, dt};
+        auto value = [&](int ii, int jj) -> float {
+            return moved ? next_at(na, ii, jj)
+                         : tout[(size_t)(TY0 + jj) * kTilePitch + TX0 + ii];
+        };
+        for (int v = 0; v < VW; ++v) {
+            double aPer = 0.0;
+            for (int i = tid + v * NT; i < dwx * dwy; i += kNT) {
+                const int b = i / dwx, aa = i - (i / dwx) * dwx;
+                const int ii = aa + sx, jj = b + sy;
+                const bool iin = (unsigned)ii < (unsigned)WX;
+                const bool jin = (unsigned)jj < (unsigned)WY;
+                float e = 0.0f, w = 0.0f, nn = 0.0f, ss = 0.0f;
+                if (jin) {
+                    if ((unsigned)(ii + 1) < (unsigned)WX) e = value(ii + 1, jj);
+                    if ((unsigned)(ii - 1) < (unsigned)WX) w = value(ii - 1, jj);
                 }
-                __builtin_amdgcn_sched_barrier(0);
+                if (iin) {
+                    if ((unsigned)(jj + 1) < (unsigned)WY) nn = value(ii, jj + 1);
+                    if ((unsigned)(jj - 1) < (unsigned)WY) ss = value(ii, jj - 1);
+                }
+                const float pgx = 0.5f * (e - w), pgy = 0.5f * (nn - ss);
+                aPer += (double)sqrtf(pgx * pgx + pgy * pgy);
             }
-        }
-        lds_barrier();                         // all reads of phi_s done
-        if (active) {
-#pragma unroll
-            for (int k = 0; k < RB; ++k)
-                if (row_ok(k)) cbw[(k + 1) * PX] = pns[k];
-        }
-        lds_barrier();
-        for (int i = tid; i < dwx * dwy; i += kNT) {
-            const int b = i / dwx, aa = i - (i / dwx) * dwx;
-            const int ii = aa + sx, jj = b + sy;
-            const bool iin = (unsigned)ii < (unsigned)WX;
-            const bool jin = (unsigned)jj < (unsigned)WY;
-            float e = 0.0f, w = 0.0f, nn = 0.0f, ss = 0.0f;
-            if (jin) {
-                const float* pr = rowp(jj) + ii;
-                if ((unsigned)(ii + 1) < (unsigned)WX) e = pr[1];
-                if ((unsigned)(ii - 1) < (unsigned)WX) w = pr[-1];
-            }
-            if (iin) {
-                if ((unsigned)(jj + 1) < (unsigned)WY) nn = rowp(jj + 1)[ii];
-                if ((unsigned)(jj - 1) < (unsigned)WY) ss = rowp(jj - 1)[ii];
-            }
-            const float pgx = 0.5f * (e - w), pgy = 0.5f * (nn - ss);
-            aPer += (double)sqrtf(pgx * pgx + pgy * pgy);
+            aPer = wave_sum(aPer);
+            if (lane == 0) sm.red[lw_of(v) * 4 + 3] = aPer;
         }
     }
-    // The next cell's scalars, on a thread of wave 1: the first waves of each
-    // SIMD finish phase B early, wave 0 (control lanes, commit) the latest.
+    // The next cell's scalars, then the commit by wave 0. The other waves go
+    // on to the next cell: its first barrier orders their next partials.
     if (tid == kScalarsThread) fetch4b<kBatch>(A, sm, nxt, step);
-    if constexpr (CLS == 0) {
-        // piece 1 of the next window: each wave issues its rows as it
-        // finishes phase B
-        if (next_nn >= 0)
-            copy_rows0(A, next_nn, phi_s + (pslot ^ 1) * Split0::P1_FLOATS + PX + 4, 0,
-                       Split0::R1 + 1);
-    }
+    lds_barrier();
     if constexpr (kCheck) {
-        commit_position(A, n, sm, c, [&]() {
-            if (next_nn >= 0) copy_rows0(A, next_nn, base2 + 4, Split0::P2_R0, WY);
-        });
-        pre = next_nn >= 0 ? 1 : 0;
-        if (pre) pslot ^= 1;
-    } else if constexpr (CLS == 0) {
-        reduce_commit<CLS>(A, n, sm, c, sm.csraw[nxt ^ 1], aV, aCx, aCy, aPer,
-                           blox, bhix, bloy, bhiy, pmaxb, [&]() {
-            if (next_nn >= 0) copy_rows0(A, next_nn, base2 + 4, Split0::P2_R0, WY);
-        });
-        pre = next_nn >= 0 ? 1 : 0;
-        if (pre) pslot ^= 1;
+        commit_position(A, n, c);
     } else {
-        reduce_commit<CLS>(A, n, sm, c, sm.csraw[nxt ^ 1], aV, aCx, aCy, aPer,
-                           blox, bhix, bloy, bhiy, pmaxb);
+        if (wave == 0) commit_cell<CLS>(A, n, sm, c, sm.csraw[nxt ^ 1]);
     }
 }
 
 // -------------------------------------------------------------------------
 // Global-memory path: class 4 (window zeros synthesized) and the fallback
 // class 5 (the tile's own one-pixel zero ring), src/kernels.cu:604-937.
+// Logical thread t owns pixels t, t + 1024, ...
 // -------------------------------------------------------------------------
-template <int CLS, bool kBatch = false, int kObs = 0>
+template <int CLS, int NW, bool kBatch = false, int kObs = 0>
 __device__ void cell_global(const pfh2d_step_args& A, int n,
                             unsigned long long step, Smem& sm, Ctl& c, int nxt) {
     constexpr int WX = kShapes[CLS].wx, WY = kShapes[CLS].wy;
     constexpr int TX0 = kShapes[CLS].tx0, TY0 = kShapes[CLS].ty0;
+    constexpr int NT = NW * kWave, VW = kWaves / NW;
     const int tid = opaque_tid();
+    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
     const Dom dm = cell_dom<kBatch>(A, sm.slot[nxt ^ 1]);
     const int L = dm.L, P = dm.P;
     const uint32_t* S_rd = A.S_rd + dm.off;
     uint32_t* S_sc = A.S_sc ? A.S_sc + dm.off : nullptr;
-    if (tid < kControlLanes) fetch_all<kBatch>(A, sm, nxt, step);
+    if (wave == 0) fetch_all<kBatch>(A, sm, nxt, step);
     const int gx0 = c.gx0, gy0 = c.gy0;
     const float* tin = A.phi_in + (size_t)n * kTileArea;
     float* tout = A.phi_out + (size_t)n * kTileArea;
@@ -1196,36 +1286,46 @@ __device__ void cell_global(const pfh2d_step_args& A, int n,
             return 0.0f;
         return tin[(size_t)(TY0 + yy) * kTilePitch + TX0 + xx];
     };
-    if (c.zero_tile) zero_outside_window(tout, c.dwx, c.dwy, c.dtx0, c.dty0);
+    if (c.zero_tile) zero_outside_window<NT>(tout, c.dwx, c.dwy, c.dtx0, c.dty0);
 
-    double aIx = 0.0, aIy = 0.0;
     uint32_t negc = 0u;
-    ObsSums ob;
-    for (int p = tid; p < WX * WY; p += kNT) {
-        const int y = p / WX, x = p - (p / WX) * WX;
-        const float cc = pin(x, y);
-        const float gxv = 0.5f * (pin(x + 1, y) - pin(x - 1, y));
-        const float gyv = 0.5f * (pin(x, y + 1) - pin(x, y - 1));
-        const uint32_t qS = S_rd[(size_t)wrapi(gy0 + y, L) * P + wrapi(gx0 + x, L)];
-        const uint32_t qc = q_of(cc);
-        float So = 0.0f;
-        if (qS >= qc) So = (float)(qS - qc) * kQInv;
-        else negc += 1u;
-        aIx += (double)(cc * gxv * So);
-        aIy += (double)(cc * gyv * So);
-        if constexpr (kObs == 2)
-            observe_pixel(ob, x, y, cc, pin(x + 1, y), pin(x - 1, y), pin(x, y + 1),
-                          pin(x, y - 1), pin(x + 1, y + 1), pin(x - 1, y + 1),
-                          pin(x + 1, y - 1), pin(x - 1, y - 1), So, c.gam, c.dwC,
-                          A.rep_coeff, c.og2iv, c.ocx, c.ocy);
+    double aIxv[VW], aIyv[VW];
+#pragma unroll
+    for (int v = 0; v < VW; ++v) {
+        double aIx = 0.0, aIy = 0.0;
+        ObsSums ob;
+        for (int p = tid + v * NT; p < WX * WY; p += kNT) {
+            const int y = p / WX, x = p - (p / WX) * WX;
+            const float cc = pin(x, y);
+            const float gxv = 0.5f * (pin(x + 1, y) - pin(x - 1, y));
+            const float gyv = 0.5f * (pin(x, y + 1) - pin(x, y - 1));
+            const uint32_t qS = S_rd[(size_t)wrapi(gy0 + y, L) * P + wrapi(gx0 + x, L)];
+            const uint32_t qc = q_of(cc);
+            float So = 0.0f;
+            if (qS >= qc) So = (float)(qS - qc) * kQInv;
+            else negc += 1u;
+            aIx += (double)(cc * gxv * So);
+            aIy += (double)(cc * gyv * So);
+            if constexpr (kObs == 2)
+                observe_pixel(ob, x, y, cc, pin(x + 1, y), pin(x - 1, y), pin(x, y + 1),
+                              pin(x, y - 1), pin(x + 1, y + 1), pin(x - 1, y + 1),
+                              pin(x + 1, y - 1), pin(x - 1, y - 1), So, c.gam, c.dwC,
+                              A.rep_coeff, c.og2iv, c.ocx, c.ocy);
+        }
+        aIxv[v] = aIx;
+        aIyv[v] = aIy;
+        if constexpr (kObs == 2) publish_observer(sm, wave + NW * v, ob);
     }
-    reduce_velocity<kObs>(A, n, sm, c, aIx, aIy, ob);
+    publish_velocity<NW, VW>(sm, wave, aIxv, aIyv);
+    lds_barrier();
+    float vx, vy;
+    finish_velocity<kObs>(A, n, sm, c, vx, vy);
 
     const float gam = c.gam, dwC = c.dwC, volC = c.volC, repC = A.rep_coeff;
-    const float vx = c.vx, vy = c.vy, mrel = c.mrel, dt = A.dt;
+    const float mrel = c.mrel, dt = A.dt;
     const int sx = c.sx, sy = c.sy, dwx = c.dwx, dwy = c.dwy;
     const int dtx0 = c.dtx0, dty0 = c.dty0;
-    for (int p = tid; p < WX * WY; p += kNT) {
+    for (int p = tid; p < WX * WY; p += NT) {
         const int y = p / WX, x = p - (p / WX) * WX;
         const float cC = pin(x, y);
         const float cE = pin(x + 1, y), cW = pin(x - 1, y);
@@ -1247,7 +1347,7 @@ __device__ void cell_global(const pfh2d_step_args& A, int n,
             tout[(size_t)(dty0 + b) * kTilePitch + dtx0 + a] = pn;
     }
     if (negc) flag_add(A.flags, PFH_FLAG_S_NEGATIVE, negc);
-    for (int i = tid; i < dwx * dwy; i += kNT) {
+    for (int i = tid; i < dwx * dwy; i += NT) {
         const int b = i / dwx, a = i - (i / dwx) * dwx;
         const int ii = a + sx, jj = b + sy;
         if (!((unsigned)ii < (unsigned)WX && (unsigned)jj < (unsigned)WY))
@@ -1257,59 +1357,67 @@ __device__ void cell_global(const pfh2d_step_args& A, int n,
     __syncthreads();
 
     const int gx0n = c.gx0n, gy0n = c.gy0n, fm = c.fm;
-    double aV = 0.0, aCx = 0.0, aCy = 0.0, aPer = 0.0;
-    int blox = dwx, bhix = -1, bloy = dwy, bhiy = -1, pmaxb = 0;
     bool nonfin = false, clampf = false, ovf = false;
-    for (int i = tid; i < dwx * dwy; i += kNT) {
-        const int b = i / dwx, a = i - (i / dwx) * dwx;
-        const size_t row = (size_t)(dty0 + b) * kTilePitch + dtx0;
-        const float pn = tout[row + a];
-        nonfin |= !isfinite(pn);
-        clampf |= (pn * pn > kQClampPhiSq);
-        pmaxb = max(pmaxb, (int)__float_as_uint(fabsf(pn)));
-        const uint32_t q = q_of(pn);
-        if (q && S_sc) {
-            const uint32_t old = atomicAdd(
-                &S_sc[(size_t)wrapi(gy0n + b, L) * P + wrapi(gx0n + a, L)], q);
-            ovf |= old > 0xFFFFFFFFu - q;
+    for (int v = 0; v < VW; ++v) {
+        double aPer = 0.0;
+        Part pt;
+        pt.blox = dwx; pt.bhix = -1; pt.bloy = dwy; pt.bhiy = -1; pt.pmaxb = 0;
+        for (int i = tid + v * NT; i < dwx * dwy; i += kNT) {
+            const int b = i / dwx, a = i - (i / dwx) * dwx;
+            const size_t row = (size_t)(dty0 + b) * kTilePitch + dtx0;
+            const float pn = tout[row + a];
+            nonfin |= !isfinite(pn);
+            clampf |= (pn * pn > kQClampPhiSq);
+            pt.pmaxb = max(pt.pmaxb, (int)__float_as_uint(fabsf(pn)));
+            const uint32_t q = q_of(pn);
+            if (q && S_sc) {
+                const uint32_t old = atomicAdd(
+                    &S_sc[(size_t)wrapi(gy0n + b, L) * P + wrapi(gx0n + a, L)], q);
+                ovf |= old > 0xFFFFFFFFu - q;
+            }
+            const double d = (double)pn * (double)pn;
+            pt.V += d;
+            pt.Cx += d * (double)a;
+            pt.Cy += d * (double)b;
+            if (pn > kSupportEps) {
+                pt.blox = min(pt.blox, a); pt.bhix = max(pt.bhix, a);
+                pt.bloy = min(pt.bloy, b); pt.bhiy = max(pt.bhiy, b);
+            }
+            if (fm) {
+                const float e = a + 1 < dwx ? tout[row + a + 1] : 0.0f;
+                const float w = a > 0 ? tout[row + a - 1] : 0.0f;
+                const float nn = b + 1 < dwy ? tout[row + kTilePitch + a] : 0.0f;
+                const float ss = b > 0 ? tout[row - kTilePitch + a] : 0.0f;
+                const float pgx = 0.5f * (e - w), pgy = 0.5f * (nn - ss);
+                aPer += (double)sqrtf(pgx * pgx + pgy * pgy);
+            }
         }
-        const double d = (double)pn * (double)pn;
-        aV += d;
-        aCx += d * (double)a;
-        aCy += d * (double)b;
-        if (pn > kSupportEps) {
-            blox = min(blox, a); bhix = max(bhix, a);
-            bloy = min(bloy, b); bhiy = max(bhiy, b);
-        }
+        pt.blox = __builtin_amdgcn_readfirstlane(wave_min(pt.blox));
+        pt.bhix = __builtin_amdgcn_readfirstlane(wave_max(pt.bhix));
+        publish_part(sm, wave + NW * v, pt);
         if (fm) {
-            const float e = a + 1 < dwx ? tout[row + a + 1] : 0.0f;
-            const float w = a > 0 ? tout[row + a - 1] : 0.0f;
-            const float nn = b + 1 < dwy ? tout[row + kTilePitch + a] : 0.0f;
-            const float ss = b > 0 ? tout[row - kTilePitch + a] : 0.0f;
-            const float pgx = 0.5f * (e - w), pgy = 0.5f * (nn - ss);
-            aPer += (double)sqrtf(pgx * pgx + pgy * pgy);
+            aPer = wave_sum(aPer);
+            if ((tid & (kWave - 1)) == 0) sm.red[(wave + NW * v) * 4 + 3] = aPer;
         }
     }
     if (nonfin) flag_or(A.flags, PFH_FLAG_NONFINITE);
     if (clampf) flag_or(A.flags, PFH_FLAG_Q_CLAMP);
     if (ovf) flag_or(A.flags, PFH_FLAG_S_OVERFLOW);
-    reduce_commit<CLS>(A, n, sm, c, sm.csraw[nxt ^ 1], aV, aCx, aCy, aPer,
-                       blox, bhix, bloy, bhiy, pmaxb);
+    lds_barrier();
+    if (wave == 0) commit_cell<CLS>(A, n, sm, c, sm.csraw[nxt ^ 1]);
 }
 
 // Classes other than the round class 0 run out of line, with their own
 // register allocation, so their longer per-thread columns (up to 29 rows) do
 // not raise the pressure of the hot class-0 path.
-template <int CLS, bool kBatch = false, int kObs = 0>
-__device__ __noinline__ void cell_cold(const pfh2d_step_args* A, int n,
-                                       unsigned long long step, Smem* sm, int cur) {
-    if constexpr (CLS <= kClassStagedMax) {
-        int none = 0, slot0 = 0;
-        cell_staged<CLS, false, kBatch, kObs>(*A, n, step, *sm, sm->slot[cur].ctl, cur ^ 1,
-                                              none, slot0);
-    }
+template <int CLS, int NW, bool kBatch = false, int kObs = 0>
+__device__ __noinline__ void cell_cold(const pfh2d_step_args* A, int n, unsigned long long step,
+                                       Smem* sm, PFH_LDS float* win, int cur) {
+    n = __builtin_amdgcn_readfirstlane(n);
+    if constexpr (CLS <= kClassStagedMax)
+        cell_walk<CLS, NW, false, kBatch, kObs>(*A, n, step, *sm, win, sm->slot[cur].ctl, cur ^ 1);
     else
-        cell_global<CLS, kBatch, kObs>(*A, n, step, *sm, sm->slot[cur].ctl, cur ^ 1);
+        cell_global<CLS, NW, kBatch, kObs>(*A, n, step, *sm, sm->slot[cur].ctl, cur ^ 1);
 }
 
 // -------------------------------------------------------------------------
@@ -1320,33 +1428,18 @@ __device__ __noinline__ void cell_cold(const pfh2d_step_args* A, int n,
 // cells; each S slot one arena holding every replica's aggregate; the
 // clear-ahead sweeps the whole arena), and each cell's side, S pitch, S
 // offset and polarity stream come from its replica's record.
-template <bool kCheck, bool kBatch = false, int kObs = 0>
-__global__ __launch_bounds__(kNT, 1) void k_step(const pfh2d_step_args A, const int* run_if,
-                                                 const pfh2d_replica* reps,
-                                                 const uint16_t* cell_rep) {
+template <int NW, bool kCheck, bool kBatch = false, int kObs = 0>
+__global__ __launch_bounds__(NW * kWave, 4) void k_step(const pfh2d_step_args A,
+                                                        const int* run_if,
+                                                        const pfh2d_replica* reps,
+                                                        const uint16_t* cell_rep) {
+    constexpr int NT = NW * kWave;
     __shared__ Smem sm;
+    __shared__ __attribute__((aligned(16))) float window[kWindowFloats<NW>];
+    PFH_LDS float* const win = (PFH_LDS float*)window;
     const int tid = (int)threadIdx.x;
     if (run_if != nullptr && *run_if == 0) return;   // gated-off launch: no effect
 
-    // Clear S[(step+2)%3] ahead: this slot is neither read nor scattered
-    // into by this launch. Non-temporal stores keep it out of the caches.
-    if (A.clear_ahead_words > 0ull) {
-        u32x4* dst = reinterpret_cast<u32x4*>(A.S_cl);
-        const u32x4 zero4 = {0u, 0u, 0u, 0u};
-        const size_t nvec = (size_t)(A.clear_ahead_words >> 2);
-        const size_t stride = (size_t)gridDim.x * kNT;
-        for (size_t i = (size_t)blockIdx.x * kNT + tid; i < nvec; i += stride)
-            __builtin_nontemporal_store(zero4, &dst[i]);
-        for (size_t i = (nvec << 2) + (size_t)blockIdx.x * kNT + tid;
-             i < (size_t)A.clear_ahead_words; i += stride)
-            A.S_cl[i] = 0u;
-    }
-    // Cursor and step slots alternate with the phi parity; the kernel
-    // boundary orders the reset and publication for the next launch.
-    if (blockIdx.x == 0 && tid == 0) {
-        *A.cursor_clear = 0ull;
-        *A.step_wr = *A.step_rd + 1ull;
-    }
     const unsigned long long step = *A.step_rd;
     if (tid == 0) {
         sm.args = A;
@@ -1357,41 +1450,49 @@ __global__ __launch_bounds__(kNT, 1) void k_step(const pfh2d_step_args A, const 
             sm.cell_rep = cell_rep;
         }
     }
-
-    // The control wavefront fetches each next cell one cell ahead (ticket,
-    // id, class, CellState, scalars) while the other wavefronts compute, so
-    // the queue's global round trips stay off the critical path.
-    if (tid < kControlLanes) fetch_all<kBatch>(A, sm, 0, step);
+    // Wave 0 fetches each next cell one cell ahead (ticket, id, class,
+    // CellState) while it computes, so the queue's global round trips stay
+    // off the critical path.
+    if (tid < kWave) fetch_first<kBatch>(A, sm, step);
+    // Clear S[(step+2)%3] ahead: this slot is neither read nor scattered
+    // into by this launch. Non-temporal stores keep it out of the caches.
+    if (A.clear_ahead_words > 0ull) {
+        u32x4* dst = reinterpret_cast<u32x4*>(A.S_cl);
+        const u32x4 zero4 = {0u, 0u, 0u, 0u};
+        const size_t nvec = (size_t)(A.clear_ahead_words >> 2);
+        const size_t stride = (size_t)gridDim.x * NT;
+        for (size_t i = (size_t)blockIdx.x * NT + tid; i < nvec; i += stride)
+            __builtin_nontemporal_store(zero4, &dst[i]);
+        for (size_t i = (nvec << 2) + (size_t)blockIdx.x * NT + tid;
+             i < (size_t)A.clear_ahead_words; i += stride)
+            A.S_cl[i] = 0u;
+    }
+    // Cursor and step slots alternate with the phi parity; the kernel
+    // boundary orders the reset and publication for the next launch.
+    if (blockIdx.x == 0 && tid == 0) {
+        *A.cursor_clear = 0ull;
+        *A.step_wr = step + 1ull;
+    }
     lds_barrier();
     int cur = 0;
-    int pre = 0;                       // the current class-0 window is already in LDS
-    int pslot = 0;                     // slot of the class-0 window's piece 1
-    int ring = 0;                      // the class-0 layout's zero ring is set up
     for (;;) {
         const int cls = __builtin_amdgcn_readfirstlane(sm.slot[cur].cls);
         const int n = __builtin_amdgcn_readfirstlane(sm.slot[cur].n);
         if (cls < 0) break;
         switch (cls) {
             case 0:
-                cell_staged<0, kCheck, kBatch, kObs>(A, n, step, sm, sm.slot[cur].ctl, cur ^ 1,
-                                                     pre, pslot, &ring);
+                cell_walk<0, NW, kCheck, kBatch, kObs>(sm.args, n, step, sm, win,
+                                                       sm.slot[cur].ctl, cur ^ 1);
                 break;
-            case 1: cell_cold<1, kBatch, kObs>(&sm.args, n, step, &sm, cur); break;
-            case 2: cell_cold<2, kBatch, kObs>(&sm.args, n, step, &sm, cur); break;
-            case 3: cell_cold<3, kBatch, kObs>(&sm.args, n, step, &sm, cur); break;
-            case 4: cell_cold<4, kBatch, kObs>(&sm.args, n, step, &sm, cur); break;
-            case 5: cell_cold<5, kBatch, kObs>(&sm.args, n, step, &sm, cur); break;
+            case 1: cell_cold<1, NW, kBatch, kObs>(&sm.args, n, step, &sm, win, cur); break;
+            case 2: cell_cold<2, NW, kBatch, kObs>(&sm.args, n, step, &sm, win, cur); break;
+            case 3: cell_cold<3, NW, kBatch, kObs>(&sm.args, n, step, &sm, win, cur); break;
+            case 4: cell_cold<4, NW, kBatch, kObs>(&sm.args, n, step, &sm, win, cur); break;
+            case 5: cell_cold<5, NW, kBatch, kObs>(&sm.args, n, step, &sm, win, cur); break;
             default:                       // unsupported id, flagged at fetch
-                if (tid < kControlLanes) fetch_all<kBatch>(A, sm, cur ^ 1, step);
+                if (tid < kWave) fetch_all<kBatch>(sm.args, sm, cur ^ 1, step);
                 lds_barrier();
                 break;
-        }
-        if (cls != 0) {
-            pre = 0;
-            ring = 0;
-            // Retire the out-of-line paths' register reloads here, so that the
-            // loop head does not wait on them (with everything else in flight).
-            __builtin_amdgcn_s_waitcnt(0);
         }
         cur ^= 1;
     }
@@ -1931,6 +2032,24 @@ int unsupported(const char* what) {
 }  // namespace pfh_host
 using namespace pfh_host;
 
+namespace {
+// grid compute units: two 8-wave workgroups on each when there are more
+// cells than compute units, one 16-wave workgroup each otherwise (a lone
+// cell then has the whole compute unit).
+template <bool kCheck, bool kBatch, int kObs>
+void launch_k_step(const pfh2d_step_args& a, const int* run_if, const pfh2d_replica* reps,
+                   const uint16_t* cell_rep, int grid, void* stream) {
+    if (a.N > grid)
+        hipLaunchKernelGGL((pfh::k_step<8, kCheck, kBatch, kObs>), dim3(2u * (unsigned)grid),
+                           dim3(8 * pfh::kWave), 0, as_stream(stream), a, run_if, reps,
+                           cell_rep);
+    else
+        hipLaunchKernelGGL((pfh::k_step<16, kCheck, kBatch, kObs>), dim3((unsigned)grid),
+                           dim3(16 * pfh::kWave), 0, as_stream(stream), a, run_if, reps,
+                           cell_rep);
+}
+}  // namespace
+
 extern "C" {
 
 int pfh_abi_version(void) { return 10000; }
@@ -1978,19 +2097,14 @@ int step_launch(const pfh2d_step_args* a, const int* run_if, int grid, void* str
         return invalid("aggregate larger than 4 GiB");
     const pfh2d_replica* no_reps = nullptr;
     const uint16_t* no_map = nullptr;
-    const dim3 g((unsigned)grid), b(pfh::kNT);
     if (check)
-        hipLaunchKernelGGL((pfh::k_step<true, false>), g, b, 0, as_stream(stream), *a, run_if,
-                           no_reps, no_map);
+        launch_k_step<true, false, 0>(*a, run_if, no_reps, no_map, grid, stream);
     else if (observation == PFH_OBSERVE_ADVECTION)
-        hipLaunchKernelGGL((pfh::k_step<false, false, 1>), g, b, 0, as_stream(stream), *a,
-                           run_if, no_reps, no_map);
+        launch_k_step<false, false, 1>(*a, run_if, no_reps, no_map, grid, stream);
     else if (observation == PFH_OBSERVE_SPATIAL)
-        hipLaunchKernelGGL((pfh::k_step<false, false, 2>), g, b, 0, as_stream(stream), *a,
-                           run_if, no_reps, no_map);
+        launch_k_step<false, false, 2>(*a, run_if, no_reps, no_map, grid, stream);
     else
-        hipLaunchKernelGGL((pfh::k_step<false, false>), g, b, 0, as_stream(stream), *a, run_if,
-                           no_reps, no_map);
+        launch_k_step<false, false, 0>(*a, run_if, no_reps, no_map, grid, stream);
     return launch_status("k_step");
 }
 }  // namespace
@@ -2044,20 +2158,20 @@ int pfh2d_launch_batch_step(const pfh2d_step_args* a, const pfh2d_replica* repli
         return invalid("batch step: replica sides must be at least 256");
     if (4ull * (unsigned long long)max_pitch * (unsigned long long)max_side > 0xFFFFFFFFull)
         return invalid("aggregate larger than 4 GiB");
-    hipLaunchKernelGGL((pfh::k_step<false, true>), dim3((unsigned)grid), dim3(pfh::kNT), 0,
-                       as_stream(stream), *a, (const int*)nullptr, replicas, cell_replica);
+    launch_k_step<false, true, 0>(*a, nullptr, replicas, cell_replica, grid, stream);
     return launch_status("k_step (batched)");
 }
 
 int pfh2d_query_step_stats(int device, pfh_kernel_stats* out) {
     if (!out) return invalid("out");
     hipFuncAttributes fa{};
-    int st = hip_status(hipFuncGetAttributes(&fa, reinterpret_cast<const void*>(pfh::k_step<false, false>)),
+    int st = hip_status(hipFuncGetAttributes(&fa, reinterpret_cast<const void*>(pfh::k_step<8, false>)),
                         "hipFuncGetAttributes(k_step)");
     if (st != PFH_OK) return st;
     int blocks = 0;
     st = hip_status(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                        &blocks, reinterpret_cast<const void*>(pfh::k_step<false, false>), pfh::kNT, 0),
+                        &blocks, reinterpret_cast<const void*>(pfh::k_step<8, false>),
+                        8 * pfh::kWave, 0),
                     "hipOccupancyMaxActiveBlocksPerMultiprocessor(k_step)");
     if (st != PFH_OK) return st;
     int max_threads = 0;
@@ -2070,8 +2184,8 @@ int pfh2d_query_step_stats(int device, pfh_kernel_stats* out) {
     out->static_smem = (int)fa.sharedSizeBytes;
     out->dynamic_smem = 0;
     out->ctas_per_sm = blocks;
-    out->warps_per_sm = blocks * pfh::kNT / pfh::kWave;
-    out->occupancy = (double)(blocks * pfh::kNT) / (double)max_threads;
+    out->warps_per_sm = blocks * 8;
+    out->occupancy = (double)(blocks * 8 * pfh::kWave) / (double)max_threads;
     return PFH_OK;
 }
 

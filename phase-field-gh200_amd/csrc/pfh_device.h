@@ -80,40 +80,10 @@ template <int CLS> struct Staged {
     static constexpr int NB = kPixThreads / WX;
     static constexpr int RB = (WY + NB - 1) / NB;
     static constexpr int RFULL = WY - (NB - 1) * RB;    // rows every band holds
-    static constexpr int NCH = WX / 4;                  // 16 B chunks per row
-    static constexpr int NCHUNK = WY * NCH;
-    static constexpr int KCH = (NCHUNK + kNT - 1) / kNT;
-    static constexpr int PX = WX + 4;                   // LDS row pitch
-    static constexpr int LDS_FLOATS = (WY + 2) * PX + 4;
-    static_assert(WX % 4 == 0 && TX0 % 4 == 0, "16 B phi rows");
+    static_assert(WX % 16 == 0 && TX0 % 4 == 0, "16 B phi groups, runs of whole groups");
+    static_assert(WX >= kWave, "a wave spans at most two bands");
     static_assert(NB * RB >= WY, "bands must cover the window");
 };
-constexpr int max2(int a, int b) { return a > b ? a : b; }
-
-// Class 0 keeps its LDS window in two pieces, so that the next cell's window
-// can be copied in while the current one is still being read: piece 1 holds
-// rows -1..R1 (read by bands 0..KB-1) in one of two slots, piece 2 rows
-// P2_R0..WY (read by bands KB..NB-1). Rows P2_R0 and R1 are in both pieces.
-// Each piece has the padded row layout of the whole window, with four floats
-// after its last row (that row's east pad).
-struct Split0 {
-    using G = Staged<0>;
-    static constexpr int KB = 5;
-    static constexpr int R1 = KB * G::RB;              // first row of band KB
-    static constexpr int P2_R0 = R1 - 1;
-    static constexpr int P1_ROWS = R1 + 2;             // rows -1..R1
-    static constexpr int P2_ROWS = G::WY + 1 - P2_R0;  // rows P2_R0..WY
-    static constexpr int P1_FLOATS = P1_ROWS * G::PX + 4;
-    static constexpr int P2_FLOATS = P2_ROWS * G::PX + 4;
-    static constexpr int FLOATS = 2 * P1_FLOATS + P2_FLOATS;
-    static_assert(KB < G::NB && (G::NB - 1) * G::RB < G::WY, "two non-empty pieces");
-    static_assert(P1_FLOATS % 4 == 0 && P2_FLOATS % 4 == 0, "16 B piece alignment");
-};
-
-constexpr int kPhiLdsFloats =
-    max2(max2(Split0::FLOATS, Staged<1>::LDS_FLOATS),
-         max2(Staged<2>::LDS_FLOATS, Staged<3>::LDS_FLOATS));
-
 // ---- Q5.27 ----
 constexpr float kQScale = 134217728.0f;             // 2^27
 constexpr float kQInv = 7.45058059692382812e-09f;   // 2^-27
@@ -259,20 +229,90 @@ __device__ __forceinline__ void lds_barrier() {
 }
 
 // ---- wavefront reductions: lane tree with offsets 32..1 ----
+// The result is lane 0's (the other lanes end with partial results): lane i
+// adds lane i + d for d = 32, 16 (row swaps of gfx950), then 8, 4, 2, 1 within
+// the first row of 16 lanes (DPP row shifts). No step goes through LDS, whose
+// round trip a shuffle waits for six times over.
+__device__ __forceinline__ int wave_down32(int v) {
+    return (int)__builtin_amdgcn_permlane32_swap((unsigned)v, (unsigned)v, false, false)[1];
+}
+__device__ __forceinline__ int wave_down16(int v) {
+    return (int)__builtin_amdgcn_permlane16_swap((unsigned)v, (unsigned)v, false, false)[1];
+}
+// lane i of each row of 16: lane i + kD's value (0 past the row's end, where
+// the tree's result is not read)
+template <int kD>
+__device__ __forceinline__ int row_down(int v) {
+    return __builtin_amdgcn_update_dpp(0, v, 0x100 + kD, 0xf, 0xf, true);
+}
+template <class F>
+__device__ __forceinline__ int wave_tree(int v, F op) {
+    v = op(v, wave_down32(v));
+    v = op(v, wave_down16(v));
+    v = op(v, row_down<8>(v));
+    v = op(v, row_down<4>(v));
+    v = op(v, row_down<2>(v));
+    return op(v, row_down<1>(v));
+}
 __device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-    for (int d = kWave / 2; d > 0; d >>= 1) v += __shfl_down(v, d, kWave);
+    auto both = [](double x, auto f) {
+        return __hiloint2double(f(__double2hiint(x)), f(__double2loint(x)));
+    };
+    v += both(v, [](int x) { return wave_down32(x); });
+    v += both(v, [](int x) { return wave_down16(x); });
+    v += both(v, [](int x) { return row_down<8>(x); });
+    v += both(v, [](int x) { return row_down<4>(x); });
+    v += both(v, [](int x) { return row_down<2>(x); });
+    v += both(v, [](int x) { return row_down<1>(x); });
+    return v;
+}
+// Four trees at once, each with the order of wave_sum / wave_tree: the first
+// row swap puts two values in the two halves of the wave, the second two more
+// in the rows of 16, and the row steps then serve all four. Lane 0 ends with
+// a's result, lane 32 with b's, lane 16 with c's, lane 48 with d's: about a
+// quarter of the instructions of four separate trees.
+template <class F>
+__device__ __forceinline__ int wave_tree4(int a, int b, int c, int d, F op) {
+    auto p32 = [](int x, int y) {
+        return __builtin_amdgcn_permlane32_swap((unsigned)x, (unsigned)y, false, false);
+    };
+    const auto ab = p32(a, b), cd = p32(c, d);
+    const int u = op((int)ab[0], (int)ab[1]), w = op((int)cd[0], (int)cd[1]);
+    const auto r = __builtin_amdgcn_permlane16_swap((unsigned)u, (unsigned)w, false, false);
+    int v = op((int)r[0], (int)r[1]);
+    v = op(v, row_down<8>(v));
+    v = op(v, row_down<4>(v));
+    v = op(v, row_down<2>(v));
+    return op(v, row_down<1>(v));
+}
+__device__ __forceinline__ double wave_sum4(double a, double b, double c, double d) {
+    auto p32 = [](double x, double y) {
+        const auto l = __builtin_amdgcn_permlane32_swap(
+            (unsigned)__double2loint(x), (unsigned)__double2loint(y), false, false);
+        const auto h = __builtin_amdgcn_permlane32_swap(
+            (unsigned)__double2hiint(x), (unsigned)__double2hiint(y), false, false);
+        return __hiloint2double((int)h[0], (int)l[0]) + __hiloint2double((int)h[1], (int)l[1]);
+    };
+    const double u = p32(a, b), w = p32(c, d);
+    const auto l = __builtin_amdgcn_permlane16_swap(
+        (unsigned)__double2loint(u), (unsigned)__double2loint(w), false, false);
+    const auto h = __builtin_amdgcn_permlane16_swap(
+        (unsigned)__double2hiint(u), (unsigned)__double2hiint(w), false, false);
+    double v = __hiloint2double((int)h[0], (int)l[0]) + __hiloint2double((int)h[1], (int)l[1]);
+    auto row = [](double x, auto f) {
+        return __hiloint2double(f(__double2hiint(x)), f(__double2loint(x)));
+    };
+    v += row(v, [](int x) { return row_down<8>(x); });
+    v += row(v, [](int x) { return row_down<4>(x); });
+    v += row(v, [](int x) { return row_down<2>(x); });
+    v += row(v, [](int x) { return row_down<1>(x); });
     return v;
 }
 __device__ __forceinline__ int wave_min(int v) {
-#pragma unroll
-    for (int d = kWave / 2; d > 0; d >>= 1) v = min(v, __shfl_down(v, d, kWave));
-    return v;
+    return wave_tree(v, [](int a, int b) { return min(a, b); });
 }
 __device__ __forceinline__ int wave_max(int v) {
-#pragma unroll
-    for (int d = kWave / 2; d > 0; d >>= 1) v = max(v, __shfl_down(v, d, kWave));
-    return v;
+    return wave_tree(v, [](int a, int b) { return max(a, b); });
 }
 
 // ---- moments of one cell's window with the update's thread mapping ----
