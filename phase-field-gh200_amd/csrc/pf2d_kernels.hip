@@ -1,21 +1,20 @@
 // gfx950 kernels of the 2D per-cell phase-field update and their C ABI.
 //
-// The step is one persistent work-queue launch: one 1024-thread workgroup per
-// compute unit takes cell tickets from a device cursor (reference step_body,
-// src/kernels.cu:948-1024) and advances one cell at a time through:
-//   A  stage the cell's active window of phi in LDS (16 B vector loads) and
-//      hold its S window in VGPRs; a column-walk 3x3 register stencil gives
-//      the interaction integral terms and, for every pixel, the passive
-//      right-hand side and both gradients, which stay in VGPRs;
-//   -  fixed-order fp64 reduction (64-lane tree, 16 wavefronts ascending) of
-//      the interaction integral and the cell velocity;
+// The step is one persistent work-queue launch: two 8-wave workgroups per
+// compute unit (one of 16 waves when there are fewer cells) take cells from a
+// device cursor (reference step_body, src/kernels.cu:948-1024) and advance
+// one cell at a time through:
+//   A  a column walk with a 3x3 register stencil over rows that each wave
+//      stages in LDS for itself; it gives the interaction integral terms and,
+//      for every pixel, the passive right-hand side, which stays in VGPRs;
+//   -  fixed-order fp64 reduction (64-lane tree, 16 logical waves ascending)
+//      of the interaction integral and the cell velocity;
 //   B  the explicit Euler update from the held terms plus advection, the
 //      shifted store, the Q5.27 scatter into the next S with integer atomics,
 //      and the moments/support/phi_max of the stored field;
 //   -  a second fixed-order reduction and the CellState commit.
-// Classes 0-3 take the LDS path; classes 4 (224x224, larger than gfx950's
-// 160 KB LDS once fp32 phi is staged) and 5 (fallback) read the tile from
-// global memory.
+// Classes 0-3 take this walk; the rare classes 4 (224x224) and 5 (fallback)
+// read the tile from global memory.
 //
 // Arithmetic follows the reference's host semantics exactly: binary32
 // operations in source order with no multiply-add contraction (the build
@@ -969,6 +968,11 @@ __device__ void cell_walk(const pfh2d_step_args& A, int n, unsigned long long st
             if constexpr (kObs == 2)
                 observe_pixel(ob, g.x(), g.y0() + k, q.cC, q.cE, q.cW, q.nC, q.sC, q.nE, q.nW,
                               q.sE, q.sW, So, gam, dwC, repC, c.og2iv, c.ocx, c.ocy);
+            // added up here: sunk to the end of the pass, the sums would keep
+            // every row's stencil live
+            if constexpr (kObs == 2)
+                asm volatile("" : "+v"(ob.gx), "+v"(ob.gy), "+v"(ob.kx), "+v"(ob.ky),
+                                  "+v"(ob.bx), "+v"(ob.by));
             if (wave_any(So != 0.0f)) {
                 pas[v][k] = with_repulsion(head, repC, q.cC, So);
                 const float gxv = 0.5f * (q.cE - q.cW);

@@ -338,3 +338,29 @@ def test_restart_equivalence(sim_mod):
     assert np.array_equal(a.phi_now().view(np.uint32), c.phi_now().view(np.uint32))
     assert np.array_equal(a.S_now(), c.S_now())
     assert_cells_equal(a.cells(), c.cells(), "restart")
+
+
+@pytest.mark.parametrize("grid,step0", [(11, 99), (12, 99), (5, 98), (4, 99)])
+def test_workgroup_shapes_agree_on_every_class(sim_mod, oracle, grid, step0):
+    """Both sides of the launch rule on the forced state of 12 cells: fewer
+    compute units than cells (two 8-wave workgroups each, two logical waves
+    per wave) and one for each cell (16 waves), with every window class,
+    recentring shifts, class changes and the full-moment step 99 -> 100, whose
+    perimeter is read back from the stored tile."""
+    wl, phi, S, cells, cls = _forced_state(oracle)
+    cells = cells.copy()
+    # push two centroids off the window centre: shifts in both directions
+    cells["Cx"][0] += 3.0 * cells["V"][0]
+    cells["Cy"][3] -= 2.0 * cells["V"][3]
+    say(f"launch shapes: 12 cells of every class on {grid} compute units, step {step0}")
+    sim = sim_mod.Sim2D(wl)
+    sim.grid = grid
+    orc = oracle.OracleSim2D(wl, threads=8)
+    sim.load_state(phi, S, cells, cls, step0)
+    orc.load_state(phi, S, cells, cls, step0)
+    for k in range(3):
+        sim.step(1)
+        orc.step(1)
+        sim.sync()
+        assert_state_equal(sim, orc, f"grid {grid}, step {step0 + k + 1}")
+    assert sim.cells()["shift_ctr"].sum() > 0
