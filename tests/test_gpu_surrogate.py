@@ -623,3 +623,89 @@ def test_long_run_stays_within_tolerance_of_plain():
     assert r["rel_l2_vs_plain_max"] <= 1e-3
     assert r["accepted_cell_fraction"] > 0.0
 
+
+
+def _bf16(x: torch.Tensor) -> torch.Tensor:
+    return x.to(torch.bfloat16)
+
+
+@pytest.mark.parametrize("cin,crops,shift", [(8, 1, 0), (8, 3, 1), (32, 2, 0), (32, 3, 1)])
+def test_training_kernels_on_odd_batches(cin, crops, shift):
+    """The convolution (Y and the mask aligned for 16 B accesses or one
+    element off), the weight gradients and the output layer's backward on 1-3
+    crops, against plain fp64 sums on the CPU: corners, edges and every
+    32-pixel block boundary included. Bounds: bf16 results one rounding
+    (2^-8 of the value) plus fp32 sums; sums of n fp32 terms n 2^-24 of the sum
+    of their magnitudes."""
+    from pfh import abi
+    lib, dev = abi.load(), "cuda:0"
+    gen = torch.Generator().manual_seed(100 * cin + crops)
+    rnd = lambda *s: _bf16(torch.randn(*s, generator=gen))          # noqa: E731
+    X, W = rnd(crops, 96, 96, cin), _bf16(rnd(32, 9, cin) * 0.1)
+    dY, H = rnd(crops, 96, 96, 32), rnd(crops, 96, 96, 32)
+    bias, g = torch.randn(32, generator=gen), torch.randn(crops, 96, 96, generator=gen)
+    W4 = torch.randn(9, 32, generator=gen)
+    up = lambda t: t.contiguous().to(dev)                            # noqa: E731
+
+    def taps(a):                         # [9, crops, 96, 96, c], a at p + off(tap)
+        p = torch.nn.functional.pad(a.double(), (0, 0, 1, 1, 1, 1))
+        return torch.stack([p[:, ky:ky + 96, kx:kx + 96] for ky in range(3) for kx in range(3)])
+
+    # convolution, ReLU and mask
+    Xd, Wd, bd = up(X), up(W), up(bias)
+    room = torch.zeros(dY.numel() + 8, dtype=torch.bfloat16, device=dev)
+    mask_room = torch.zeros_like(room)
+    Y = room[shift:shift + dY.numel()]
+    mask = mask_room[shift:shift + dY.numel()]
+    mask.copy_(up(H).view(-1))
+    abi.check(lib.pfh_sur_conv(cin, Xd.data_ptr(), Wd.data_ptr(), bd.data_ptr(),
+                               mask.data_ptr(), Y.data_ptr(), crops, 1, None), "conv")
+    xt = taps(X)
+    ref = torch.einsum("tnyxi,oti->nyxo", xt, W.double()) + bias.double()
+    mag = torch.einsum("tnyxi,oti->nyxo", xt.abs(), W.double().abs()) + bias.double().abs()
+    ref = torch.where(H.double() > 0, ref, 0.0).clamp(min=0.0)
+    err = (Y.view(ref.shape).cpu().double() - ref).abs()
+    assert bool((err <= ref.abs() * 2.0 ** -8 + mag * (9 * cin * 2.0 ** -24)).all())
+    assert float(room[:shift].abs().sum()) == 0.0 and float(room[shift + dY.numel():].abs().sum()) == 0.0
+
+    # weight gradient, per crop
+    width = 32 * 9 * cin + 32
+    part = torch.zeros(crops * width, dtype=torch.float32, device=dev)
+    dYd = up(dY)
+    abi.check(lib.pfh_sur_wgrad(cin, dYd.data_ptr(), Xd.data_ptr(), part.data_ptr(), crops,
+                                None), "wgrad")
+    got = part.cpu().double().view(crops, width)
+    dw = torch.einsum("nyxo,tnyxi->noti", dY.double(), xt)
+    dm = torch.einsum("nyxo,tnyxi->noti", dY.double().abs(), xt.abs())
+    lim = 9216 * 2.0 ** -24
+    assert bool(((got[:, :-32].view(dw.shape) - dw).abs() <= lim * dm).all())
+    db, bm = dY.double().sum((1, 2)), dY.double().abs().sum((1, 2))
+    assert bool(((got[:, -32:] - db).abs() <= lim * bm).all())
+
+    # output layer's backward
+    gd, Hd, W4d = up(g), up(H), up(W4)
+    dH = torch.zeros_like(Hd)
+    p4 = torch.zeros(crops * 289, dtype=torch.float32, device=dev)
+    abi.check(lib.pfh_sur_out_bwd(gd.data_ptr(), Hd.data_ptr(), W4d.data_ptr(), dH.data_ptr(),
+                                  p4.data_ptr(), crops, None), "out_bwd")
+    gt = taps(g[..., None]).flip(0)[..., 0]                          # g at q - off(tap)
+    ref = torch.einsum("tnyx,tc->nyxc", gt, W4.double())
+    mag = torch.einsum("tnyx,tc->nyxc", gt.abs(), W4.double().abs())
+    ref = torch.where(H.double() > 0, ref, 0.0)
+    err = (dH.cpu().double() - ref).abs()
+    assert bool((err <= ref.abs() * 2.0 ** -8 + mag * (9 * 2.0 ** -24)).all())
+    got = p4.cpu().double().view(crops, 289)
+    dw4 = torch.einsum("tnyx,nyxc->ntc", gt, H.double())
+    m4 = torch.einsum("tnyx,nyxc->ntc", gt.abs(), H.double().abs())
+    assert bool(((got[:, :-1].view(dw4.shape) - dw4).abs() <= lim * m4).all())
+    assert bool(((got[:, -1] - g.double().sum((1, 2))).abs()
+                 <= lim * g.double().abs().sum((1, 2))).all())
+
+    # the reduction over crops keeps the ascending order
+    out = torch.zeros(289, dtype=torch.float32, device=dev)
+    many = torch.randn(37 * 289, generator=gen).to(dev)
+    abi.check(lib.pfh_sur_reduce(many.data_ptr(), 37, 289, out.data_ptr(), None), "reduce")
+    acc = torch.zeros(289)
+    for row in many.cpu().view(37, 289):
+        acc = acc + row
+    assert torch.equal(out.cpu(), acc)
