@@ -166,6 +166,40 @@ struct ConvShape {
     static constexpr int HALO = (kRowsPerItem + 2) * kHaloCols;
 };
 
+// The halo tile of an item (6 rows x 98 columns, zeros outside the crop),
+// loaded into registers and stored to LDS by a 256-thread workgroup.
+template <int CIN>
+struct HaloTile {
+    static constexpr int CH8 = CIN / 8;
+    static constexpr int CHUNKS = (kRowsPerItem + 2) * kHaloCols * CH8;
+    static constexpr int PER = (CHUNKS + 255) / 256;
+    u32x4 v[PER];
+    __device__ __forceinline__ void load(const bf16_t* X, int item, int items) {
+        if (item >= items) return;
+        const int crop = item / kItemsPerCrop;
+        const int y0 = (item - crop * kItemsPerCrop) * kRowsPerItem;
+#pragma unroll
+        for (int u = 0; u < PER; ++u) {
+            const int i = (int)threadIdx.x + 256 * u;
+            const int px = i / CH8, c8 = i - px * CH8;
+            const int r = px / kHaloCols, cc = px - r * kHaloCols;
+            const int y = y0 - 1 + r, x = cc - 1;
+            v[u] = u32x4{0u, 0u, 0u, 0u};
+            if (i < CHUNKS && (unsigned)y < (unsigned)kCrop && (unsigned)x < (unsigned)kCrop)
+                v[u] = *reinterpret_cast<const u32x4*>(
+                    X + (((size_t)crop * kCrop + y) * kCrop + x) * CIN + 8 * c8);
+        }
+    }
+    __device__ __forceinline__ void store(bf16_t* tile, int pitch) const {
+#pragma unroll
+        for (int u = 0; u < PER; ++u) {
+            const int i = (int)threadIdx.x + 256 * u;
+            const int px = i / CH8, c8 = i - px * CH8;
+            if (i < CHUNKS) *reinterpret_cast<u32x4*>(tile + px * pitch + 8 * c8) = v[u];
+        }
+    }
+};
+
 template <int CIN>
 __device__ __forceinline__ f32x16 mfma_step(const bf16_t* a, const bf16_t* b, f32x16 acc) {
     if constexpr (CIN == 8) {
@@ -185,7 +219,8 @@ __device__ __forceinline__ f32x16 mfma_step(const bf16_t* a, const bf16_t* b, f3
 // lane's 16 accumulators are 16 consecutive channels of one pixel: with kVec
 // (Y and the mask 16 B aligned) the mask is two 16 B loads and the result two
 // 16 B stores per pixel half, where a lane per channel took 16 stores of 2 B
-// (128 crops, 32 channels: 101 -> 58 us, 2.6 TB/s of input and output).
+// (with the next tile in flight during the products, 128 crops of 32 channels:
+// 101 -> 45 us, 3.4 TB/s of input and output).
 template <int CIN, bool kVec>
 __global__ __launch_bounds__(256) void k_sur_conv(const bf16_t* X, const bf16_t* W,
                                                   const float* bias, const bf16_t* mask,
@@ -212,23 +247,17 @@ __global__ __launch_bounds__(256) void k_sur_conv(const bf16_t* X, const bf16_t*
     }
 
     const int items = ncrops * kItemsPerCrop;
+    // rows y0-1 .. y0+4, columns -1 .. 96 of an item, in 8-channel chunks: the
+    // next item's travel through registers while this one is multiplied
+    HaloTile<CIN> halo;
+    halo.load(X, (int)blockIdx.x, items);
     for (int item = (int)blockIdx.x; item < items; item += (int)gridDim.x) {
         const int crop = item / kItemsPerCrop;
         const int y0 = (item - crop * kItemsPerCrop) * kRowsPerItem;
         __syncthreads();
-        // stage rows y0-1 .. y0+4, columns -1 .. 96 (8-channel chunks)
-        constexpr int CH8 = CIN / 8;
-        for (int i = tid; i < SH::HALO * CH8; i += 256) {
-            const int px = i / CH8, c8 = i - px * CH8;
-            const int r = px / kHaloCols, cc = px - r * kHaloCols;
-            const int y = y0 - 1 + r, x = cc - 1;
-            u32x4 v = {0u, 0u, 0u, 0u};
-            if ((unsigned)y < (unsigned)kCrop && (unsigned)x < (unsigned)kCrop)
-                v = *reinterpret_cast<const u32x4*>(
-                    X + (((size_t)crop * kCrop + y) * kCrop + x) * CIN + 8 * c8);
-            *reinterpret_cast<u32x4*>(xl + px * SH::PIX + 8 * c8) = v;
-        }
+        halo.store(xl, SH::PIX);
         __syncthreads();
+        halo.load(X, item + (int)gridDim.x, items);
 
         f32x16 acc0 = {}, acc1 = {}, acc2 = {};
 #pragma unroll 3
@@ -299,7 +328,7 @@ __global__ void k_sur_round_bf16(const float* x, uint32_t* y, int npairs) {
 // Persistent over (crop, 4-row block) items like k_sur_conv: the 6 x 98
 // halo tile of h3 is staged in LDS. Four lanes share a pixel, eight channels
 // each, whose 72 weights stay in registers (a lane per pixel read all 288
-// from LDS for every pixel: 60 -> 45 us for 128 crops); fp32 sums, the four
+// from LDS for every pixel: 60 -> 37 us for 128 crops, the next tile in flight); fp32 sums, the four
 // lanes' partial sums added pairwise.
 __global__ __launch_bounds__(256) void k_sur_out(const bf16_t* H, const float* W4, float b4,
                                                  const float* phic, float* dphi, float* out,
@@ -314,21 +343,15 @@ __global__ __launch_bounds__(256) void k_sur_out(const bf16_t* H, const float* W
 #pragma unroll
         for (int k = 0; k < 8; ++k) w[t][k] = W4[t * kCH + 8 * c8 + k];
     const int items = ncrops * kItemsPerCrop;
+    HaloTile<kCH> halo;
+    halo.load(H, (int)blockIdx.x, items);
     for (int item = (int)blockIdx.x; item < items; item += (int)gridDim.x) {
         const int crop = item / kItemsPerCrop;
         const int y0 = (item - crop * kItemsPerCrop) * kRowsPerItem;
         __syncthreads();
-        for (int i = tid; i < (kRowsPerItem + 2) * kHaloCols * 4; i += 256) {
-            const int px = i >> 2, c8i = i & 3;
-            const int r = px / kHaloCols, cc = px - r * kHaloCols;
-            const int y = y0 - 1 + r, x = cc - 1;
-            u32x4 v = {0u, 0u, 0u, 0u};
-            if ((unsigned)y < (unsigned)kCrop && (unsigned)x < (unsigned)kCrop)
-                v = *reinterpret_cast<const u32x4*>(
-                    H + (((size_t)crop * kCrop + y) * kCrop + x) * kCH + 8 * c8i);
-            *reinterpret_cast<u32x4*>(hl + px * PIXP + 8 * c8i) = v;
-        }
+        halo.store(hl, PIXP);
         __syncthreads();
+        halo.load(H, item + (int)gridDim.x, items);
         for (int q = tid >> 2; q < kRowsPerItem * kCrop; q += 64) {
             const int r = q / kCrop, x = q - r * kCrop;
             const bf16_t* h = hl + (r * kHaloCols + x) * PIXP + 8 * c8;
@@ -802,22 +825,35 @@ __global__ __launch_bounds__(kIT, 1) void k_sur_infer(const InferArgs A) {
     }
 }
 
-// Per-crop loss partial and g = 2 (dphi - target) / count
-__global__ __launch_bounds__(256) void k_sur_loss(const float* dphi, const float* target,
-                                                  float* g, double* crop_loss, float scale) {
-    __shared__ double red[4];
+// Per-crop loss partial and g = 2 (dphi - target) / count: one 1024-thread
+// workgroup per crop, all nine of a thread's pixels in flight (with 256
+// threads and one pixel at a time the loop waited for memory: 17 -> 5 us for
+// 128 crops).
+constexpr int kLossNT = 1024;
+__global__ __launch_bounds__(kLossNT) void k_sur_loss(const float* dphi, const float* target,
+                                                      float* g, double* crop_loss, float scale) {
+    __shared__ double red[kLossNT / 64];
     const int n = (int)blockIdx.x;
+    constexpr int PER = kCropPix / kLossNT;
+    static_assert(PER * kLossNT == kCropPix, "whole pixels per thread");
+    const size_t base = (size_t)n * kCropPix + threadIdx.x;
+    float e[PER];
+#pragma unroll
+    for (int k = 0; k < PER; ++k) e[k] = dphi[base + k * kLossNT] - target[base + k * kLossNT];
     double acc = 0.0;
-    for (int p = (int)threadIdx.x; p < kCropPix; p += 256) {
-        const size_t i = (size_t)n * kCropPix + p;
-        const float e = dphi[i] - target[i];
-        g[i] = scale * e;
-        acc += (double)e * (double)e;
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+        g[base + k * kLossNT] = scale * e[k];
+        acc += (double)e[k] * (double)e[k];
     }
     acc = pfh::wave_sum(acc);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
     __syncthreads();
-    if (threadIdx.x == 0) crop_loss[n] = ((red[0] + red[1]) + red[2]) + red[3];
+    if (threadIdx.x == 0) {
+        double s = 0.0;
+        for (int w = 0; w < kLossNT / 64; ++w) s += red[w];
+        crop_loss[n] = s;
+    }
 }
 
 // Backward of the output layer in one pass over h3, one 1024-thread workgroup
@@ -1835,7 +1871,7 @@ int pfh_sur_round_bf16(const float* x, uint16_t* y, int n, void* stream) {
 int pfh_sur_loss(const float* dphi, const float* target, float* g, double* crop_loss,
                  int ncrops, float scale, void* stream) {
     if (!dphi || !target || !g || !crop_loss || ncrops <= 0) return invalid("sur_loss");
-    hipLaunchKernelGGL(sur::k_sur_loss, dim3((unsigned)ncrops), dim3(256), 0,
+    hipLaunchKernelGGL(sur::k_sur_loss, dim3((unsigned)ncrops), dim3(sur::kLossNT), 0,
                        as_stream(stream), dphi, target, g, crop_loss, scale);
     return launch_status("k_sur_loss");
 }
