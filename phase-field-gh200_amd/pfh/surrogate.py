@@ -76,8 +76,11 @@ class Net:
             self.views[k] = self.w[o:o + SIZES[k]]
             self.gviews[k] = self.g[o:o + SIZES[k]]
             o += SIZES[k]
-        self.wb = {k: torch.zeros(SIZES[k], dtype=torch.int16, device=self.dev)
-                   for k in ("W1", "W2", "W3")}
+        # bf16 copies: one vector laid out like w, so that the Adam kernel
+        # writes them with the update (every MFMA tensor starts 16 B aligned)
+        self.wb_all = torch.zeros(NPARAM, dtype=torch.int16, device=self.dev)
+        off = {k: self.views[k].storage_offset() for k in ORDER}
+        self.wb = {k: self.wb_all[off[k]:off[k] + SIZES[k]] for k in ("W1", "W2", "W3")}
         self.wflip = {k: torch.zeros(SIZES[k], dtype=torch.int16, device=self.dev)
                       for k in ("W2", "W3")}
         self._init(seed)
@@ -109,6 +112,9 @@ class Net:
         """bf16 copies and the tap-flipped backward-data weights."""
         for k in ("W1", "W2", "W3"):
             self.wb[k].copy_(bf16_bits_torch(self.views[k]))
+        self._flip()
+
+    def _flip(self) -> None:
         for k in ("W2", "W3"):
             abi.check(self.lib.pfh_sur_flip(_ptr(self.wb[k]), _ptr(self.wflip[k]), None),
                       "pfh_sur_flip")
@@ -219,21 +225,17 @@ def backward(net: Net, ws: Workspace, n: int, target: torch.Tensor, X0=None, str
     # output layer: dh3 and dW4/db4 (partials laid out [n][289])
     abi.check(lib.pfh_sur_out_bwd(_ptr(ws.g), _ptr(ws.h[2]), _ptr(net.views["W4"]),
                                   _ptr(ws.dh[2]), _ptr(ws.part), n, stream), "out_bwd")
-    tmp = torch.empty(9 * CH + 1, dtype=torch.float32, device=net.dev)
-    abi.check(lib.pfh_sur_reduce(_ptr(ws.part), n, 9 * CH + 1, _ptr(tmp), stream), "reduce4")
-    gv["W4"].copy_(tmp[:9 * CH])
-    gv["b4"].copy_(tmp[9 * CH:])
+    # (a layer's weights and bias lie together in g as in the partials)
+    abi.check(lib.pfh_sur_reduce(_ptr(ws.part), n, 9 * CH + 1, _ptr(gv["W4"]), stream),
+              "reduce4")
     # hidden layers 3, 2, 1
     layers = [("W3", "b3", ws.h[1], 32), ("W2", "b2", ws.h[0], 32), ("W1", "b1", X0, 8)]
     dys = [ws.dh[2], ws.dh[1], ws.dh[0]]
-    for i, (wk, bk, Xin, cin) in enumerate(layers):
+    for i, (wk, _, Xin, cin) in enumerate(layers):
         dY = dys[i]
         width = CH * 9 * cin + CH
         abi.check(lib.pfh_sur_wgrad(cin, _ptr(dY), _ptr(Xin), _ptr(ws.part), n, stream), "wgrad")
-        red = torch.empty(width, dtype=torch.float32, device=net.dev)
-        abi.check(lib.pfh_sur_reduce(_ptr(ws.part), n, width, _ptr(red), stream), "reduce")
-        gv[wk].copy_(red[:CH * 9 * cin])
-        gv[bk].copy_(red[CH * 9 * cin:])
+        abi.check(lib.pfh_sur_reduce(_ptr(ws.part), n, width, _ptr(gv[wk]), stream), "reduce")
         if cin == 32:
             # dX = conv(dY, flipped W) masked by the layer input's ReLU
             abi.check(lib.pfh_sur_conv(32, _ptr(dY), _ptr(net.wflip[wk]), None, _ptr(Xin),
@@ -245,9 +247,10 @@ def adam_step(net: Net, lr: float, b1=0.9, b2=0.999, eps=1e-8) -> None:
     net.t += 1
     c1 = 1.0 - b1 ** net.t
     c2 = 1.0 - b2 ** net.t
-    abi.check(net.lib.pfh_sur_adam(_ptr(net.w), _ptr(net.g), _ptr(net.m), _ptr(net.v), None,
-                                   NPARAM, lr, b1, b2, eps, c1, c2, None), "adam")
-    net.refresh()
+    abi.check(net.lib.pfh_sur_adam(_ptr(net.w), _ptr(net.g), _ptr(net.m), _ptr(net.v),
+                                   _ptr(net.wb_all), NPARAM, lr, b1, b2, eps, c1, c2, None),
+              "adam")
+    net._flip()
 
 
 # ---------------------------------------------------------------------------
