@@ -644,6 +644,254 @@ __device__ __noinline__ void clip_voxel(const ClipArgs a, pfh3d_cell_state* cs,
     if (fabsf(nx) > kEps) raise3(cs, a.flags, PFH3D_FLAG_DESTINATION_CLIP);
 }
 
+// ---------------------------------------------------------------------------
+// update without a recentring shift (almost every step of almost every cell):
+// the source voxel is the destination voxel. Against the general walk below:
+//   - a plane of the part lies in LDS as it does in memory, so a lane reads
+//     its row of six values with one 16 B and two 4 B reads;
+//   - every plane load is unconditional (a buffer descriptor over the cube
+//     gives zeros outside it);
+//   - the lane's four S words are one 16 B load, except where the brick wraps
+//     around the domain in x (kWrapX);
+//   - the four results are computed without branches; a plane in which any
+//     value is not finite or above the clamp, decided by one test per wave, is
+//     redone voxel by voxel in the reference's order;
+//   - the scatter goes through LDS so that a wave's four atomic instructions
+//     each cover 64 consecutive words of the wave's 256 voxels: a lane's own
+//     four words touch four times as many lines per instruction (1.32 M atomic
+//     requests per 256^3 / 128-cell step before).
+// ---------------------------------------------------------------------------
+constexpr uint32_t kNone = 0x80000000u;          // past every descriptor's end
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc3(const void* p, uint32_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, 0x00020000);
+}
+__device__ __forceinline__ float uni(float v) {
+    return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(v)));
+}
+__device__ __forceinline__ bool wave_any(bool v) {
+    return __builtin_amdgcn_ballot_w64(v) != 0ull;
+}
+typedef u32x4 u32x4_4 __attribute__((aligned(4)));
+
+template <bool kWrapX>
+__device__ __forceinline__ void update_plain(const pfh3d_step_args& a, pfh3d_cell_state* cs,
+                                             const CellCoef& kc, int n, int zb, int ze, int yb,
+                                             int ye, int ox, int oy, int oz, float* lds) {
+    const int B = a.B, L = a.L, P = a.P;
+    const int tid = (int)threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int gpr = B / 4, rows = ye - yb, G = rows * gpr, units = (rows + 2) * gpr;
+    const bool act = tid < G;
+    const int r_ = act ? tid / gpr : 0;
+    const int gx0 = act ? 4 * (tid - r_ * gpr) : 0;
+    const int PX = B + 8, PL = (rows + 2) * PX;
+    const uint32_t plane = 4u * (uint32_t)(B * B);
+    const uint32_t words = plane * (uint32_t)B;
+    const size_t cube = (size_t)n * B * B * B;
+    const __amdgpu_buffer_rsrc_t bin = rsrc3(a.phi_in + cube, words);
+    const __amdgpu_buffer_rsrc_t bout = rsrc3(a.phi_out + cube, words);
+    const float gamma = uni(kc.gamma), bulk = uni(kc.bulk), volume = uni(kc.volume);
+    const float vx = uni(kc.vx), vy = uni(kc.vy), vz = uni(kc.vz);
+    const float dt = uni(kc.dt), ic = uni(kc.ic);
+    const CellCoef k{gamma, bulk, volume, vx, vy, vz, dt, ic};
+
+    // the part's rows and a halo row on each side: up to two groups a lane
+    uint32_t so[2];
+    int sl[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const int i = tid + u * (int)blockDim.x;
+        const int r = i / gpr, g = i - r * gpr, y = yb - 1 + r;
+        so[u] = i < units && (unsigned)y < (unsigned)B ? 4u * (uint32_t)(y * B + 4 * g) : kNone;
+        sl[u] = i < units ? r * PX + 4 + 4 * g : -1;
+    }
+    const bool two = units > (int)blockDim.x;
+    auto load_plane = [&](int p, u32x4 (&v)[2]) {
+        const uint32_t o = (uint32_t)p * plane;
+        v[0] = __builtin_amdgcn_raw_buffer_load_b128(bin, (int)(so[0] + o), 0, 0);
+        if (two) v[1] = __builtin_amdgcn_raw_buffer_load_b128(bin, (int)(so[1] + o), 0, 0);
+    };
+    auto stage = [&](float* pl, const u32x4 (&v)[2]) {
+        if (sl[0] >= 0) *reinterpret_cast<u32x4*>(pl + sl[0]) = v[0];
+        if (two && sl[1] >= 0) *reinterpret_cast<u32x4*>(pl + sl[1]) = v[1];
+    };
+    uint32_t* const qbuf = reinterpret_cast<uint32_t*>(lds + 2 * PL) + 256 * wave;
+    for (int i = tid; i < 2 * PL; i += (int)blockDim.x) lds[i] = 0.0f;
+
+    // S byte offsets within a plane: the lane's row of four words, and the
+    // four words it adds to (word 64 j + lane of the wave's 256)
+    auto s_off = [&](int t, int e) -> uint32_t {
+        const int r = t / gpr, x = 4 * (t - r * gpr) + e;
+        return 4u * (uint32_t)(wrap_off(oy, yb + r, L) * P + wrap_off(ox, x, L));
+    };
+    uint32_t si[4], sa[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        si[j] = s_off(act ? tid : 0, j);
+        const int t = 64 * wave + 16 * j + (lane >> 2);
+        sa[j] = s_off(t < G ? t : 0, lane & 3);
+    }
+    auto s_plane = [&](const uint32_t* S, int z) {
+        return reinterpret_cast<const PFH_GLOBAL char*>(gptr(const_cast<uint32_t*>(S))) +
+               4u * (size_t)wrap_off(oz, z, L) * (size_t)L * (size_t)P;
+    };
+    auto load_s = [&](int z, uint32_t (&v)[4]) {
+        const PFH_GLOBAL char* base = s_plane(a.S_in, z);
+        if constexpr (kWrapX) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                v[j] = *reinterpret_cast<const PFH_GLOBAL uint32_t*>(base + si[j]);
+        } else {
+            const u32x4 w = *reinterpret_cast<const PFH_GLOBAL u32x4_4*>(base + si[0]);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[j] = w[j];
+        }
+    };
+
+    const int pbeg = zb - 1, pcount = ze - zb + 2;
+    u32x4 R[2], Rn[2];
+    load_plane(pbeg, R);
+    load_plane(pbeg + 1, Rn);
+    __syncthreads();
+    stage(lds, R);
+    __syncthreads();
+
+    float T[4] = {0.f, 0.f, 0.f, 0.f}, Q1p[4] = {0.f, 0.f, 0.f, 0.f};
+    float Am2[4] = {0.f, 0.f, 0.f, 0.f}, Am1[4] = {0.f, 0.f, 0.f, 0.f};
+    float gxm[4] = {0.f, 0.f, 0.f, 0.f}, gym[4] = {0.f, 0.f, 0.f, 0.f};
+    uint32_t Su[4] = {0u, 0u, 0u, 0u};
+    uint32_t pold[4] = {0u, 0u, 0u, 0u}, pq[4] = {0u, 0u, 0u, 0u};
+    uint32_t n_nonfin = 0u, n_neg = 0u, n_clamp = 0u, n_over = 0u;
+    const int rd = (r_ + 1) * PX + 4 + gx0;
+    const uint32_t dst = act ? 4u * (uint32_t)((yb + r_) * B + gx0) : kNone;
+    // the previous plane's scatters: an addend is at most 2^29
+    auto check_overflow = [&]() {
+        const uint32_t big = max(max(pold[0], pold[1]), max(pold[2], pold[3]));
+        if (big >= 0xE0000000u) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) n_over += pold[j] > 0xffffffffu - pq[j] ? 1u : 0u;
+        }
+    };
+
+    for (int i = 0; i < pcount; ++i) {
+        const int p = pbeg + i;
+        const float* pl = lds + (i & 1) * PL + rd;
+        u32x4 Rnn[2];
+        load_plane(i + 2 < pcount ? p + 2 : B, Rnn);     // past the slab: zeros
+        uint32_t Sun[4] = {0u, 0u, 0u, 0u};
+        if (i >= 1 && i + 1 < pcount) load_s(p, Sun);
+        float A[4], Q1[4], Q0[4], GX[4], GY[4];
+        {
+            float r0[6], r1[6], r2[6];
+            auto row = [&](const float* q, float (&r)[6]) {
+                const f32x4 v = *reinterpret_cast<const f32x4*>(q);
+                r[0] = q[-1];
+                r[1] = v[0]; r[2] = v[1]; r[3] = v[2]; r[4] = v[3];
+                r[5] = q[4];
+            };
+            row(pl - PX, r0);
+            row(pl, r1);
+            row(pl + PX, r2);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const PlaneSums q = plane_sums(r0[j], r0[j + 1], r0[j + 2], r1[j], r1[j + 1],
+                                               r1[j + 2], r2[j], r2[j + 1], r2[j + 2]);
+                A[j] = q.A; Q1[j] = q.q1; Q0[j] = q.q0; GX[j] = q.gx; GY[j] = q.gy;
+            }
+        }
+        if (i >= 2) {
+            // destination plane p - 1
+            float nx[4];
+            uint32_t q[4];
+            bool neg = false, zero = false;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const float c = Am1[j];
+                const float lap = (T[j] + Q1[j]) * (float)(1.0 / 30.0);
+                const float gz = 0.5f * (A[j] - Am2[j]);
+                const uint32_t own = q_of(c);
+                const bool ng = Su[j] < own;
+                neg |= ng;
+                zero |= c == 0.0f;
+                const float other = ng ? 0.0f : (float)(Su[j] - own) * pfh::kQInv;
+                nx[j] = rhs_next(k, c, lap, gxm[j], gym[j], gz, other);
+            }
+            // |nx| above 2 (the clamp's square root) or not finite, S below the
+            // cell's own share, or a voxel that may be exactly empty
+            const float top = fmaxf(fmaxf(fabsf(nx[0]), fabsf(nx[1])),
+                                    fmaxf(fabsf(nx[2]), fabsf(nx[3])));
+            const float all = (nx[0] + nx[1]) + (nx[2] + nx[3]);
+            const bool odd = neg || zero || !(top <= 2.0f) || !(fabsf(all) < INFINITY);
+            if (wave_any(odd)) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const float c = Am1[j];
+                    const float lap = (T[j] + Q1[j]) * (float)(1.0 / 30.0);
+                    const float gz = 0.5f * (A[j] - Am2[j]);
+                    const float v = nx[j];
+                    nx[j] = 0.0f;
+                    if (!act) continue;
+                    if (!isfinite(c)) { ++n_nonfin; continue; }
+                    if (c == 0.0f && lap == 0.0f && gxm[j] == 0.0f && gym[j] == 0.0f && gz == 0.0f)
+                        continue;
+                    n_neg += Su[j] < q_of(c) ? 1u : 0u;
+                    if (!isfinite(v)) { ++n_nonfin; continue; }
+                    n_clamp += v * v > pfh::kQClampPhiSq ? 1u : 0u;
+                    nx[j] = v;
+                }
+            }
+            check_overflow();
+#pragma unroll
+            for (int j = 0; j < 4; ++j) q[j] = act ? q_of(nx[j]) : 0u;
+            *reinterpret_cast<u32x4*>(qbuf + 4 * lane) = u32x4{q[0], q[1], q[2], q[3]};
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_raw_buffer_store_b128(
+                u32x4{__float_as_uint(nx[0]), __float_as_uint(nx[1]), __float_as_uint(nx[2]),
+                      __float_as_uint(nx[3])},
+                bout, (int)(dst + (uint32_t)(p - 1) * plane), 0, 0);
+            PFH_GLOBAL char* so_base = const_cast<PFH_GLOBAL char*>(s_plane(a.S_out, p - 1));
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                uint32_t w = qbuf[64 * j + lane];
+                pq[j] = w;
+                const bool add = w != 0u;
+                uint32_t off = sa[j];
+                asm volatile("" : "+v"(w), "+v"(off));   // the old word replaces the addend
+                if (add)
+                    w = __hip_atomic_fetch_add(
+                        reinterpret_cast<PFH_GLOBAL uint32_t*>(so_base + off), w,
+                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                pold[j] = w;
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            T[j] = Q1p[j] + Q0[j];
+            Q1p[j] = Q1[j];
+            Am2[j] = Am1[j];
+            Am1[j] = A[j];
+            gxm[j] = GX[j];
+            gym[j] = GY[j];
+            Su[j] = Sun[j];
+        }
+        if (i + 1 < pcount) stage(lds + ((i + 1) & 1) * PL, Rn);
+        pfh::lds_barrier();   // the plane buffers are the only shared data here
+        Rn[0] = Rnn[0];
+        Rn[1] = Rnn[1];
+    }
+    check_overflow();
+    auto raise = [&](uint32_t count, int f) {
+        if (count) {
+            atomicOr(&cs->flags, 1u << f);
+            atomicAdd(&a.flags[f], count);
+        }
+    };
+    raise(n_nonfin, PFH3D_FLAG_NONFINITE);
+    raise(n_neg, PFH3D_FLAG_S_NEGATIVE);
+    raise(n_clamp, PFH3D_FLAG_Q_CLAMP);
+    raise(n_over, PFH3D_FLAG_S_OVERFLOW);
+}
+
 __global__ __launch_bounds__(1024) void k3_update(const pfh3d_step_args a, const int K,
                                                   const int H) {
     extern __shared__ __align__(16) float lds[];
@@ -716,6 +964,13 @@ __global__ __launch_bounds__(1024) void k3_update(const pfh3d_step_args a, const
     kc.vz = cs->velocity_z;
     kc.dt = a.dt;
     kc.ic = a.interaction_coeff;
+    if ((sx | sy | sz) == 0) {
+        if (ox + B <= L)
+            update_plain<false>(a, cs, kc, n, zb, ze, yb, ye, ox, oy, oz, lds);
+        else
+            update_plain<true>(a, cs, kc, n, zb, ze, yb, ye, ox, oy, oz, lds);
+        return;
+    }
 
     const int GPU = B / 4 + 2 * kMarginG;            // words per sub-row
     const int PXU = update_row_pitch(B);
@@ -726,10 +981,16 @@ __global__ __launch_bounds__(1024) void k3_update(const pfh3d_step_args a, const
     // yb + sy - 1 + tid / gpr (the part's rows as the shift reads them, with
     // one halo row on each side); element e of the group goes to sub-row e
     const int g = gx0 >> 2;
-    const int srow = yb + sy - 1 + tid / gpr;
-    const bool stg = tid < (ye - yb + 2) * gpr && (unsigned)srow < (unsigned)B;
-    const int sg = tid % gpr;
-    const int stage = (srow + kMargin) * PXU + kMarginG + sg;
+    // (lanes past the workgroup's last in a second turn)
+    int srow[2], sg[2];
+    bool stg[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const int i = tid + u * NT;
+        srow[u] = yb + sy - 1 + i / gpr;
+        sg[u] = i % gpr;
+        stg[u] = i < (ye - yb + 2) * gpr && (unsigned)srow[u] < (unsigned)B;
+    }
     // reading: destination group (gx0.., gy_) reads source x = gx0 + sx + c - 1,
     // c = 0..5, of rows gy_ + sy - 1..gy_ + sy + 1: sub-row (sx + c - 1) & 3,
     // group g + ((sx + c - 1) >> 2), both offsets uniform
@@ -740,27 +1001,36 @@ __global__ __launch_bounds__(1024) void k3_update(const pfh3d_step_args a, const
         const int t = sx + c - 1;
         roff[c] = (t & 3) * GPU + (t >> 2);
     }
-    auto stage_plane = [&](float* plane, const f32x4& v) {
-        float* st = plane + stage;
-        st[0] = v[0];
-        st[GPU] = v[1];
-        st[2 * GPU] = v[2];
-        st[3 * GPU] = v[3];
+    struct Groups { f32x4 g[2]; };
+    auto stage_plane = [&](float* plane, const Groups& v) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            if (!stg[u]) continue;
+            float* st = plane + (srow[u] + kMargin) * PXU + kMarginG + sg[u];
+            st[0] = v.g[u][0];
+            st[GPU] = v.g[u][1];
+            st[2 * GPU] = v.g[u][2];
+            st[3 * GPU] = v.g[u][3];
+        }
     };
-    auto load_plane = [&](int p) -> f32x4 {
-        f32x4 v = {0.f, 0.f, 0.f, 0.f};
-        if (stg && (unsigned)p < (unsigned)B)
-            v = *reinterpret_cast<const PFH_GLOBAL f32x4*>(gsrc + (size_t)p * B * B +
-                                                          (size_t)srow * B + 4 * sg);
+    auto load_plane = [&](int p) -> Groups {
+        Groups v;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            v.g[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+            if (stg[u] && (unsigned)p < (unsigned)B)
+                v.g[u] = *reinterpret_cast<const PFH_GLOBAL f32x4*>(
+                    gsrc + (size_t)p * B * B + (size_t)srow[u] * B + 4 * sg[u]);
+        }
         return v;
     };
 
     const int pbeg = zb + sz - 1;
     const int pcount = ze - zb + 2;
-    f32x4 R = load_plane(pbeg);
-    f32x4 Rn = load_plane(pbeg + 1);
+    Groups R = load_plane(pbeg);
+    Groups Rn = load_plane(pbeg + 1);
     __syncthreads();
-    if (stg) stage_plane(lds, R);
+    stage_plane(lds, R);
     __syncthreads();
 
     float T[4] = {0.f, 0.f, 0.f, 0.f}, Q1p[4] = {0.f, 0.f, 0.f, 0.f};
@@ -809,7 +1079,7 @@ __global__ __launch_bounds__(1024) void k3_update(const pfh3d_step_args a, const
     for (int i = 0; i < pcount; ++i) {
         const int p = pbeg + i;
         const int cur = i & 1;
-        const f32x4 Rnn = (i + 2 < pcount) ? load_plane(p + 2) : f32x4{0.f, 0.f, 0.f, 0.f};
+        const Groups Rnn = load_plane(i + 2 < pcount ? p + 2 : -1);
         float A[4] = {0.f, 0.f, 0.f, 0.f}, Q1[4] = {0.f, 0.f, 0.f, 0.f},
               Q0[4] = {0.f, 0.f, 0.f, 0.f}, GX[4] = {0.f, 0.f, 0.f, 0.f},
               GY[4] = {0.f, 0.f, 0.f, 0.f};
@@ -884,7 +1154,7 @@ __global__ __launch_bounds__(1024) void k3_update(const pfh3d_step_args a, const
             gxm[j] = GX[j];
             gym[j] = GY[j];
         }
-        if (i + 1 < pcount && stg) stage_plane(lds + (cur ^ 1) * PLU, Rn);
+        if (i + 1 < pcount) stage_plane(lds + (cur ^ 1) * PLU, Rn);
         pfh::lds_barrier();   // the plane buffers are the only shared data here
         Rn = Rnn;
 #pragma unroll
@@ -1187,14 +1457,21 @@ int block_threads(int B) {
 // on a compute unit (one 13-wave workgroup otherwise): 208 against 212 us per
 // step at 256^3 / 128 cells.
 int update_parts(int B) { return B >= 32 ? 2 : 1; }
+// a lane per 16 B group of a part's rows; the halo rows' groups are staged in a
+// second turn (as lanes of their own they made nine waves of eight at B = 64,
+// and two such workgroups do not fit a compute unit's registers)
 int update_threads(int B) {
-    const int g = (B / update_parts(B) + 2) * (B / 4);   // rows + two halo rows
+    const int g = (B / update_parts(B)) * (B / 4);
     return ((g + 63) / 64) * 64;
 }
 size_t measure_lds(int B) { return 4u * (size_t)(B + 2) * (size_t)(B + 4) * sizeof(float); }
 size_t update_lds(int B) {
-    return 2u * (size_t)(B + 2 * pfh3::kMargin + 1) * (size_t)pfh3::update_row_pitch(B) *
-           sizeof(float);
+    // the general walk's two planes; the plain one's and 1 KiB per wave
+    const size_t gen = 2u * (size_t)(B + 2 * pfh3::kMargin + 1) *
+                       (size_t)pfh3::update_row_pitch(B);
+    const size_t plain = 2u * (size_t)(B / update_parts(B) + 2) * (size_t)(B + 8) +
+                         4u * (size_t)update_threads(B);
+    return (gen > plain ? gen : plain) * sizeof(float);
 }
 
 int check_geometry(const pfh3d_step_args* a) {
