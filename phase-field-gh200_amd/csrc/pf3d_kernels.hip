@@ -15,14 +15,15 @@
 // gfx950 mapping. A brick plane of B*B voxels is B*B/4 sixteen-byte x
 // groups; one lane owns one group (B = 48: 576 lanes = 9 waves), so every
 // global access of a plane is one coalesced 16 B load or store per lane.
-//   k3_measure  grid N*shards, shard = a contiguous z range. Planes roll
-//               through registers (z neighbours) and a two-buffer LDS ring
-//               (x/y neighbours). Per-lane fp64 sums in z-then-x order, a
-//               64-lane shuffle tree, waves in ascending order; the last
-//               shard of a cell to arrive adds the shard partials in
-//               ascending order and commits the cell (centroid shift,
-//               support check) and its motion. The same launch zeroes the
-//               next aggregate buffer and snapshots the accepted cell state.
+//   k3_measure  grid N*shards, shard = a contiguous z range. Each lane's own
+//               groups roll through registers and it reads its neighbours'
+//               itself, from cache, with no barrier in the plane loop.
+//               Per-lane fp64 sums in z-then-x order, a 64-lane tree, waves
+//               in ascending order; the last shard of a cell to arrive adds
+//               the shard partials in ascending order and commits the cell
+//               (centroid shift, support check) and its motion. The same
+//               launch zeroes the next aggregate buffer and snapshots the
+//               accepted cell state.
 //   k3_update   grid N*slabs*parts, slab = a contiguous range of
 //               destination planes, part = a contiguous range of their rows
 //               (two parts from B = 32). Source planes (the part's rows and
@@ -119,6 +120,33 @@ __device__ __forceinline__ bool fatal_present(const pfh3d_cell_state* c,
                                               const uint32_t* flags) {
     return (ld_relaxed(&c->flags) & kFatal) != 0u || global_fatal(flags);
 }
+
+// Raw buffer descriptors: a byte offset past the end reads zeros and stores
+// nothing.
+constexpr uint32_t kNone = 0x80000000u;          // past every descriptor's end
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc3(const void* p, uint32_t bytes) {
+    // (the address of a uniform pointer may still have been computed per lane)
+    const uint64_t v = reinterpret_cast<uint64_t>(p);
+    const uint64_t u =
+        (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(v >> 32)) << 32 |
+        (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)v);
+    return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(u), 0, (int)bytes,
+                                             0x00020000);
+}
+__device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ float uni(float v) {
+    return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(v)));
+}
+// LDS that only one wave uses: its operations complete in order; this keeps
+// the compiler's order too.
+__device__ __forceinline__ void wave_order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+__device__ __forceinline__ bool wave_any(bool v) {
+    return __builtin_amdgcn_ballot_w64(v) != 0ull;
+}
+typedef u32x4 u32x4_4 __attribute__((aligned(4)));
 
 // other_field, src/pf3d/device_common.cuh:182-191
 __device__ __forceinline__ float other_field(uint32_t agg, float phi,
@@ -288,22 +316,14 @@ __device__ __forceinline__ int wmax(int v) {
 
 __global__ __launch_bounds__(1024) void k3_measure(const pfh3d_step_args a,
                                                    const MeasureMode m) {
-    extern __shared__ __align__(16) float lds[];
     __shared__ double red[16][8];
     __shared__ int ired[16][7];
+    __shared__ f32x4 strip[16][128];
 
     const int B = a.B, S = a.shards, L = a.L, P = a.P;
     const int NT = (int)blockDim.x, tid = (int)threadIdx.x;
-    const int n = (int)blockIdx.x / S, sh = (int)blockIdx.x - n * S;
+    const int n = uni((int)blockIdx.x / S), sh = (int)blockIdx.x - n * S;
 
-    if (m.clear_out) {
-        const size_t total4 = (size_t)L * (size_t)L * (size_t)P / 4u;
-        const u32x4 z4 = {0u, 0u, 0u, 0u};
-        u32x4* dst = reinterpret_cast<u32x4*>(a.S_out);
-        for (size_t i = (size_t)blockIdx.x * NT + tid; i < total4;
-             i += (size_t)gridDim.x * NT)
-            __builtin_nontemporal_store(z4, dst + i);
-    }
     if (m.snapshot && sh == 0 && tid < 16) {
         const f32x4* s4 = reinterpret_cast<const f32x4*>(a.cells + n);
         f32x4* d4 = reinterpret_cast<f32x4*>(a.accepted + n);
@@ -311,9 +331,9 @@ __global__ __launch_bounds__(1024) void k3_measure(const pfh3d_step_args a,
     }
 
     pfh3d_cell_state* cs = a.cells + n;
-    const int ox = wrap_origin(cs->origin_x, L);
-    const int oy = wrap_origin(cs->origin_y, L);
-    const int oz = wrap_origin(cs->origin_z, L);
+    const int ox = uni(wrap_origin(cs->origin_x, L));
+    const int oy = uni(wrap_origin(cs->origin_y, L));
+    const int oz = uni(wrap_origin(cs->origin_z, L));
     int surface = m.surface_mode;
     if (surface == 2)
         surface = a.full_moment_every > 0 &&
@@ -324,168 +344,195 @@ __global__ __launch_bounds__(1024) void k3_measure(const pfh3d_step_args a,
     const bool act = tid < G;
     const int y = act ? tid / gpr : 0;
     const int x0 = act ? 4 * (tid - y * gpr) : 0;
-    const int PX = B + 4, PL = (B + 2) * PX;
-    const int own = (y + 1) * PX + 4 + x0;
 
-    // A ring of four planes in LDS, each with a zero border (x/y neighbours
-    // past the brick): the plane a lane measures, its two z neighbours, and
-    // the plane being filled. Lanes only ever write their own 16 B of a
-    // plane's interior, so the border stays zero.
-    for (int i = tid; i < 4 * PL; i += NT) lds[i] = 0.0f;
-    auto slot = [&](int p) -> float* { return lds + ((p - zb + 1) & 3) * PL; };
+    // The lane's own group rolls through registers as planes z - 1, z, z + 1.
+    // Its wave's 64 groups of plane z are a contiguous strip of the plane; the
+    // wave keeps them in LDS with the row before and the row after (the halo
+    // groups, one load by the first 2 * gpr lanes) and reads the rows y - 1,
+    // y + 1 and the words beside the group there. No wave waits for another:
+    // in a ring of planes that all waves share the barrier of every plane took
+    // most of the time, and neighbours read from cache cost more L2 traffic
+    // than the halo (380 us against 335 for two steps of 128 bricks of 56).
+    // A buffer descriptor over the cube gives the zeros around it. The halo and
+    // the S words are requested one plane ahead, the lane's own group, which
+    // comes from memory, three.
+    const uint32_t plane = 4u * (uint32_t)(B * B);
+    const __amdgpu_buffer_rsrc_t bin =
+        rsrc3(a.phi_in + (size_t)n * B * B * B, plane * (uint32_t)B);
+    const int lane = tid & 63, w0 = tid - lane;
+    const uint32_t o_own = act ? 16u * (uint32_t)tid : kNone;
+    // halo slot of this lane: 0 .. gpr - 1 before the strip, 64 + lane after it
+    // (slots past the row after it hold zeros; slot 127 is the zero beside the
+    // first and the last group of a row)
+    const int hg = lane < gpr ? w0 - gpr + lane : w0 + 64 - gpr + lane;
+    const uint32_t o_halo =
+        lane < 2 * gpr && hg >= 0 && hg < G ? 16u * (uint32_t)hg : kNone;
+    auto group = [&](uint32_t o, int z) -> f32x4 {
+        // (past the shard's last neighbour plane nothing is needed)
+        const uint32_t zo = z <= ze ? (uint32_t)z * plane : kNone / 2u;
+        const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(bin, (int)(o + zo), 0, 0);
+        return __builtin_bit_cast(f32x4, v);
+    };
+    f32x4* const mine4 = strip[tid >> 6];
+    f32x4* const w_own = mine4 + gpr + lane;
+    f32x4* const w_halo = mine4 + (lane < gpr ? lane : 64 + lane);
+    const f32x4* const r_ym = mine4 + (act ? lane : 127);
+    const f32x4* const r_yp = mine4 + 2 * gpr + lane;
+    const float* const r_xl = reinterpret_cast<const float*>(x0 > 0 ? w_own : mine4 + 128) - 1;
+    const float* const r_xr =
+        reinterpret_cast<const float*>(x0 < B - 4 ? w_own + 1 : mine4 + 127);
 
-    // Every vector load of the plane loop is unconditional and the loop
-    // stores nothing to global memory, so the compiler's wait before each
-    // use counts only the loads issued after it: a plane arrives one
-    // iteration after it is requested, the aggregate words one plane ahead
-    // of their use, and no iteration waits for its own requests. Planes
-    // outside the brick are read from a clamped address and replaced by
-    // zeros; inactive lanes read group 0.
-    const PFH_GLOBAL float* tile = gptr(a.phi_in) + (size_t)n * B * B * B;
-    const PFH_GLOBAL uint32_t* Sin = gptr(a.S_in);
-    const int lane_off = act ? 4 * tid : 0;
-    // (the raw request, and the zeros applied where the plane is used, so
-    // that nothing touches the loaded registers before then)
-    auto request_plane = [&](int p) -> f32x4 {
-        const int pc = p < 0 ? 0 : (p >= B ? B - 1 : p);
-        return *reinterpret_cast<const PFH_GLOBAL f32x4*>(tile + (size_t)pc * B * B +
-                                                          lane_off);
-    };
-    auto in_brick = [&](const f32x4& v, int p) -> f32x4 {
-        const bool in = act && (unsigned)p < (unsigned)B;
-        return f32x4{in ? v[0] : 0.f, in ? v[1] : 0.f, in ? v[2] : 0.f, in ? v[3] : 0.f};
-    };
-    auto load_plane = [&](int p) -> f32x4 { return in_brick(request_plane(p), p); };
-    const int wy = wrap_off(oy, y, L);
-    int wx[4];
+    // The next aggregate is cleared on the way: 16 B of each lane after each
+    // plane's requests, the rest after the walk.
+    const size_t s_words4 = (size_t)L * (size_t)L * (size_t)P / 4u;
+    const size_t s_lanes = (size_t)gridDim.x * (size_t)NT;
+    const bool clear_in =
+        m.clear_out && s_words4 < (size_t)(kNone / 16u) && s_lanes < (size_t)(kNone / 16u);
+    const __amdgpu_buffer_rsrc_t bclr =
+        rsrc3(a.S_out, clear_in ? (uint32_t)s_words4 * 16u : 0u);
+    const uint32_t clr_step = 16u * (uint32_t)s_lanes;
+    uint32_t o_clr = 16u * (blockIdx.x * (uint32_t)NT + (uint32_t)tid);
+    // S words of the lane's voxels: one 16 B load, or four where the brick
+    // wraps around the domain in x
+    const bool wraps = ox + B > L;
+    uint32_t o_s[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) wx[j] = wrap_off(ox, x0 + j, L);
-    // S words of this lane's 4 voxels in plane z, read only where that
-    // plane's phi is nonzero (the interaction reads S nowhere else, and most
-    // of a brick is empty); the other requests go to word 0, one cache line
-    // for the whole launch. The plane loop reads a word only where its
-    // voxel's phi is nonzero, the same mask.
-    auto load_s = [&](int z, const f32x4& ph, uint32_t (&sv)[4]) {
-        const size_t srow = s_index(L, P, 0, wy, wrap_off(oz, z < B ? z : B - 1, L));
-        const bool zin = act && z < ze;
+    for (int j = 0; j < 4; ++j)
+        o_s[j] = 4u * (uint32_t)(wrap_off(oy, y, L) * P + wrap_off(ox, x0 + j, L));
+    const size_t s_plane = (size_t)L * (size_t)P;
+    auto load_s = [&](int z) -> u32x4 {
+        const __amdgpu_buffer_rsrc_t bs =
+            rsrc3(a.S_in + (size_t)wrap_off(oz, z < ze ? z : ze - 1, L) * s_plane,
+                  4u * (uint32_t)s_plane);
+        if (!wraps) return __builtin_amdgcn_raw_buffer_load_b128(bs, (int)o_s[0], 0, 0);
+        u32x4 v;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const size_t idx = (zin && ph[j] != 0.0f) ? srow + (size_t)wx[j] : 0u;
-            sv[j] = Sin[idx];
-        }
+        for (int j = 0; j < 4; ++j)
+            v[j] = __builtin_amdgcn_raw_buffer_load_b32(bs, (int)o_s[j], 0, 0);
+        return v;
     };
 
-    {
-        const f32x4 Pm = load_plane(zb - 1);
-        const f32x4 P0 = load_plane(zb);
-        const f32x4 P1 = load_plane(zb + 1);
-        __syncthreads();                        // the ring's zeros are written
-        if (act) {
-            *reinterpret_cast<f32x4*>(slot(zb - 1) + own) = Pm;
-            *reinterpret_cast<f32x4*>(slot(zb) + own) = P0;
-            *reinterpret_cast<f32x4*>(slot(zb + 1) + own) = P1;
-        }
-    }
-    // Two planes in flight (z + 2 and z + 3 while plane z is measured) and
-    // the aggregate words of two planes (z and z + 1): each request has two
-    // iterations to arrive.
-    // (issued in the order the loop issues them: S0, R0, S1, R1)
-    uint32_t S0[4], S1[4];
-    f32x4 R0, R1;
-    int Rp0 = zb + 2, Rp1 = zb + 3;            // the planes' indices
-    {
-        const f32x4 P0 = *reinterpret_cast<const f32x4*>(slot(zb) + own);
-        const f32x4 P1 = *reinterpret_cast<const f32x4*>(slot(zb + 1) + own);
-        load_s(zb, P0, S0);
-        R0 = request_plane(Rp0);
-        load_s(zb + 1, P1, S1);
-        R1 = request_plane(Rp1);
-    }
-    __syncthreads();
-
+    const double xd0 = (double)x0, yd = (double)y;
     double aV = 0.0, aCx = 0.0, aCy = 0.0, aCz = 0.0, aS = 0.0, aIx = 0.0, aIy = 0.0,
            aIz = 0.0;
-    int lo0 = B, lo1 = B, lo2 = B, hi0 = -1, hi1 = -1, hi2 = -1;
-    uint32_t pmax = 0u, n_nonfin = 0u, n_neg = 0u;
+    float vmax = 0.0f;
+    uint32_t n_nonfin = 0u, n_neg = 0u;
+    // the support: lanes whose voxel j was above the bound (the lane's y and
+    // x0 + j), and the wave's first and last such plane
+    uint64_t sup[4] = {0ull, 0ull, 0ull, 0ull};
+    int lo2 = B, hi2 = -1;
 
-    // One plane: measure plane z with the aggregate words requested two
-    // planes earlier (set Sz), store the plane that arrived (z + 2, in Rz)
-    // into the ring, request its aggregate words into Sz and plane z + 4
-    // into Rz.
-    // This lane's own groups of planes z - 1 and z roll through registers
-    // (read from the ring once each, as plane z + 1)
-    f32x4 Am = *reinterpret_cast<const f32x4*>(slot(zb - 1) + own);
-    f32x4 A0 = *reinterpret_cast<const f32x4*>(slot(zb) + own);
-    auto plane_step = [&](int z, uint32_t (&Sz)[4], f32x4& Rz, int& Rpz) {
-        const uint32_t (&Sc)[4] = Sz;
-        const f32x4 Ap = *reinterpret_cast<const f32x4*>(slot(z + 1) + own);
-        if (act) {
-            const float* pl = slot(z);
-            const f32x4 ym = *reinterpret_cast<const f32x4*>(pl + own - PX);
-            const f32x4 yp = *reinterpret_cast<const f32x4*>(pl + own + PX);
-            const float xl = pl[own - 1], xr = pl[own + 4];
+    // Voxel j of plane z; every sum takes its terms in the reference's order.
+    // (An empty voxel adds zeros only: no test for it.)
+    auto voxel = [&](double xd, double zd, float c, float gx, float gy, float gz,
+                     uint32_t agg) {
+        // other_field (src/pf3d/device_common.cuh:182-191), its S_NEGATIVE
+        // event counted here and raised after the loop
+        const uint32_t mine = q_of(c);
+        const bool neg = agg < mine;
+        n_neg += neg ? 1u : 0u;
+        const float other = neg ? 0.0f : (float)(agg - mine) * pfh::kQInv;
+        const double sq = (double)c * (double)c;
+        aV += sq;
+        aCx += sq * xd;
+        aCy += sq * yd;
+        aCz += sq * zd;
+        aIx += (double)(c * gx * other);
+        aIy += (double)(c * gy * other);
+        aIz += (double)(c * gz * other);
+        vmax = fmaxf(vmax, fabsf(c));
+    };
+    f32x4 Am = group(o_own, zb - 1), A0 = group(o_own, zb), Ap = group(o_own, zb + 1);
+    f32x4 H = group(o_halo, zb);
+    u32x4 S0 = load_s(zb), S1;
+    f32x4 R0 = group(o_own, zb + 2), R1;
+    // plane z: S words in Sz, plane z + 1's requested into Sn; the lane's group
+    // of plane z + 2 in Rz, plane z + 3's requested into Rn
+    auto plane_step = [&](int z, const u32x4& Sz, u32x4& Sn, const f32x4& Rz, f32x4& Rn) {
+        *w_own = A0;
+        *w_halo = H;
+        wave_order();
+        const f32x4 Ym = *r_ym, Yp = *r_yp;
+        const float Xl = *r_xl, Xr = *r_xr;
+        wave_order();
+        H = group(o_halo, z + 1);
+        Sn = load_s(z + 1);
+        Rn = group(o_own, z + 3);
+        const u32x4 z4 = {0u, 0u, 0u, 0u};
+        __builtin_amdgcn_raw_buffer_store_b128(z4, bclr, (int)o_clr, 0, 2);
+        o_clr = min(o_clr + clr_step, kNone);
+        float gx[4], gy[4], gz[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const float xm = j == 0 ? Xl : A0[j == 0 ? 0 : j - 1];
+            const float xp = j == 3 ? Xr : A0[j == 3 ? 3 : j + 1];
+            gx[j] = 0.5f * (xp - xm);
+            gy[j] = 0.5f * (Yp[j] - Ym[j]);
+            gz[j] = 0.5f * (Ap[j] - Am[j]);
+        }
+        // A value that is not finite is counted and adds nothing (zeros); one
+        // test per wave. (A neighbour's shows in the sums as it always did.)
+        f32x4 c = A0;
+        const float all = (A0[0] + A0[1]) + (A0[2] + A0[3]);
+        if (wave_any(!(fabsf(all) < INFINITY))) {
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                const float c = A0[j];
-                if (!isfinite(c)) {
-                    ++n_nonfin;
-                    continue;
-                }
-                const float xm = j == 0 ? xl : A0[j == 0 ? 0 : j - 1];
-                const float xp = j == 3 ? xr : A0[j == 3 ? 3 : j + 1];
-                const float gx = 0.5f * (xp - xm);
-                const float gy = 0.5f * (yp[j] - ym[j]);
-                const float gz = 0.5f * (Ap[j] - Am[j]);
-                if (c == 0.0f && gx == 0.0f && gy == 0.0f && gz == 0.0f) continue;
-                float other = 0.0f;
-                const int x = x0 + j;
-                if (c != 0.0f) {
-                    // other_field (src/pf3d/device_common.cuh:182-191), its
-                    // S_NEGATIVE event counted here and raised after the loop
-                    const uint32_t agg = Sc[j], mine = q_of(c);
-                    if (agg >= mine) other = (float)(agg - mine) * pfh::kQInv;
-                    else ++n_neg;
-                }
-                const double sq = (double)c * (double)c;
-                aV += sq;
-                aCx += sq * (double)x;
-                aCy += sq * (double)y;
-                aCz += sq * (double)z;
-                if (surface)
-                    aS += sqrt((double)gx * (double)gx + (double)gy * (double)gy +
-                               (double)gz * (double)gz);
-                aIx += (double)(c * gx * other);
-                aIy += (double)(c * gy * other);
-                aIz += (double)(c * gz * other);
-                const float ac = fabsf(c);
-                pmax = max(pmax, __float_as_uint(ac));
-                if (ac > kEps) {
-                    lo0 = min(lo0, x); hi0 = max(hi0, x);
-                    lo1 = min(lo1, y); hi1 = max(hi1, y);
-                    lo2 = min(lo2, z); hi2 = max(hi2, z);
-                }
+                const bool bad = !isfinite(c[j]);
+                n_nonfin += bad ? 1u : 0u;
+                c[j] = bad ? 0.0f : c[j];
+                gx[j] = bad ? 0.0f : gx[j];
+                gy[j] = bad ? 0.0f : gy[j];
+                gz[j] = bad ? 0.0f : gz[j];
             }
         }
-        // plane z + 2 replaces plane z - 2, last read before the previous
-        // barrier; a plane past the shard's last neighbour (ze) is never
-        // read, and its request is the cached plane ze again
+        uint64_t hit = 0ull;
+        const double zd = (double)z;
+        double xd = xd0;      // x0 + j, not four registers pairs over the walk
+        asm volatile("" : "+v"(xd));
+#pragma unroll
+        for (int j = 0; j < 4; ++j, xd += 1.0) {
+            voxel(xd, zd, c[j], gx[j], gy[j], gz[j], Sz[j]);
+            const uint64_t in = __builtin_amdgcn_ballot_w64(fabsf(c[j]) > kEps);
+            sup[j] |= in;
+            hit |= in;
+        }
+        if (surface) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                aS += sqrt((double)gx[j] * (double)gx[j] + (double)gy[j] * (double)gy[j] +
+                           (double)gz[j] * (double)gz[j]);
+        }
+        if (hit) {
+            lo2 = min(lo2, z);
+            hi2 = z;
+        }
         Am = A0;
         A0 = Ap;
-        const f32x4 An = in_brick(Rz, Rpz);
-        if (act) *reinterpret_cast<f32x4*>(slot(z + 2) + own) = An;
-        load_s(z + 2, An, Sz);
-        Rpz = z + 4 <= ze ? z + 4 : ze;
-        Rz = request_plane(Rpz);
-        pfh::lds_barrier();   // the ring is the only data shared here
+        Ap = Rz;
     };
-    // pairs of planes, then an odd last plane: both steps of a pair run
-    // unconditionally, so the request counts the waits see are fixed
     int z = zb;
     for (; z + 1 < ze; z += 2) {
-        plane_step(z, S0, R0, Rp0);
-        plane_step(z + 1, S1, R1, Rp1);
+        plane_step(z, S0, S1, R0, R1);
+        plane_step(z + 1, S1, S0, R1, R0);
     }
-    if (z < ze) plane_step(z, S0, R0, Rp0);
+    if (z < ze) plane_step(z, S0, S1, R0, R1);
+    if (m.clear_out) {
+        const u32x4 z4 = {0u, 0u, 0u, 0u};
+        u32x4* dst = reinterpret_cast<u32x4*>(a.S_out);
+        const size_t done = clear_in ? (size_t)(ze - zb) * s_lanes : 0u;
+        for (size_t i = done + (size_t)blockIdx.x * NT + tid; i < s_words4; i += s_lanes)
+            __builtin_nontemporal_store(z4, dst + i);
+    }
+    int lo0 = B, lo1 = B, hi0 = -1, hi1 = -1;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        if ((sup[j] >> (tid & 63)) & 1ull) {
+            lo0 = min(lo0, x0 + j);
+            hi0 = max(hi0, x0 + j);
+            lo1 = hi1 = y;
+        }
+    }
+    uint32_t pmax = __float_as_uint(vmax);
     if (n_nonfin) {
         atomicOr(&cs->flags, 1u << PFH3D_FLAG_NONFINITE);
         atomicAdd(&a.flags[PFH3D_FLAG_NONFINITE], n_nonfin);
@@ -501,7 +548,7 @@ __global__ __launch_bounds__(1024) void k3_measure(const pfh3d_step_args a,
     lo0 = wmin(lo0); lo1 = wmin(lo1); lo2 = wmin(lo2);
     hi0 = wmax(hi0); hi1 = wmax(hi1); hi2 = wmax(hi2);
     pmax = (uint32_t)wmax((int)pmax);   // |phi| bit patterns are non-negative ints
-    const int wave = tid >> 6, lane = tid & 63;
+    const int wave = tid >> 6;
     if (lane == 0) {
         red[wave][0] = aV; red[wave][1] = aCx; red[wave][2] = aCy; red[wave][3] = aCz;
         red[wave][4] = aS; red[wave][5] = aIx; red[wave][6] = aIy; red[wave][7] = aIz;
@@ -661,18 +708,6 @@ __device__ __noinline__ void clip_voxel(const ClipArgs a, pfh3d_cell_state* cs,
 //     four words touch four times as many lines per instruction (1.32 M atomic
 //     requests per 256^3 / 128-cell step before).
 // ---------------------------------------------------------------------------
-constexpr uint32_t kNone = 0x80000000u;          // past every descriptor's end
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc3(const void* p, uint32_t bytes) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, 0x00020000);
-}
-__device__ __forceinline__ float uni(float v) {
-    return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(v)));
-}
-__device__ __forceinline__ bool wave_any(bool v) {
-    return __builtin_amdgcn_ballot_w64(v) != 0ull;
-}
-typedef u32x4 u32x4_4 __attribute__((aligned(4)));
-
 template <bool kWrapX>
 __device__ __forceinline__ void update_plain(const pfh3d_step_args& a, pfh3d_cell_state* cs,
                                              const CellCoef& kc, int n, int zb, int ze, int yb,
@@ -1464,7 +1499,6 @@ int update_threads(int B) {
     const int g = (B / update_parts(B)) * (B / 4);
     return ((g + 63) / 64) * 64;
 }
-size_t measure_lds(int B) { return 4u * (size_t)(B + 2) * (size_t)(B + 4) * sizeof(float); }
 size_t update_lds(int B) {
     // the general walk's two planes; the plain one's and 1 KiB per wave
     const size_t gen = 2u * (size_t)(B + 2 * pfh3::kMargin + 1) *
@@ -1493,18 +1527,8 @@ int launch_measure(const pfh3d_step_args* a, const pfh3::MeasureMode& m, void* s
     if (a->max_shift < 0 || a->max_shift > PFH3D_MAX_SHIFT) return invalid("max_shift");
     if (m.clear_out && !a->S_out) return invalid("S_out");
     if (m.snapshot && !a->accepted) return invalid("accepted");
-    // four ring planes: 55.7 KB at B = 56, 71.8 KB at B = 64 (above the
-    // default 64 KB of dynamic LDS, so the limit is raised for the kernel)
-    const size_t lds = measure_lds(a->B);
-    if (lds > 65536u) {
-        st = hip_status(hipFuncSetAttribute(reinterpret_cast<const void*>(&pfh3::k3_measure),
-                                            hipFuncAttributeMaxDynamicSharedMemorySize,
-                                            (int)lds),
-                        "hipFuncSetAttribute(k3_measure)");
-        if (st != PFH_OK) return st;
-    }
     hipLaunchKernelGGL(pfh3::k3_measure, dim3((unsigned)(a->N * a->shards)),
-                       dim3((unsigned)block_threads(a->B)), lds, as_stream(stream), *a, m);
+                       dim3((unsigned)block_threads(a->B)), 0, as_stream(stream), *a, m);
     return launch_status("k3_measure");
 }
 

@@ -243,3 +243,63 @@ def test_rejected_step_matches_oracle(sim3, o3):
     assert np.array_equal(sim.S_now(), S)
     assert sim.cells().tobytes() == cells.tobytes()
     assert np.array_equal(sim.flag_counts() != 0, orc.flags != 0)
+
+
+@pytest.mark.parametrize("B,radius,lam,L,shards,slabs,moved", [
+    (16, 1.5, 1.0, 33, 16, 16, 0),   # one plane a shard and slab, odd domain
+    (16, 1.5, 1.0, 33, 3, 1, 2),
+    (24, 3.0, 1.5, 37, 1, 5, 1),     # 144 lanes: a partly filled wave
+    (32, 4.0, 2.0, 41, 5, 3, 3),
+    (40, 8.0, 3.5, 47, 2, 0, -2),
+    (64, 12.0, 3.5, 77, 7, 4, 0),    # the largest brick: 1024 lanes
+    (64, 12.0, 3.5, 77, 2, 2, -4),
+])
+def test_every_walk_agrees_with_the_oracle(sim3, o3, B, radius, lam, L, shards, slabs, moved):
+    """Bricks inside the domain, across its x face at an odd offset and across
+    its corner, without and with a recentring shift: the walks that these
+    select give the oracle's bits, also at signed and exact zeros, at
+    denormals and after the shift, and refuse a field beyond 2 as it does."""
+    say(f"walks B={B} L={L} shards={shards} slabs={slabs} moved={moved}")
+    p = params3d.SimParams3D(Nx=L, num_cells=4, target_radius=radius, lambda_=lam, seed=3,
+                             brick_edge_override=B, full_moment_every=2)
+    h = np.float32(L / 2)
+    wl = params3d.Workload3D("walks", p, np.array([h, 1, L - 2, h + 3], np.float32),
+                             np.array([h, h, 2, h - 2], np.float32),
+                             np.array([h, h + 1, L - 1, 0], np.float32))
+    sim, orc = _pair(sim3, o3, wl, shards, slabs)
+    assert sim.B == B
+    phi = sim.phi_now().copy().reshape(sim.N, B, B, B)
+    c = B // 2
+    phi[:, c, c, c - 1] = 1.9
+    phi[1, c + 1, c, c] = -1.25
+    phi[2, c - 1, c - 2:c + 2, c - 2:c + 2] = 0.0
+    phi[3, c, c + 1, c - 1:c + 2] = -0.0
+    phi[0, c, c, c + 1] = 1e-40
+    if moved:
+        phi[0] = np.roll(phi[0], (moved, 0, 0), axis=(0, 1, 2))
+        phi[1] = np.roll(phi[1], (0, -moved, moved), axis=(0, 1, 2))
+        phi[2] = np.roll(phi[2], (0, 0, moved), axis=(0, 1, 2))
+    # the aggregate of these fields and the measurement that plans the shifts
+    orc.load_state(phi.reshape(sim.N, -1), np.zeros_like(sim.S_now()), sim.cells(), (0, 0))
+    orc.lib.pfo3d_scatter(orc.phi[0].ctypes.data, orc.cells.ctypes.data, orc.S[0].ctypes.data,
+                          orc.flags.ctypes.data, orc.N, orc.B, orc.L, orc.P)
+    S = orc.S[0].copy()
+    import ctypes as C
+    orc.lib.pfo3d_measure(C.byref(orc._args(0)), 0, 0, 1, 1, THREADS)
+    orc.flags[:] = 0
+    sim.load_state(phi.reshape(sim.N, -1), S, orc.cells.copy(), (0, 0))
+    for k in range(2):
+        sim.step(1)
+        orc.step(1)
+        sim.sync()
+        assert_state_equal(sim, orc, f"walks step {k}")
+        assert not sim.fatal()
+    phi, S, cells = sim.phi_now().copy(), sim.S_now().copy(), sim.cells().copy()
+    phi.reshape(sim.N, B, B, B)[:, c, c, c] = 2.5
+    sim.load_state(phi, S, cells, (2, 2))
+    orc.load_state(phi, S, cells, (2, 2))
+    sim.step(1)
+    orc.step(1)
+    sim.sync()
+    assert_state_equal(sim, orc, "walks, refused step")
+    assert sim.fatal()
