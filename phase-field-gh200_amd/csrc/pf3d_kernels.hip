@@ -250,11 +250,14 @@ struct MotionArgs {
 };
 
 __device__ __noinline__ void motion_cell(pfh3d_cell_state* s, const MotionArgs a,
-                                         int apply_tumble) {
-    if (fatal_present(s, a.flags)) return;
+                                         int apply_tumble, double Ix, double Iy,
+                                         double Iz) {
+    // (requested before the flags are waited for)
     const uint64_t step = a.counters ? a.counters[0] : 0u;
     const bool active = step >= a.aging_steps;
     double pol[3] = {s->polarity_x, s->polarity_y, s->polarity_z};
+    const float v_A = s->v_A;
+    if (fatal_present(s, a.flags)) return;
     bool tumbled = false;
     if (apply_tumble && active) {
         const uint64_t st = step - a.aging_steps;
@@ -272,11 +275,11 @@ __device__ __noinline__ void motion_cell(pfh3d_cell_state* s, const MotionArgs a
         }
     }
     const float px = (float)pol[0], py = (float)pol[1], pz = (float)pol[2];
-    const float speed = active ? s->v_A : 0.0f;
+    const float speed = active ? v_A : 0.0f;
     const float mot = a.motility_coeff;
-    const float vx = speed * px + mot * (float)s->Ix;
-    const float vy = speed * py + mot * (float)s->Iy;
-    const float vz = speed * pz + mot * (float)s->Iz;
+    const float vx = speed * px + mot * (float)Ix;
+    const float vy = speed * py + mot * (float)Iy;
+    const float vz = speed * pz + mot * (float)Iz;
     if (!isfinite(px) || !isfinite(py) || !isfinite(pz) || !isfinite(vx) ||
         !isfinite(vy) || !isfinite(vz)) {
         raise3(s, a.flags, PFH3D_FLAG_NONFINITE);
@@ -297,22 +300,6 @@ struct MeasureMode {
     int clear_out;      // zero S_out (the next aggregate) in this launch
     int snapshot;       // copy cells -> accepted before committing
 };
-
-__device__ __forceinline__ double wsum(double v) {
-#pragma unroll
-    for (int d = 32; d > 0; d >>= 1) v += __shfl_down(v, d, 64);
-    return v;
-}
-__device__ __forceinline__ int wmin(int v) {
-#pragma unroll
-    for (int d = 32; d > 0; d >>= 1) v = min(v, __shfl_down(v, d, 64));
-    return v;
-}
-__device__ __forceinline__ int wmax(int v) {
-#pragma unroll
-    for (int d = 32; d > 0; d >>= 1) v = max(v, __shfl_down(v, d, 64));
-    return v;
-}
 
 __global__ __launch_bounds__(1024) void k3_measure(const pfh3d_step_args a,
                                                    const MeasureMode m) {
@@ -542,70 +529,90 @@ __global__ __launch_bounds__(1024) void k3_measure(const pfh3d_step_args a,
         atomicAdd(&a.flags[PFH3D_FLAG_S_NEGATIVE], n_neg);
     }
 
-    // 64-lane trees, then waves in ascending order
-    aV = wsum(aV); aCx = wsum(aCx); aCy = wsum(aCy); aCz = wsum(aCz);
-    aS = wsum(aS); aIx = wsum(aIx); aIy = wsum(aIy); aIz = wsum(aIz);
-    lo0 = wmin(lo0); lo1 = wmin(lo1); lo2 = wmin(lo2);
-    hi0 = wmax(hi0); hi1 = wmax(hi1); hi2 = wmax(hi2);
-    pmax = (uint32_t)wmax((int)pmax);   // |phi| bit patterns are non-negative ints
-    const int wave = tid >> 6;
-    if (lane == 0) {
-        red[wave][0] = aV; red[wave][1] = aCx; red[wave][2] = aCy; red[wave][3] = aCz;
-        red[wave][4] = aS; red[wave][5] = aIx; red[wave][6] = aIy; red[wave][7] = aIz;
-        ired[wave][0] = lo0; ired[wave][1] = hi0; ired[wave][2] = lo1;
-        ired[wave][3] = hi1; ired[wave][4] = lo2; ired[wave][5] = hi2;
-        ired[wave][6] = (int)pmax;
-    }
-    __syncthreads();
-    if (tid != 0) return;
-
-    Acc t = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-    Box b = {{B, B, B}, {-1, -1, -1}, 0u};
-    for (int w = 0; w < NT / 64; ++w) {
-        t.V += red[w][0]; t.Cx += red[w][1]; t.Cy += red[w][2]; t.Cz += red[w][3];
-        t.surf += red[w][4]; t.Ix += red[w][5]; t.Iy += red[w][6]; t.Iz += red[w][7];
-        b.lo[0] = min(b.lo[0], ired[w][0]); b.hi[0] = max(b.hi[0], ired[w][1]);
-        b.lo[1] = min(b.lo[1], ired[w][2]); b.hi[1] = max(b.hi[1], ired[w][3]);
-        b.lo[2] = min(b.lo[2], ired[w][4]); b.hi[2] = max(b.hi[2], ired[w][5]);
-        b.pmax = max(b.pmax, (uint32_t)ired[w][6]);
-    }
-
-    Acc tot = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-    Box tb = {{B, B, B}, {-1, -1, -1}, 0u};
-    if (S > 1) {
-        pfh3d_moment_partial* pp = a.partials + (size_t)n * S;
-        pfh3d_moment_partial mine;
-        mine.V = t.V; mine.Cx = t.Cx; mine.Cy = t.Cy; mine.Cz = t.Cz;
-        mine.surface = t.surf; mine.Ix = t.Ix; mine.Iy = t.Iy; mine.Iz = t.Iz;
-        mine.lo_x = b.lo[0]; mine.hi_x = b.hi[0]; mine.lo_y = b.lo[1];
-        mine.hi_y = b.hi[1]; mine.lo_z = b.lo[2]; mine.hi_z = b.hi[2];
-        mine.phi_max_bits = b.pmax; mine.padding = 0u;
-        pp[sh] = mine;
-        __threadfence();
-        const uint32_t prev = atomicAdd(a.arrivals + n, 1u);
-        if (prev != (uint32_t)(S - 1)) return;
-        __threadfence();
-        for (int k = 0; k < S; ++k) {
-            const volatile pfh3d_moment_partial* q = pp + k;
-            tot.V += q->V; tot.Cx += q->Cx; tot.Cy += q->Cy; tot.Cz += q->Cz;
-            tot.surf += q->surface; tot.Ix += q->Ix; tot.Iy += q->Iy; tot.Iz += q->Iz;
-            tb.lo[0] = min(tb.lo[0], (int)q->lo_x); tb.hi[0] = max(tb.hi[0], (int)q->hi_x);
-            tb.lo[1] = min(tb.lo[1], (int)q->lo_y); tb.hi[1] = max(tb.hi[1], (int)q->hi_y);
-            tb.lo[2] = min(tb.lo[2], (int)q->lo_z); tb.hi[2] = max(tb.hi[2], (int)q->hi_z);
-            tb.pmax = max(tb.pmax, (uint32_t)q->phi_max_bits);
+    // 64-lane trees (lane 0 ends with the first value, lane 32 with the second,
+    // 16 and 48 with the third and fourth), then waves in ascending order: lane
+    // i of the first wave adds value i.
+    {
+        const double s0 = pfh::wave_sum4(aV, aCx, aCy, aCz);
+        const double s1 = pfh::wave_sum4(aS, aIx, aIy, aIz);
+        const int mn = pfh::wave_tree4(lo0, lo1, lo2, lo2,
+                                       [](int x, int y_) { return min(x, y_); });
+        // |phi| bit patterns are non-negative ints
+        const int mx = pfh::wave_tree4(hi0, hi1, hi2, (int)pmax,
+                                       [](int x, int y_) { return max(x, y_); });
+        const int wave = tid >> 6, v = ((lane >> 5) & 1) | ((lane >> 3) & 2);
+        if ((lane & 15) == 0) {
+            red[wave][v] = s0;
+            red[wave][4 + v] = s1;
+            if (v < 3) ired[wave][2 * v] = mn;
+            ired[wave][v < 3 ? 2 * v + 1 : 6] = mx;
         }
-        atomicExch(a.arrivals + n, 0u);
-    } else {
-        tot.V += t.V; tot.Cx += t.Cx; tot.Cy += t.Cy; tot.Cz += t.Cz;
-        tot.surf += t.surf; tot.Ix += t.Ix; tot.Iy += t.Iy; tot.Iz += t.Iz;
-        tb = b;
     }
+    // the wave's flag counts have arrived before the barrier lets the cell's
+    // last shard read them
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (tid >= 64) return;
+
+    // lanes 0..7: V, Cx, Cy, Cz, surface, Ix, Iy, Iz; lanes 8..14: the box and
+    // the largest |phi|, in the record's order
+    const int vi = lane >= 8 && lane < 15 ? lane - 8 : 6, vd = lane & 7;
+    const bool low = vi < 6 && (vi & 1) == 0;
+    const int v0 = low ? B : vi < 6 ? -1 : 0;
+    double sd = 0.0;
+    int si = v0;
+    for (int w = 0; w < NT / 64; ++w) {
+        sd += red[w][vd];
+        si = low ? min(si, ired[w][vi]) : max(si, ired[w][vi]);
+    }
+    if (S > 1) {
+        // A record travels by stores and loads at the device's scope, complete
+        // before the arrival: no write-back of the whole L2, which a fence of
+        // that scope would be.
+        pfh3d_moment_partial* pp = a.partials + (size_t)n * S;
+        if (lane < 8)
+            __hip_atomic_store(reinterpret_cast<unsigned long long*>(pp + sh) + lane,
+                               (unsigned long long)__double_as_longlong(sd), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+        else if (lane < 16)
+            __hip_atomic_store(reinterpret_cast<uint32_t*>(pp + sh) + 8 + lane,
+                               lane < 15 ? (uint32_t)si : 0u, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        uint32_t prev = 0u;
+        if (lane == 0)
+            prev = __hip_atomic_fetch_add(a.arrivals + n, 1u, __ATOMIC_RELAXED,
+                                          __HIP_MEMORY_SCOPE_AGENT);
+        if (uni((int)prev) != S - 1) return;
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        sd = 0.0;
+        si = v0;
+        for (int k = 0; k < S; ++k) {
+            sd += __longlong_as_double((long long)__hip_atomic_load(
+                reinterpret_cast<const unsigned long long*>(pp + k) + vd, __ATOMIC_RELAXED,
+                __HIP_MEMORY_SCOPE_AGENT));
+            const int x = (int)__hip_atomic_load(
+                reinterpret_cast<const uint32_t*>(pp + k) + 16 + vi, __ATOMIC_RELAXED,
+                __HIP_MEMORY_SCOPE_AGENT);
+            si = low ? min(si, x) : max(si, x);
+        }
+        if (lane == 0)
+            __hip_atomic_store(a.arrivals + n, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    auto at = [&](int l) {
+        return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(sd), l),
+                                __builtin_amdgcn_readlane(__double2loint(sd), l));
+    };
+    auto ati = [&](int l) { return (int)__builtin_amdgcn_readlane(si, 8 + l); };
+    const Acc tot = {at(0), at(1), at(2), at(3), at(4), at(5), at(6), at(7)};
+    const Box tb = {{ati(0), ati(2), ati(4)}, {ati(1), ati(3), ati(5)}, (uint32_t)ati(6)};
+    if (lane != 0) return;
     const CommitArgs ca{a.flags, B, a.max_shift, a.support_margin};
     commit_cell(cs, ca, tot, tb, surface);
     if (m.apply_motion) {
         const MotionArgs ma{a.flags, a.counters, a.aging_steps, a.polarity_stream,
                             a.p_tumble, a.motility_coeff};
-        motion_cell(cs, ma, m.apply_tumble);
+        motion_cell(cs, ma, m.apply_tumble, tot.Ix, tot.Iy, tot.Iz);
     }
 }
 
