@@ -394,6 +394,49 @@ __device__ WindowMoments window_moments(int cls, F phi_at) {
     return reduce_moments(p, wx, wy);
 }
 
+// window_moments of a stored field (t: its window's first pixel). A thread's
+// pixels are requested kAhead at a time and then visited in their order: one
+// after the other, each waited for, they took 50 us for 1024 windows of
+// 144 x 144, this way 37 us (85 MB).
+__device__ __forceinline__ WindowMoments stored_moments(int cls, const float* t) {
+    constexpr int kAhead = 8;
+    const Shape sc = shape_of(cls);
+    const int wx = sc.wx, wy = sc.wy;
+    const int tid = (int)threadIdx.x;
+    MomentPart p = {0.0, 0.0, 0.0, wx, -1, wy, -1, 0};
+    float v[kAhead];
+    if (cls <= kClassStagedMax) {
+        const int nb = kPixThreads / wx, rb = (wy + nb - 1) / nb;
+        const int pix = tid - kControlLanes;
+        const int x = pix % wx, band = pix / wx;
+        if (pix >= 0 && band < nb) {
+            const int end = min(band * rb + rb, wy);
+            for (int y = band * rb; y < end; y += kAhead) {
+#pragma unroll
+                for (int k = 0; k < kAhead; ++k)
+                    v[k] = y + k < end ? t[(size_t)(y + k) * kTilePitch + x] : 0.0f;
+#pragma unroll
+                for (int k = 0; k < kAhead; ++k)
+                    if (y + k < end) moment_visit(p, v[k], x, y + k);
+            }
+        }
+    } else {
+        for (int q = tid; q < wx * wy; q += kAhead * kNT) {
+#pragma unroll
+            for (int k = 0; k < kAhead; ++k) {
+                const int i = q + k * kNT;
+                v[k] = i < wx * wy ? t[(size_t)(i / wx) * kTilePitch + i % wx] : 0.0f;
+            }
+#pragma unroll
+            for (int k = 0; k < kAhead; ++k) {
+                const int i = q + k * kNT;
+                if (i < wx * wy) moment_visit(p, v[k], i % wx, i / wx);
+            }
+        }
+    }
+    return reduce_moments(p, wx, wy);
+}
+
 // Moments into the cell state; the interaction integral restarts at zero.
 __device__ __forceinline__ void store_moments(pfh_cell_state* cs, const WindowMoments& m) {
     cs->V = m.V; cs->Cx = m.Cx; cs->Cy = m.Cy;
