@@ -222,7 +222,8 @@ int pfh2d_configure_step(void);
  * LDS is static (sized for 16384 cells), so this only validates the size. */
 int pfh2d_configure_morton(int smem_bytes);
 /* Replaces k_step_grid(device) (include/kernels.cuh:221): the persistent
- * grid, one 1024-thread workgroup per compute unit. Returns the grid size,
+ * grid, the number of compute units (a step runs one 16-wave workgroup on each,
+ * or two of 8 waves where it has more cells than that). Returns the grid size,
  * or a negative status. */
 int pfh2d_step_grid(int device);
 

@@ -16,9 +16,9 @@
 // groups; one lane owns one group (B = 48: 576 lanes = 9 waves), so every
 // global access of a plane is one coalesced 16 B load or store per lane.
 //   k3_measure  grid N*shards, shard = a contiguous z range. Each lane's own
-//               groups roll through registers and it reads its neighbours'
-//               itself, from cache, with no barrier in the plane loop.
-//               Per-lane fp64 sums in z-then-x order, a 64-lane tree, waves
+//               groups roll through registers; a wave stages its strip of the
+//               plane and the rows beside it in LDS for itself, with no
+//               barrier in the plane loop. Per-lane fp64 sums in z-then-x order, a 64-lane tree, waves
 //               in ascending order; the last shard of a cell to arrive adds
 //               the shard partials in ascending order and commits the cell
 //               (centroid shift, support check) and its motion. The same
@@ -27,9 +27,11 @@
 //   k3_update   grid N*slabs*parts, slab = a contiguous range of
 //               destination planes, part = a contiguous range of their rows
 //               (two parts from B = 32). Source planes (the part's rows and
-//               one halo row on each side) stream through a two-buffer LDS ring
-//               with a zero margin of five, so the recentring shift (|s| <= 4)
-//               reads zeros outside the brick without branches. Each plane
+//               one halo row on each side) stream through a two-buffer LDS
+//               ring: laid out as in memory for a cell without a recentring
+//               shift (update_plain), and with a zero margin of five where
+//               there is one, so that the shift (|s| <= 4) reads zeros outside
+//               the brick without branches. Each plane
 //               is reduced once to per-voxel plane sums (centre/edge/corner
 //               weights of the 27-point stencil) held in registers, and a
 //               destination plane is finished when its upper neighbour
@@ -337,12 +339,16 @@ __global__ __launch_bounds__(1024) void k3_measure(const pfh3d_step_args a,
     // wave keeps them in LDS with the row before and the row after (the halo
     // groups, one load by the first 2 * gpr lanes) and reads the rows y - 1,
     // y + 1 and the words beside the group there. No wave waits for another:
-    // in a ring of planes that all waves share the barrier of every plane took
-    // most of the time, and neighbours read from cache cost more L2 traffic
-    // than the halo (380 us against 335 for two steps of 128 bricks of 56).
-    // A buffer descriptor over the cube gives the zeros around it. The halo and
-    // the S words are requested one plane ahead, the lane's own group, which
-    // comes from memory, three.
+    // with a ring of planes that all waves share, the barrier of every plane
+    // left the arithmetic idle (128 bricks of 56, two shards: 90 -> 72 us a
+    // launch, and 64 with the reduction below; neighbours read from cache
+    // instead cost more L2 traffic than the halo, 118 us). A buffer descriptor
+    // over the cube gives the zeros around it. The halo and the S words are
+    // requested one plane ahead, the lane's own group, which comes from
+    // memory, three. Bound by arithmetic and latency together: about 300
+    // instructions a lane and plane, a third of them fp64, are 37 us of the
+    // 64, and field, S words and clear, 224 MB, are 47 us at the rate of a
+    // copy.
     const uint32_t plane = 4u * (uint32_t)(B * B);
     const __amdgpu_buffer_rsrc_t bin =
         rsrc3(a.phi_in + (size_t)n * B * B * B, plane * (uint32_t)B);
@@ -714,6 +720,9 @@ __device__ __noinline__ void clip_voxel(const ClipArgs a, pfh3d_cell_state* cs,
 //     each cover 64 consecutive words of the wave's 256 voxels: a lane's own
 //     four words touch four times as many lines per instruction (1.32 M atomic
 //     requests per 256^3 / 128-cell step before).
+// 128 bricks of 56: 96 -> 69 us a launch (380 MB of field, S words and
+// scatter, 80 us at the rate of a copy: part of S stays in cache); 224 bricks
+// of 64: 300 -> 169 us (780 MB, 164 us).
 // ---------------------------------------------------------------------------
 template <bool kWrapX>
 __device__ __forceinline__ void update_plain(const pfh3d_step_args& a, pfh3d_cell_state* cs,

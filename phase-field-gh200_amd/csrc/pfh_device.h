@@ -30,7 +30,7 @@ constexpr int kNT = 1024;
 constexpr int kWave = 64;
 constexpr int kWaves = kNT / kWave;
 // Threads that may own pixels in the LDS path (column bands).
-constexpr int kControlLanes = 16;   // lanes 0-15 of wave 0: next-cell fetch
+constexpr int kControlLanes = 16;   // the first logical threads own no pixels
 constexpr int kPixThreads = kNT - kControlLanes;
 
 // ---- fixed tile and shape classes (include/params.cuh:121-147) ----

@@ -326,17 +326,23 @@ __global__ void k_sur_round_bf16(const float* x, uint32_t* y, int npairs) {
 // ---------------------------------------------------------------------------
 // dphi = b4 + sum_{tap, ci} W4[tap][ci] h3[p + off(tap)][ci]; out = phic + dphi.
 // Persistent over (crop, 4-row block) items like k_sur_conv: the 6 x 98
-// halo tile of h3 is staged in LDS. Four lanes share a pixel, eight channels
-// each, whose 72 weights stay in registers (a lane per pixel read all 288
-// from LDS for every pixel: 60 -> 37 us for 128 crops, the next tile in flight); fp32 sums, the four
-// lanes' partial sums added pairwise.
-__global__ __launch_bounds__(256) void k_sur_out(const bf16_t* H, const float* W4, float b4,
+// halo tile of h3 is staged in LDS. Four lanes, eight channels each, whose 72
+// weights stay in registers, walk six pixels of a row: every column of three
+// values is read and unpacked once and added to the up to three pixels that it
+// meets (one pixel at a time, 60 us for 128 crops with the weights in LDS, 37
+// with them in registers: each value was read and unpacked nine times; now
+// 25); fp32 sums, the four lanes' partial sums added pairwise. The pixel
+// pitch of 96 B puts four neighbouring walks on different banks.
+__global__ __launch_bounds__(256, 2) void k_sur_out(const bf16_t* H, const float* W4, float b4,
                                                  const float* phic, float* dphi, float* out,
                                                  int ncrops) {
-    constexpr int PIXP = kCH + 8;
+    constexpr int PIXP = kCH + 16, kRun = 6, kRuns = kCrop / kRun;
+    static_assert(kRowsPerItem * kRuns * 4 == 256, "a walk per four lanes");
     __shared__ __align__(16) bf16_t hl[(kRowsPerItem + 2) * kHaloCols * PIXP];
     const int tid = (int)threadIdx.x;
     const int c8 = tid & 3;
+    const int r = (tid >> 2) / kRuns, x = ((tid >> 2) - r * kRuns) * kRun;
+    const bf16_t* const h = hl + (r * kHaloCols + x) * PIXP + 8 * c8;
     float w[9][8];
 #pragma unroll
     for (int t = 0; t < 9; ++t)
@@ -352,26 +358,49 @@ __global__ __launch_bounds__(256) void k_sur_out(const bf16_t* H, const float* W
         halo.store(hl, PIXP);
         __syncthreads();
         halo.load(H, item + (int)gridDim.x, items);
-        for (int q = tid >> 2; q < kRowsPerItem * kCrop; q += 64) {
-            const int r = q / kCrop, x = q - r * kCrop;
-            const bf16_t* h = hl + (r * kHaloCols + x) * PIXP + 8 * c8;
-            float a0 = 0.0f, a1 = 0.0f;
+        float acc[kRun][2];
 #pragma unroll
-            for (int t = 0; t < 9; ++t) {
-                const u32x4 v = *reinterpret_cast<const u32x4*>(
-                    h + ((t / 3) * kHaloCols + t % 3) * PIXP);
+        for (int p = 0; p < kRun; ++p) acc[p][0] = acc[p][1] = 0.0f;
+        u32x4 v[2][3];      // a column of three rows, the next one requested ahead
+        auto column = [&](int c) {
+#pragma unroll
+            for (int ry = 0; ry < 3; ++ry)
+                v[c & 1][ry] = *reinterpret_cast<const u32x4*>(h + (ry * kHaloCols + c) * PIXP);
+        };
+        column(0);
+#pragma unroll
+        for (int c = 0; c < kRun + 2; ++c) {
+            if (c + 1 < kRun + 2) column(c + 1);
+#pragma unroll
+            for (int ry = 0; ry < 3; ++ry) {
 #pragma unroll
                 for (int k = 0; k < 4; ++k) {
-                    a0 = fmaf(w[t][2 * k], bf2f((bf16_t)(v[k] & 0xFFFFu)), a0);
-                    a1 = fmaf(w[t][2 * k + 1], bf2f((bf16_t)(v[k] >> 16)), a1);
+                    const uint32_t pair = v[c & 1][ry][k];
+                    const float f0 = bf2f((bf16_t)(pair & 0xFFFFu));
+                    const float f1 = bf2f((bf16_t)(pair >> 16));
+#pragma unroll
+                    for (int rx = 0; rx < 3; ++rx) {
+                        const int p = c - rx;
+                        if (p < 0 || p >= kRun) continue;
+                        acc[p][0] = fmaf(w[3 * ry + rx][2 * k], f0, acc[p][0]);
+                        acc[p][1] = fmaf(w[3 * ry + rx][2 * k + 1], f1, acc[p][1]);
+                    }
                 }
             }
-            float acc = a0 + a1;
-            acc += __shfl_xor(acc, 1, 64);
-            acc += __shfl_xor(acc, 2, 64);
-            if (c8 != 0) continue;
-            const size_t g = (size_t)crop * kCropPix + (size_t)(y0 + r) * kCrop + x;
-            const float d = acc + b4;
+            // the sums stay sums: not terms kept for later
+#pragma unroll
+            for (int p = 0; p < kRun; ++p)
+                asm volatile("" : "+v"(acc[p][0]), "+v"(acc[p][1]));
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int p = 0; p < kRun; ++p) {
+            float d = acc[p][0] + acc[p][1];
+            d += __shfl_xor(d, 1, 64);
+            d += __shfl_xor(d, 2, 64);
+            if (c8 != (p & 3)) continue;
+            const size_t g = (size_t)crop * kCropPix + (size_t)(y0 + r) * kCrop + x + p;
+            d += b4;
             if (dphi) dphi[g] = d;
             if (out) out[g] = phic[g] + d;
         }
