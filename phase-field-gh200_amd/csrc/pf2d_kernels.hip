@@ -841,7 +841,9 @@ struct Share {
 // kCheck: a check step (the surrogate's acceptance field), which needs the
 // new field and the cell's window position only: no scatter, moments,
 // support, flags or perimeter, and a commit of the position alone.
-template <int CLS, int NW, bool kCheck = false, bool kBatch = false, int kObs = 0>
+// kStream: the new field bypasses the caches (see kStreamBytes).
+template <int CLS, int NW, bool kCheck = false, bool kBatch = false, int kObs = 0,
+          bool kStream = false>
 __device__ void cell_walk(const pfh2d_step_args& A, int n, unsigned long long step, Smem& sm,
                           PFH_LDS float* win, Ctl& c, int nxt) {
     using G = Staged<CLS>;
@@ -1071,10 +1073,11 @@ __device__ void cell_walk(const pfh2d_step_args& A, int n, unsigned long long st
             if constexpr (kGen) {
                 uint32_t o = st + (uint32_t)k * kTileRow;
                 if (k >= G::RFULL) o = y0 + k < WY ? o : kOffNone;
-                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(pn), tst, (int)o, 0, 0);
+                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(pn), tst, (int)o, 0,
+                                                      kStream ? 2 : 0);
             } else {
                 __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(pn), tst, (int)st,
-                                                      (int)(k * kTileRow), 0);
+                                                      (int)(k * kTileRow), kStream ? 2 : 0);
             }
             if constexpr (!kCheck) {
                 // A lane whose destination is outside the window contributes
@@ -1432,7 +1435,7 @@ __device__ __noinline__ void cell_cold(const pfh2d_step_args* A, int n, unsigned
 // cells; each S slot one arena holding every replica's aggregate; the
 // clear-ahead sweeps the whole arena), and each cell's side, S pitch, S
 // offset and polarity stream come from its replica's record.
-template <int NW, bool kCheck, bool kBatch = false, int kObs = 0>
+template <int NW, bool kCheck, bool kBatch = false, int kObs = 0, bool kStream = false>
 __global__ __launch_bounds__(NW * kWave, 4) void k_step(const pfh2d_step_args A,
                                                         const int* run_if,
                                                         const pfh2d_replica* reps,
@@ -1485,8 +1488,8 @@ __global__ __launch_bounds__(NW * kWave, 4) void k_step(const pfh2d_step_args A,
         if (cls < 0) break;
         switch (cls) {
             case 0:
-                cell_walk<0, NW, kCheck, kBatch, kObs>(sm.args, n, step, sm, win,
-                                                       sm.slot[cur].ctl, cur ^ 1);
+                cell_walk<0, NW, kCheck, kBatch, kObs, kStream>(sm.args, n, step, sm, win,
+                                                                sm.slot[cur].ctl, cur ^ 1);
                 break;
             case 1: cell_cold<1, NW, kBatch, kObs>(&sm.args, n, step, &sm, win, cur); break;
             case 2: cell_cold<2, NW, kBatch, kObs>(&sm.args, n, step, &sm, win, cur); break;
@@ -2058,20 +2061,38 @@ int unsupported(const char* what) {
 using namespace pfh_host;
 
 namespace {
+// Both fields of the population (class-0 windows) against the 256 MB Infinity
+// Cache. While the step after this one finds the field there, its stores go
+// through the caches; larger populations store it non-temporally and leave the
+// cache to the aggregate. us per step, cached / non-temporal: 1024 cells (162
+// MiB) 80.7 / 82.1, 1536 (243 MiB) 115.9 / 114.4, 2048 161.4 / 155.6, 4096
+// 299.8 / 285.6; the line is where the two meet.
+constexpr size_t kStreamBytes = (size_t)208 << 20;
+constexpr size_t kCellFieldBytes =
+    2u * sizeof(float) * (size_t)pfh::kShapes[0].wx * (size_t)pfh::kShapes[0].wy;
+
 // grid compute units: two 8-wave workgroups on each when there are more
 // cells than compute units, one 16-wave workgroup each otherwise (a lone
 // cell then has the whole compute unit).
 template <bool kCheck, bool kBatch, int kObs>
 void launch_k_step(const pfh2d_step_args& a, const int* run_if, const pfh2d_replica* reps,
                    const uint16_t* cell_rep, int grid, void* stream) {
-    if (a.N > grid)
-        hipLaunchKernelGGL((pfh::k_step<8, kCheck, kBatch, kObs>), dim3(2u * (unsigned)grid),
-                           dim3(8 * pfh::kWave), 0, as_stream(stream), a, run_if, reps,
-                           cell_rep);
-    else
+    const dim3 pairs(2u * (unsigned)grid), threads8(8 * pfh::kWave);
+    if (a.N <= grid) {
         hipLaunchKernelGGL((pfh::k_step<16, kCheck, kBatch, kObs>), dim3((unsigned)grid),
                            dim3(16 * pfh::kWave), 0, as_stream(stream), a, run_if, reps,
                            cell_rep);
+        return;
+    }
+    if constexpr (!kCheck && kObs == 0) {
+        if ((size_t)a.N * kCellFieldBytes > kStreamBytes) {
+            hipLaunchKernelGGL((pfh::k_step<8, kCheck, kBatch, kObs, true>), pairs, threads8, 0,
+                               as_stream(stream), a, run_if, reps, cell_rep);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((pfh::k_step<8, kCheck, kBatch, kObs>), pairs, threads8, 0,
+                       as_stream(stream), a, run_if, reps, cell_rep);
 }
 }  // namespace
 

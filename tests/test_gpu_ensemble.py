@@ -102,6 +102,25 @@ def test_replica_equals_single_population_step():
     assert ens.replica_cells(1).tobytes() == lone.cells().tobytes()
 
 
+@pytest.mark.parametrize("counts", [(655, 659), (655, 660)])
+def test_large_batch_equals_lone_runs(counts):
+    """Ensembles on both sides of the line from which fields are stored
+    non-temporally: each replica equals its lone run, which is below it."""
+    from pfh import ensemble, sim2d
+    wls = [params.ensemble_replica(1536, n, 11 + k) for k, n in enumerate(counts)]
+    say(f"large batch: {sum(counts)} cells")
+    ens = ensemble.Ensemble2D(wls)
+    ens.step(3)
+    ens.sync()
+    for r, w in enumerate(wls):
+        lone = sim2d.Sim2D(w)
+        lone.step(3)
+        lone.sync()
+        assert np.array_equal(ens.replica_phi(r).view(np.uint32), lone.phi_now().view(np.uint32))
+        assert np.array_equal(ens.replica_S(r), lone.S_now())
+        assert ens.replica_cells(r).tobytes() == lone.cells().tobytes()
+
+
 def test_autotuned_ensemble_and_3d_shapes_keep_results():
     """The autotuner times every candidate and picks the fastest; the tuned
     ensemble order leaves every replica's state unchanged, and a tuned 3D

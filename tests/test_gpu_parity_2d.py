@@ -364,3 +364,17 @@ def test_workgroup_shapes_agree_on_every_class(sim_mod, oracle, grid, step0):
         sim.sync()
         assert_state_equal(sim, orc, f"grid {grid}, step {step0 + k + 1}")
     assert sim.cells()["shift_ctr"].sum() > 0
+
+
+@pytest.mark.parametrize("N", [1314, 1315])
+def test_both_sides_of_the_streaming_line(sim_mod, oracle, N):
+    """The largest population whose fields are stored through the caches and
+    the smallest one that stores them non-temporally, against the oracle."""
+    wl = params.monolayer(N, 2368, 20.0, 37, 4.0, 7)
+    say(f"field stores: {N} cells")
+    sim = sim_mod.Sim2D(wl)
+    orc = oracle.OracleSim2D(wl, threads=8)
+    sim.step(2)
+    orc.step(2)
+    sim.sync()
+    assert_state_equal(sim, orc, f"{N} cells, step 2")
