@@ -33,8 +33,8 @@ HIP_FLAGS = [
     "-I", str(REPO / "include"), "-I", str(CSRC),
 ]
 
-# Per-source additions. The 2D step kernel runs at the 128-VGPR limit of a
-# 1024-thread workgroup; sinking definitions towards their uses removes most
+# Per-source additions. The 2D step kernel runs at the 128-VGPR limit of
+# four waves on a SIMD; sinking definitions towards their uses removes most
 # of its scratch spills (each spill reload waits for every load in flight).
 FILE_FLAGS = {
     "pf2d_kernels.hip": ["-mllvm", "-sink-insts-to-avoid-spills"],

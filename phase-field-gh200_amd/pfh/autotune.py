@@ -1,6 +1,6 @@
 """Launch-shape autotuner: times candidate shapes of the 3D step (measurement
 shards per cell x update slabs per cell, i.e. the z extent of each
-workgroup's LDS plane ring) and the queue order of the batched 2D ensemble
+workgroup's walk) and the queue order of the batched 2D ensemble
 on the actual workload, with HIP events on the launch stream, and keeps the
 fastest. Results are cached per (device, workload signature) in memory and,
 when a cache path is given (or PFH_AUTOTUNE_CACHE is set), in a JSON file.
