@@ -2071,14 +2071,24 @@ constexpr size_t kStreamBytes = (size_t)208 << 20;
 constexpr size_t kCellFieldBytes =
     2u * sizeof(float) * (size_t)pfh::kShapes[0].wx * (size_t)pfh::kShapes[0].wy;
 
-// grid compute units: two 8-wave workgroups on each when there are more
-// cells than compute units, one 16-wave workgroup each otherwise (a lone
-// cell then has the whole compute unit).
+// grid compute units: two 8-wave workgroups on each, or one of 16 waves where a
+// cell would mostly be alone on its unit: no more cells than units, or three
+// rounds of them, which pairs would take as two rounds of which the second is
+// half empty. us per step, pairs / 16 waves: 560 cells on 256 units 62.0 / 49.9,
+// 640 66.7 / 52.9, 768 69.3 / 58.4; 1024 cells 79.5 / 82.6, 1280 88.9 / 93.1,
+// 1792 122.4 / 129.2, 4096 296 / 320: with more rounds the workgroups drift
+// apart and none is empty. (Two full rounds, 512 cells, are 44.7 / 42.2; the
+// smaller populations of two rounds were not compared and stay pairs.)
+bool one_cell_per_unit(int N, int grid) {
+    const long long rounds = ((long long)N + grid - 1) / grid;
+    return rounds <= 1 || rounds == 3;
+}
+
 template <bool kCheck, bool kBatch, int kObs>
 void launch_k_step(const pfh2d_step_args& a, const int* run_if, const pfh2d_replica* reps,
                    const uint16_t* cell_rep, int grid, void* stream) {
     const dim3 pairs(2u * (unsigned)grid), threads8(8 * pfh::kWave);
-    if (a.N <= grid) {
+    if (one_cell_per_unit(a.N, grid)) {
         hipLaunchKernelGGL((pfh::k_step<16, kCheck, kBatch, kObs>), dim3((unsigned)grid),
                            dim3(16 * pfh::kWave), 0, as_stream(stream), a, run_if, reps,
                            cell_rep);

@@ -340,11 +340,12 @@ def test_restart_equivalence(sim_mod):
     assert_cells_equal(a.cells(), c.cells(), "restart")
 
 
-@pytest.mark.parametrize("grid,step0", [(11, 99), (12, 99), (5, 98), (4, 99)])
+@pytest.mark.parametrize("grid,step0", [(11, 99), (12, 99), (5, 98), (4, 99), (3, 99), (2, 98)])
 def test_workgroup_shapes_agree_on_every_class(sim_mod, oracle, grid, step0):
     """Both sides of the launch rule on the forced state of 12 cells: fewer
     compute units than cells (two 8-wave workgroups each, two logical waves
-    per wave) and one for each cell (16 waves), with every window class,
+    per wave, or one of 16 waves at three rounds) and one for each cell (16
+    waves), with every window class,
     recentring shifts, class changes and the full-moment step 99 -> 100, whose
     perimeter is read back from the stored tile."""
     wl, phi, S, cells, cls = _forced_state(oracle)
