@@ -303,11 +303,16 @@ struct MeasureMode {
     int snapshot;       // copy cells -> accepted before committing
 };
 
+constexpr int kStripGroups = 128;        // 16 B groups of a wave's strip in LDS
 __global__ __launch_bounds__(1024) void k3_measure(const pfh3d_step_args a,
                                                    const MeasureMode m) {
+    // 2 KiB of strip for each wave of the launch (measure_lds), so that the
+    // one-wave workgroups of small bricks share a compute unit sixteen at a time
+    // (with room for sixteen waves in each workgroup only four fit: 4096 bricks of
+    // 8 41 us a launch, 21 this way; 4096 of 16, 71 and 45)
+    extern __shared__ __align__(16) float lds[];
     __shared__ double red[16][8];
     __shared__ int ired[16][7];
-    __shared__ f32x4 strip[16][128];
 
     const int B = a.B, S = a.shards, L = a.L, P = a.P;
     const int NT = (int)blockDim.x, tid = (int)threadIdx.x;
@@ -366,7 +371,7 @@ __global__ __launch_bounds__(1024) void k3_measure(const pfh3d_step_args a,
         const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(bin, (int)(o + zo), 0, 0);
         return __builtin_bit_cast(f32x4, v);
     };
-    f32x4* const mine4 = strip[tid >> 6];
+    f32x4* const mine4 = reinterpret_cast<f32x4*>(lds) + kStripGroups * (tid >> 6);
     f32x4* const w_own = mine4 + gpr + lane;
     f32x4* const w_halo = mine4 + (lane < gpr ? lane : 64 + lane);
     const f32x4* const r_ym = mine4 + (act ? lane : 127);
@@ -1503,6 +1508,9 @@ int block_threads(int B) {
     const int g = B * B / 4;
     return ((g + 63) / 64) * 64;
 }
+size_t measure_lds(int B) {
+    return (size_t)(block_threads(B) / 64) * pfh3::kStripGroups * sizeof(pfh3::f32x4);
+}
 // The update's y parts per slab: bricks from 32 split their rows in two, so
 // that a workgroup is at most 7 waves at B = 56 and two of them are resident
 // on a compute unit (one 13-wave workgroup otherwise): 208 against 212 us per
@@ -1544,7 +1552,8 @@ int launch_measure(const pfh3d_step_args* a, const pfh3::MeasureMode& m, void* s
     if (m.clear_out && !a->S_out) return invalid("S_out");
     if (m.snapshot && !a->accepted) return invalid("accepted");
     hipLaunchKernelGGL(pfh3::k3_measure, dim3((unsigned)(a->N * a->shards)),
-                       dim3((unsigned)block_threads(a->B)), 0, as_stream(stream), *a, m);
+                       dim3((unsigned)block_threads(a->B)), measure_lds(a->B),
+                       as_stream(stream), *a, m);
     return launch_status("k3_measure");
 }
 
