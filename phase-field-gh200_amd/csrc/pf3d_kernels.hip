@@ -1037,16 +1037,17 @@ __global__ __launch_bounds__(1024) void k3_update(const pfh3d_step_args a, const
     // yb + sy - 1 + tid / gpr (the part's rows as the shift reads them, with
     // one halo row on each side); element e of the group goes to sub-row e
     const int g = gx0 >> 2;
-    // (lanes past the workgroup's last in a second turn)
-    int srow[2], sg[2];
-    bool stg[2];
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-        const int i = tid + u * NT;
-        srow[u] = yb + sy - 1 + i / gpr;
-        sg[u] = i % gpr;
-        stg[u] = i < (ye - yb + 2) * gpr && (unsigned)srow[u] < (unsigned)B;
-    }
+    const int units = (ye - yb + 2) * gpr;
+    const int srow = yb + sy - 1 + tid / gpr, sg = tid % gpr;
+    const bool stg = tid < units && (unsigned)srow < (unsigned)B;
+    // Edges of 16, 32 and 64 have more groups than lanes: the first lanes own a
+    // second one, requested a plane ahead where the first has two. (A second
+    // group in every buffer, whatever the edge, took 12 registers and two
+    // spills: with every cell shifting, 512 bricks of 56 1271 us, 1242 this
+    // way, 1237 with a lane for every group; 2048 of 48 3356, 3255 and 3237.)
+    const bool two = units > NT;
+    const int srow2 = yb + sy - 1 + (tid + NT) / gpr, sg2 = (tid + NT) % gpr;
+    const bool stg2 = tid + NT < units && (unsigned)srow2 < (unsigned)B;
     // reading: destination group (gx0.., gy_) reads source x = gx0 + sx + c - 1,
     // c = 0..5, of rows gy_ + sy - 1..gy_ + sy + 1: sub-row (sx + c - 1) & 3,
     // group g + ((sx + c - 1) >> 2), both offsets uniform
@@ -1057,36 +1058,30 @@ __global__ __launch_bounds__(1024) void k3_update(const pfh3d_step_args a, const
         const int t = sx + c - 1;
         roff[c] = (t & 3) * GPU + (t >> 2);
     }
-    struct Groups { f32x4 g[2]; };
-    auto stage_plane = [&](float* plane, const Groups& v) {
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            if (!stg[u]) continue;
-            float* st = plane + (srow[u] + kMargin) * PXU + kMarginG + sg[u];
-            st[0] = v.g[u][0];
-            st[GPU] = v.g[u][1];
-            st[2 * GPU] = v.g[u][2];
-            st[3 * GPU] = v.g[u][3];
-        }
+    auto stage_plane = [&](float* plane, int row, int grp, const f32x4& v) {
+        float* st = plane + (row + kMargin) * PXU + kMarginG + grp;
+        st[0] = v[0];
+        st[GPU] = v[1];
+        st[2 * GPU] = v[2];
+        st[3 * GPU] = v[3];
     };
-    auto load_plane = [&](int p) -> Groups {
-        Groups v;
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            v.g[u] = f32x4{0.f, 0.f, 0.f, 0.f};
-            if (stg[u] && (unsigned)p < (unsigned)B)
-                v.g[u] = *reinterpret_cast<const PFH_GLOBAL f32x4*>(
-                    gsrc + (size_t)p * B * B + (size_t)srow[u] * B + 4 * sg[u]);
-        }
+    auto load_plane = [&](int p, bool own, int row, int grp) -> f32x4 {
+        f32x4 v = {0.f, 0.f, 0.f, 0.f};
+        if (own && (unsigned)p < (unsigned)B)
+            v = *reinterpret_cast<const PFH_GLOBAL f32x4*>(gsrc + (size_t)p * B * B +
+                                                          (size_t)row * B + 4 * grp);
         return v;
     };
 
     const int pbeg = zb + sz - 1;
     const int pcount = ze - zb + 2;
-    Groups R = load_plane(pbeg);
-    Groups Rn = load_plane(pbeg + 1);
+    const f32x4 R = load_plane(pbeg, stg, srow, sg);
+    f32x4 Rn = load_plane(pbeg + 1, stg, srow, sg);
+    f32x4 R2;
+    if (two) R2 = load_plane(pbeg, stg2, srow2, sg2);
     __syncthreads();
-    stage_plane(lds, R);
+    if (stg) stage_plane(lds, srow, sg, R);
+    if (two && stg2) stage_plane(lds, srow2, sg2, R2);
     __syncthreads();
 
     float T[4] = {0.f, 0.f, 0.f, 0.f}, Q1p[4] = {0.f, 0.f, 0.f, 0.f};
@@ -1135,7 +1130,9 @@ __global__ __launch_bounds__(1024) void k3_update(const pfh3d_step_args a, const
     for (int i = 0; i < pcount; ++i) {
         const int p = pbeg + i;
         const int cur = i & 1;
-        const Groups Rnn = load_plane(i + 2 < pcount ? p + 2 : -1);
+        f32x4 Rnn = {0.f, 0.f, 0.f, 0.f};
+        if (i + 2 < pcount) Rnn = load_plane(p + 2, stg, srow, sg);
+        if (two && i + 1 < pcount) R2 = load_plane(p + 1, stg2, srow2, sg2);
         float A[4] = {0.f, 0.f, 0.f, 0.f}, Q1[4] = {0.f, 0.f, 0.f, 0.f},
               Q0[4] = {0.f, 0.f, 0.f, 0.f}, GX[4] = {0.f, 0.f, 0.f, 0.f},
               GY[4] = {0.f, 0.f, 0.f, 0.f};
@@ -1210,7 +1207,11 @@ __global__ __launch_bounds__(1024) void k3_update(const pfh3d_step_args a, const
             gxm[j] = GX[j];
             gym[j] = GY[j];
         }
-        if (i + 1 < pcount) stage_plane(lds + (cur ^ 1) * PLU, Rn);
+        if (i + 1 < pcount) {
+            float* const next = lds + (cur ^ 1) * PLU;
+            if (stg) stage_plane(next, srow, sg, Rn);
+            if (two && stg2) stage_plane(next, srow2, sg2, R2);
+        }
         pfh::lds_barrier();   // the plane buffers are the only shared data here
         Rn = Rnn;
 #pragma unroll

@@ -62,3 +62,10 @@ def test_measurement_of_small_bricks_fills_a_compute_unit(kernels):
     measure, = _matching(kernels, "k3_measure")
     assert measure[".vgpr_count"] <= 128
     assert 16 * (measure[".group_segment_fixed_size"] + 2048) <= LDS_BYTES
+
+
+def test_update_keeps_its_planes_in_registers(kernels):
+    """No spills: a reload waits for every plane in flight. (Scratch that is
+    not a spill belongs to the out-of-line rare paths.)"""
+    update, = _matching(kernels, "k3_update")
+    assert update[".vgpr_spill_count"] == 0 and update[".sgpr_spill_count"] == 0
