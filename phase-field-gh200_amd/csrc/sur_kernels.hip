@@ -1451,7 +1451,10 @@ __global__ __launch_bounds__(256) void k_sur_check_cells(
 // Staged classes: each pixel thread walks its rows of one column (the update's
 // mapping), keeps the atomics' previous values in registers and tests them for
 // S_OVERFLOW after the loop, so no row waits for its scatter.
-template <int CLS>
+// kWhole: a column's chunks are unrolled, so that its reads go out early (96
+// registers, one workgroup a compute unit: see commit_whole, where both sides
+// were measured).
+template <int CLS, bool kWhole>
 __device__ void commit_staged(float* t, const float* pr, int L, int P, uint32_t* S, int gx0,
                               int gy0, int ox, int oy, pfh::MomentPart& mp, bool& ovf,
                               bool& clampf, const float* src = nullptr) {
@@ -1479,8 +1482,9 @@ __device__ void commit_staged(float* t, const float* pr, int L, int P, uint32_t*
                 ovf |= olds[k] >
                        0xFFFFFFFFu - pfh::q_of(t[(size_t)(y0 + k0 + k) * pfh::kTilePitch + x]);
     };
+    constexpr int kUnroll = kWhole ? (RB + CH - 1) / CH : 1;
     int k0 = 0;
-#pragma unroll 1
+#pragma unroll kUnroll
     for (; k0 < RB; k0 += CH) {
         // the chunk's values are read before any of its stores (the tile
         // written may be the buffer read, as far as the compiler knows), so
@@ -1520,11 +1524,11 @@ __device__ void commit_staged(float* t, const float* pr, int L, int P, uint32_t*
     test(k0 - CH);
 }
 
-__global__ __launch_bounds__(pfh::kNT, 8) void k_sur_commit(float* phi, pfh_cell_state* cells,
-                                                         const uint8_t* cls, const int* origin,
-                                                         const float* pred, int L, int P,
-                                                         uint32_t* S, uint32_t* flags,
-                                                         const int* skip_if) {
+// (the second argument: waves a SIMD at least, 8 for two workgroups a unit)
+template <bool kWhole>
+__global__ __launch_bounds__(pfh::kNT, kWhole ? 4 : 8) void k_sur_commit(
+    float* phi, pfh_cell_state* cells, const uint8_t* cls, const int* origin, const float* pred,
+    int L, int P, uint32_t* S, uint32_t* flags, const int* skip_if) {
     if (skip_if && *skip_if) return;
     const int n = (int)blockIdx.x;
     const int k = (int)cls[n];
@@ -1538,10 +1542,10 @@ __global__ __launch_bounds__(pfh::kNT, 8) void k_sur_commit(float* phi, pfh_cell
     if (k <= pfh::kClassStagedMax) {
         pfh::MomentPart mp = {0.0, 0.0, 0.0, sc.wx, -1, sc.wy, -1, 0};
         switch (k) {
-            case 0: commit_staged<0>(t, pr, L, P, S, gx0, gy0, ox, oy, mp, ovf, clampf); break;
-            case 1: commit_staged<1>(t, pr, L, P, S, gx0, gy0, ox, oy, mp, ovf, clampf); break;
-            case 2: commit_staged<2>(t, pr, L, P, S, gx0, gy0, ox, oy, mp, ovf, clampf); break;
-            default: commit_staged<3>(t, pr, L, P, S, gx0, gy0, ox, oy, mp, ovf, clampf); break;
+            case 0: commit_staged<0, kWhole>(t, pr, L, P, S, gx0, gy0, ox, oy, mp, ovf, clampf); break;
+            case 1: commit_staged<1, kWhole>(t, pr, L, P, S, gx0, gy0, ox, oy, mp, ovf, clampf); break;
+            case 2: commit_staged<2, kWhole>(t, pr, L, P, S, gx0, gy0, ox, oy, mp, ovf, clampf); break;
+            default: commit_staged<3, kWhole>(t, pr, L, P, S, gx0, gy0, ox, oy, mp, ovf, clampf); break;
         }
         m = pfh::reduce_moments(mp, sc.wx, sc.wy);
     } else {
@@ -1573,6 +1577,7 @@ __global__ __launch_bounds__(pfh::kNT, 8) void k_sur_commit(float* phi, pfh_cell
 // window position and class. Either way the field is written, q(phi) is
 // scattered into the zeroed aggregate and the moments are recomputed as in
 // k_sur_commit.
+template <bool kWhole>
 __device__ void commit_cell(
     int n, bool take, float* phi, pfh_cell_state* cells, uint8_t* cls, const int* origin,
     const float* pred, const float* phi_chk, const pfh_cell_state* cells_chk,
@@ -1598,10 +1603,10 @@ __device__ void commit_cell(
     if (k <= pfh::kClassStagedMax) {
         pfh::MomentPart mp = {0.0, 0.0, 0.0, sc.wx, -1, sc.wy, -1, 0};
         switch (k) {
-            case 0: commit_staged<0>(t, pr, L, P, S, gx0, gy0, ox, oy, mp, ovf, clampf, src); break;
-            case 1: commit_staged<1>(t, pr, L, P, S, gx0, gy0, ox, oy, mp, ovf, clampf, src); break;
-            case 2: commit_staged<2>(t, pr, L, P, S, gx0, gy0, ox, oy, mp, ovf, clampf, src); break;
-            default: commit_staged<3>(t, pr, L, P, S, gx0, gy0, ox, oy, mp, ovf, clampf, src); break;
+            case 0: commit_staged<0, kWhole>(t, pr, L, P, S, gx0, gy0, ox, oy, mp, ovf, clampf, src); break;
+            case 1: commit_staged<1, kWhole>(t, pr, L, P, S, gx0, gy0, ox, oy, mp, ovf, clampf, src); break;
+            case 2: commit_staged<2, kWhole>(t, pr, L, P, S, gx0, gy0, ox, oy, mp, ovf, clampf, src); break;
+            default: commit_staged<3, kWhole>(t, pr, L, P, S, gx0, gy0, ox, oy, mp, ovf, clampf, src); break;
         }
         m = pfh::reduce_moments(mp, sc.wx, sc.wy);
     } else {
@@ -1642,14 +1647,13 @@ __device__ void commit_cell(
     }
 }
 
-// (64 registers, so that two workgroups share a compute unit: 73 us for 1024
-// windows of 144 x 144 with one, 61 with two; 157 MB.)
-__global__ __launch_bounds__(pfh::kNT, 8) void k_sur_commit_cells(
+template <bool kWhole>
+__global__ __launch_bounds__(pfh::kNT, kWhole ? 4 : 8) void k_sur_commit_cells(
     float* phi, pfh_cell_state* cells, uint8_t* cls, const int* origin, const float* pred,
     const int* accept, const float* phi_chk, const pfh_cell_state* cells_chk,
     const uint8_t* cls_chk, int parity, int L, int P, uint32_t* S, uint32_t* flags) {
     const int n = (int)blockIdx.x;
-    commit_cell(n, accept[n] != 0, phi, cells, cls, origin, pred, phi_chk, cells_chk, cls_chk,
+    commit_cell<kWhole>(n, accept[n] != 0, phi, cells, cls, origin, pred, phi_chk, cells_chk, cls_chk,
                 parity, L, P, S, flags);
 }
 
@@ -2004,6 +2008,16 @@ int pfh_sur_check_cells(const float* phi_chk, const pfh_cell_state* cells_chk,
     return launch_status("k_sur_check_cells");
 }
 
+namespace {
+// A cell for each compute unit at most: its workgroup has the unit to itself
+// and holds whole columns in registers. More cells: two workgroups share a
+// unit, at 64 registers. us with the clearing of S, classes of 144 x 144, whole
+// / shared: commit_cells of 16 cells 16.0 / 21.3, 256 21.5 / 25.0, 257 29.3 /
+// 26.6, 1024 67.6 / 56.2; commit of 16 13.5 / 18.7, 256 18.8 / 21.2, 257 25.9 /
+// 24.7, 1024 51.0 / 50.2.
+bool commit_whole(int N) { return N <= sur_grid() / 2; }
+}  // namespace
+
 int pfh_sur_commit_cells(float* phi, pfh_cell_state* cells, uint8_t* cls, const int* origin,
                          const float* pred, const int* accept, const float* phi_chk,
                          const pfh_cell_state* cells_chk, const uint8_t* cls_chk, int parity,
@@ -2012,9 +2026,10 @@ int pfh_sur_commit_cells(float* phi, pfh_cell_state* cells, uint8_t* cls, const 
         !cls_chk || !S || !flags || N <= 0 || L < sur::kCrop || P < L || parity < 0 ||
         parity > 1)
         return invalid("sur_commit_cells");
-    hipLaunchKernelGGL(sur::k_sur_commit_cells, dim3((unsigned)N), dim3(pfh::kNT), 0,
-                       as_stream(stream), phi, cells, cls, origin, pred, accept, phi_chk,
-                       cells_chk, cls_chk, parity, L, P, S, flags);
+    auto* k = commit_whole(N) ? sur::k_sur_commit_cells<true> : sur::k_sur_commit_cells<false>;
+    hipLaunchKernelGGL(k, dim3((unsigned)N), dim3(pfh::kNT), 0, as_stream(stream), phi, cells,
+                       cls, origin, pred, accept, phi_chk, cells_chk, cls_chk, parity, L, P, S,
+                       flags);
     return launch_status("k_sur_commit_cells");
 }
 
@@ -2024,9 +2039,9 @@ int pfh_sur_commit(float* phi, pfh_cell_state* cells, const uint8_t* cls, const 
     if (!phi || !cells || !cls || !origin || !pred || !S || !flags || N <= 0 ||
         L < sur::kCrop || P < L)
         return invalid("sur_commit");
-    hipLaunchKernelGGL(sur::k_sur_commit, dim3((unsigned)N), dim3(pfh::kNT), 0,
-                       as_stream(stream), phi, cells, cls, origin, pred, L, P, S, flags,
-                       skip_if);
+    auto* k = commit_whole(N) ? sur::k_sur_commit<true> : sur::k_sur_commit<false>;
+    hipLaunchKernelGGL(k, dim3((unsigned)N), dim3(pfh::kNT), 0, as_stream(stream), phi, cells,
+                       cls, origin, pred, L, P, S, flags, skip_if);
     return launch_status("k_sur_commit");
 }
 

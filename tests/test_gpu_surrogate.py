@@ -709,3 +709,56 @@ def test_training_kernels_on_odd_batches(cin, crops, shift):
     for row in many.cpu().view(37, 289):
         acc = acc + row
     assert torch.equal(out.cpu(), acc)
+
+
+@pytest.mark.parametrize("per_cell", [False, True])
+def test_commit_in_one_call_equals_commit_in_parts(per_cell):
+    """A population of more cells than compute units and its halves of fewer
+    take different builds of the commit: the same fields, moments, aggregate
+    and flags, over every class, with zeros, a value beyond the clamp and a
+    NaN among the predictions, accepted and rejected cells."""
+    from pfh import abi
+    lib, dev = abi.load(), "cuda:0"
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    N, L, P, area = cus + 5, 1024, 1024, abi.TILE_AREA
+    rng = np.random.default_rng(17)
+    cells = np.zeros(N, abi.CELL_DTYPE)
+    cells["gx0"], cells["gy0"] = rng.integers(0, L, (2, N))
+    chk = cells.copy()
+    chk["gx0"], chk["gy0"] = (cells["gx0"] + 2) % L, (cells["gy0"] - 1) % L
+    cls, cls_chk = rng.integers(0, 6, (2, N)).astype(np.uint8)
+    centre = np.array([72, 88, 72, 80, 112, 143])[cls]
+    origin = np.stack([(cells["gx0"] + centre - 48) % L, (cells["gy0"] + centre - 48) % L], 1)
+    pred = (0.05 * rng.random((N, 9216))).astype(np.float32)
+    pred[:, ::7] = 0.0
+    pred[3, 100], pred[N - 3, 200] = 2.5, np.nan
+    accept = (rng.random(N) < 0.6).astype(np.int32)
+    phi = (0.02 * rng.random((N, area))).astype(np.float32)
+    phi_chk = (0.03 * rng.random((N, area))).astype(np.float32)
+    up = lambda a: torch.from_numpy(np.ascontiguousarray(a).view(np.uint8).reshape(-1)).to(dev)  # noqa: E731
+    fixed = [up(origin.astype(np.int32)), up(pred), up(accept), up(phi_chk), up(chk), up(cls_chk)]
+
+    def commit(parts):
+        d_phi, d_cells, d_cls = up(phi), up(cells), up(cls)
+        S = torch.zeros(L * P, dtype=torch.int32, device=dev)
+        flags = torch.zeros(abi.FLAG_COUNT, dtype=torch.int32, device=dev)
+        for lo, hi in parts:
+            at = lambda t: t.data_ptr() + lo * (t.numel() // N)                        # noqa: E731
+            og, pr, ac, pc, cc, kc = (at(t) for t in fixed)
+            if per_cell:
+                abi.check(lib.pfh_sur_commit_cells(
+                    at(d_phi), at(d_cells), at(d_cls), og, pr, ac, pc, cc, kc, 1, hi - lo, L, P,
+                    S.data_ptr(), flags.data_ptr(), None), "commit_cells")
+            else:
+                abi.check(lib.pfh_sur_commit(at(d_phi), at(d_cells), at(d_cls), og, pr, hi - lo,
+                                             L, P, S.data_ptr(), flags.data_ptr(), None, None),
+                          "commit")
+        return [t.cpu().numpy() for t in (d_phi, d_cells, d_cls, S, flags)]
+
+    say(f"commit of {N} cells on {cus} compute units, per cell: {per_cell}")
+    whole, parts = commit([(0, N)]), commit([(0, N // 2), (N // 2, N)])
+    assert all(np.array_equal(a, b) for a, b in zip(whole, parts))
+    assert whole[4].any()
+    V = whole[1].view(abi.CELL_DTYPE)["V"]
+    assert np.isnan(V).sum() == (1 if not per_cell or accept[N - 3] else 0)
+    assert (V[~np.isnan(V)] > 0.0).all()

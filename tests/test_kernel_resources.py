@@ -69,3 +69,14 @@ def test_update_keeps_its_planes_in_registers(kernels):
     not a spill belongs to the out-of-line rare paths.)"""
     update, = _matching(kernels, "k3_update")
     assert update[".vgpr_spill_count"] == 0 and update[".sgpr_spill_count"] == 0
+
+
+@pytest.mark.parametrize("kernel", ["k_sur_commitI", "k_sur_commit_cellsI"])
+def test_commit_has_a_build_for_each_population(kernels, kernel):
+    """Two 16-wave workgroups share a compute unit at 64 registers; the build
+    for populations that leave each workgroup a unit of its own is not held to
+    them. Neither spills."""
+    shared, = _matching(kernels, kernel + "Lb0E")
+    whole, = _matching(kernels, kernel + "Lb1E")
+    assert shared[".vgpr_count"] <= 64 < whole[".vgpr_count"] <= 128
+    assert shared[".vgpr_spill_count"] == whole[".vgpr_spill_count"] == 0
