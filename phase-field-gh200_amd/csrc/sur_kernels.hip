@@ -1082,13 +1082,14 @@ __global__ __launch_bounds__(64 * kWgWaves) void k_sur_wgrad(const bf16_t* dY, c
                 }
                 accb[0] = mfma(ae[0], ones, accb[0]);
                 accb[1] = mfma(ao[0], ones, accb[1]);
-            } else {
-                ae[0] = ao[0] = Frag{{0u, 0u, 0u, 0u}};
             }
             load_x();
             load_y();
 #pragma unroll
-            for (int ky = 0; ky < 3; ++ky)
+            for (int ky = 0; ky < 3; ++ky) {
+                // only where row r + 1 - ky of dY is this wave's: a zero in its
+                // place times a value of X that is not finite would be a NaN
+                if ((unsigned)(i - ky) >= (unsigned)kWgRows) continue;
 #pragma unroll
                 for (int f = 0; f < NF; ++f) {
                     f32x4* t = acc + (ky * NF + f) * 4;
@@ -1097,6 +1098,7 @@ __global__ __launch_bounds__(64 * kWgWaves) void k_sur_wgrad(const bf16_t* dY, c
                     t[2] = mfma(ao[ky], xe[f], t[2]);
                     t[3] = mfma(ao[ky], xo[f], t[3]);
                 }
+            }
         }
     }
 

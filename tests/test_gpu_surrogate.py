@@ -762,3 +762,38 @@ def test_commit_in_one_call_equals_commit_in_parts(per_cell):
     V = whole[1].view(abi.CELL_DTYPE)["V"]
     assert np.isnan(V).sum() == (1 if not per_cell or accept[N - 3] else 0)
     assert (V[~np.isnan(V)] > 0.0).all()
+
+
+@pytest.mark.parametrize("cin", [8, 32])
+def test_weight_gradient_of_values_that_are_not_finite(cin):
+    """Infinities and NaN among the inputs, in rows on every side of the edges
+    between the rows of two waves (12 rows each) and of the crop: an entry of
+    the gradient is infinite, NaN or finite exactly where the sum of its own
+    products is (finite ones within n 2^-24 of the sum of magnitudes, n fp32
+    terms)."""
+    from pfh import abi
+    lib, dev = abi.load(), "cuda:0"
+    gen = torch.Generator().manual_seed(cin)
+    X, dY = (_bf16(torch.randn(5, 96, 96, c, generator=gen)) for c in (cin, 32))
+    for n, (y, px, ch, v) in enumerate([(0, 3, 1, np.inf), (11, 95, 2, -np.inf), (12, 0, 3, np.inf),
+                                        (95, 32, 0, np.nan)]):
+        X[n, y, px, ch] = v
+    dY[4, 24, 31, 7] = np.inf
+    say(f"weight gradients of values that are not finite, {cin} channels")
+    width = 32 * 9 * cin + 32
+    part = torch.zeros(5 * width, dtype=torch.float32, device=dev)
+    dYd, Xd = dY.to(dev), X.to(dev)
+    abi.check(lib.pfh_sur_wgrad(cin, dYd.data_ptr(), Xd.data_ptr(), part.data_ptr(), 5, None),
+              "wgrad")
+    got = part.cpu().double().view(5, width)[:, :-32].reshape(5, 32, 9, cin)
+    p = torch.nn.functional.pad(X.double(), (0, 0, 1, 1, 1, 1))
+    taps = [p[:, ky:ky + 96, kx:kx + 96].reshape(5, 9216, cin) for ky in range(3) for kx in range(3)]
+    dy = dY.double().reshape(5, 9216, 32).transpose(1, 2).contiguous()
+    ref = torch.stack([torch.bmm(dy, t) for t in taps], 2)
+    mag = torch.stack([torch.bmm(dy.abs(), t.abs()) for t in taps], 2)
+    assert torch.equal(got.isnan(), ref.isnan())
+    assert torch.equal(got.isposinf(), ref.isposinf())
+    assert torch.equal(got.isneginf(), ref.isneginf())
+    ok = ref.isfinite()
+    assert 0 < int((~ok).sum()) < ok.numel() // 4
+    assert bool(((got - ref).abs()[ok] <= 9216 * 2.0 ** -24 * mag[ok]).all())
