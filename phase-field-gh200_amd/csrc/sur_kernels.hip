@@ -917,6 +917,16 @@ __global__ __launch_bounds__(kBwdNT) void k_sur_out_bwd(const float* g, const bf
             w[t][k] = W4[t * kCH + 4 * c4 + k];
             a[t][k] = 0.0f;
         }
+    // a weight that is not finite counts only where its tap lies in the crop
+    // (times the ring's zeros it would be a NaN): such a workgroup sums again,
+    // with the taps tested. The branch costs nothing (128 crops back to back
+    // 62 -> 55 us: it keeps the compiler from moving the next pixel's work up).
+    float z = 0.0f;
+#pragma unroll
+    for (int t = 0; t < 9; ++t)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) z = fmaf(w[t][k], 0.0f, z);
+    const bool odd = __any(z != 0.0f);
     __syncthreads();
     const bf16_t* Hn = H + (size_t)n * kCropPix * kCH;
     bf16_t* dHn = dH + (size_t)n * kCropPix * kCH;
@@ -939,6 +949,19 @@ __global__ __launch_bounds__(kBwdNT) void k_sur_out_bwd(const float* g, const bf
             for (int k = 0; k < 4; ++k) {
                 d[k] = fmaf(gv, w[t][k], d[k]);
                 a[t][k] = fmaf(gv, h[k], a[t][k]);
+            }
+        }
+        if (odd) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) d[k] = 0.0f;
+#pragma unroll
+            for (int t = 0; t < 9; ++t) {
+                if ((unsigned)(y + 1 - t / 3) >= (unsigned)kCrop ||
+                    (unsigned)(x + 1 - t % 3) >= (unsigned)kCrop)
+                    continue;
+                const float gv = gp[-(t / 3) * kHaloCols - t % 3];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) d[k] = fmaf(gv, w[t][k], d[k]);
             }
         }
 #pragma unroll

@@ -735,7 +735,8 @@ def test_commit_in_one_call_equals_commit_in_parts(per_cell):
     accept = (rng.random(N) < 0.6).astype(np.int32)
     phi = (0.02 * rng.random((N, area))).astype(np.float32)
     phi_chk = (0.03 * rng.random((N, area))).astype(np.float32)
-    up = lambda a: torch.from_numpy(np.ascontiguousarray(a).view(np.uint8).reshape(-1)).to(dev)  # noqa: E731
+    up = lambda a: torch.from_numpy(                                          # noqa: E731
+        np.ascontiguousarray(a).view(np.uint8).reshape(-1)).to(dev)
     fixed = [up(origin.astype(np.int32)), up(pred), up(accept), up(phi_chk), up(chk), up(cls_chk)]
 
     def commit(parts):
@@ -787,7 +788,8 @@ def test_weight_gradient_of_values_that_are_not_finite(cin):
               "wgrad")
     got = part.cpu().double().view(5, width)[:, :-32].reshape(5, 32, 9, cin)
     p = torch.nn.functional.pad(X.double(), (0, 0, 1, 1, 1, 1))
-    taps = [p[:, ky:ky + 96, kx:kx + 96].reshape(5, 9216, cin) for ky in range(3) for kx in range(3)]
+    taps = [p[:, ky:ky + 96, kx:kx + 96].reshape(5, 9216, cin)
+            for ky in range(3) for kx in range(3)]
     dy = dY.double().reshape(5, 9216, 32).transpose(1, 2).contiguous()
     ref = torch.stack([torch.bmm(dy, t) for t in taps], 2)
     mag = torch.stack([torch.bmm(dy.abs(), t.abs()) for t in taps], 2)
@@ -797,3 +799,44 @@ def test_weight_gradient_of_values_that_are_not_finite(cin):
     ok = ref.isfinite()
     assert 0 < int((~ok).sum()) < ok.numel() // 4
     assert bool(((got - ref).abs()[ok] <= 9216 * 2.0 ** -24 * mag[ok]).all())
+
+
+def test_output_gradient_of_weights_that_are_not_finite():
+    """Infinite and NaN weights of the output layer reach a pixel only through
+    a tap that lies in the crop: the gradient is infinite, NaN or finite
+    exactly where the sum of its own products is (finite ones within one bf16
+    rounding and the sums' 9 x 2^-24 of the magnitudes)."""
+    from pfh import abi
+    lib, dev = abi.load(), "cuda:0"
+    gen = torch.Generator().manual_seed(4)
+    g, W4 = torch.randn(2, 96, 96, generator=gen), torch.randn(9, 32, generator=gen)
+    H = _bf16(torch.randn(2, 96, 96, 32, generator=gen))
+    for t, ch, v in [(0, 3, np.inf), (8, 5, np.nan), (2, 7, -np.inf), (6, 7, np.inf),
+                     (4, 9, np.inf)]:
+        W4[t, ch] = v
+    say("output gradients of weights that are not finite")
+    dH = torch.zeros_like(H, device=dev)
+    part = torch.zeros(2 * 289, dtype=torch.float32, device=dev)
+    gd, Hd, Wd = g.to(dev), H.to(dev), W4.to(dev)
+    abi.check(lib.pfh_sur_out_bwd(gd.data_ptr(), Hd.data_ptr(), Wd.data_ptr(), dH.data_ptr(),
+                                  part.data_ptr(), 2, None), "out_bwd")
+    ref = torch.zeros(2, 96, 96, 32, dtype=torch.float64)
+    mag = torch.zeros_like(ref)
+    for t in range(9):
+        dy, dx = t // 3 - 1, t % 3 - 1                   # g at q - off(t)
+        q = (slice(None), slice(max(dy, 0), 96 + min(dy, 0)), slice(max(dx, 0), 96 + min(dx, 0)))
+        s = (slice(None), slice(max(-dy, 0), 96 + min(-dy, 0)),
+             slice(max(-dx, 0), 96 + min(-dx, 0)))
+        term = g.double()[s][..., None] * W4.double()[t]
+        ref[q] += term
+        mag[q] += term.abs()
+    on = H.double() > 0                                  # masked entries are exactly zero
+    ref, mag = torch.where(on, ref, 0.0), torch.where(on, mag, 0.0)
+    got = dH.cpu().double()
+    assert torch.equal(got.isnan(), ref.isnan())
+    assert torch.equal(got.isposinf(), ref.isposinf())
+    assert torch.equal(got.isneginf(), ref.isneginf())
+    ok = ref.isfinite()
+    lim = ref.abs() * 2.0 ** -8 + mag * (9 * 2.0 ** -24)
+    assert bool(((got - ref).abs()[ok] <= lim[ok]).all())
+    assert bool(ok[:, 95, :, 3].all()) and not bool(ok[:, :95, :95, 3].all())   # tap (0, 0)
