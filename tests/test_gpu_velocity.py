@@ -112,3 +112,33 @@ def test_dense_observer_matches_oracle_and_fused_rates(oracle):
         np.testing.assert_allclose(gd["q"][:, 4 + k] / dt, m["held"][:, k], rtol=1e-9,
                                    atol=1e-13)
     assert np.abs(c["Ix"]).max() > 1e-3
+
+
+@pytest.mark.parametrize("mode", [1, 2])
+@pytest.mark.parametrize("grid", [11, 5, 3, 2])
+def test_observers_on_every_workgroup_shape(oracle, grid, mode):
+    """The observed builds of both workgroup shapes on the forced state of 12
+    cells: two 8-wave workgroups a unit, each wave with two logical waves (11,
+    3 and 2 units), and one of 16 waves (5 units, three rounds). Steps 99 and
+    100, so that one is a full-moment step."""
+    from pfh import sim2d
+    wl, phi, S, cells, cls = _forced_state(oracle)
+    say(f"observer {mode} on {grid} compute units, 12 cells of every class")
+    sim = sim2d.Sim2D(wl)
+    sim.grid = grid
+    sim.attach_moments()
+    orc = oracle.OracleSim2D(wl, threads=8)
+    orc.observation = mode
+    sim.load_state(phi, S, cells, cls, 98)
+    orc.load_state(phi, S, cells, cls, 98)
+    for k in range(3):
+        sim.step(1, observation=mode)
+        orc.step(1)
+        sim.sync()
+        where = f"grid {grid}, step {99 + k}, observation {mode}"
+        assert_state_equal(sim, orc, where)
+        _adv_equal(sim.cells(), orc.cells, where)
+        assert np.array_equal(_bits(sim.moments_host()), _bits(orc.moments)), \
+            f"{where}: moment accumulators differ"
+    assert (sim.cells()["adv_count"] == 3).all()
+    assert (sim.moments_host()["spatial_count"] == (3 if mode == 2 else 0)).all()
