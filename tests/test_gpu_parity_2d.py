@@ -167,13 +167,13 @@ def test_all_classes_forced_paths_bit_exact(sim_mod, oracle, step0):
 
 @pytest.mark.parametrize("grid,step0", [(1, 0), (2, 99), (3, 5)])
 def test_few_workgroups_mixed_classes_bit_exact(sim_mod, oracle, grid, step0):
-    """The same forced state on 1-3 workgroups, so that each one takes several
-    cells of mixed classes in queue order: class-0 windows copied in ahead of
-    the next class-0 cell (and the slot of the double-buffered piece), the
-    switch to and from the out-of-line classes, and at step 99 the perimeter
-    pass of a full-moment step."""
+    """The same forced state on 1-3 compute units, so that each workgroup takes
+    several cells of mixed classes in queue order: the next cell's state
+    fetched during this one, one cell's commit under the next one's first
+    walk, the switch to and from the out-of-line classes, and at step 99 the
+    perimeter pass of a full-moment step."""
     wl, phi, S, cells, cls = _forced_state(oracle)
-    say(f"forced all-classes state L=701 N=12 on {grid} workgroup(s), start step {step0}")
+    say(f"forced all-classes state L=701 N=12 on {grid} compute unit(s), start step {step0}")
     sim = sim_mod.Sim2D(wl)
     sim.grid = grid
     orc = oracle.OracleSim2D(wl, threads=8)
@@ -187,10 +187,10 @@ def test_few_workgroups_mixed_classes_bit_exact(sim_mod, oracle, grid, step0):
 
 
 def test_c1_two_workgroups_bit_exact(sim_mod, oracle):
-    """C1's 16 class-0 cells on two workgroups: eight cells in a row per
-    workgroup, each window copied in during the previous cell."""
+    """C1's 16 class-0 cells on two compute units: several cells in a row per
+    workgroup, each fetched during the previous one."""
     wl = params.workload_c1()
-    say("C1 on 2 workgroups, 20 steps vs oracle")
+    say("C1 on 2 compute units, 20 steps vs oracle")
     sim = sim_mod.Sim2D(wl)
     sim.grid = 2
     orc = oracle.OracleSim2D(wl, threads=8)
@@ -379,3 +379,53 @@ def test_both_sides_of_the_streaming_line(sim_mod, oracle, N):
     orc.step(2)
     sim.sync()
     assert_state_equal(sim, orc, f"{N} cells, step 2")
+
+
+@pytest.mark.parametrize("grid", [8, 2, 256])
+def test_field_that_reaches_the_window_edge(sim_mod, oracle, grid):
+    """Fields that are nonzero in every row and column of their window, so
+    that the stencil of the rows past it is not zero either: the tile outside
+    the window stays untouched, in place and, a step later, across the class
+    changes that such a support asks for."""
+    p = params.SimParams(Nx=701, Ny=701, num_cells=9, rho=0.05, target_radius=20.0, seed=5,
+                         polarity_seed=6)
+    cx, cy = params.harness_centres(9, 701, 3, 6.0, 5)
+    wl = params.Workload2D("edges", p, cx, cy)
+    lib = oracle.load()
+    cls = np.array([0, 1, 2, 3, 4, 0, 3, 1, 2], np.uint8)
+    cells = oracle._host_cells(p, 9)
+    phi = [np.zeros((9, oracle.TILE_AREA), np.float32) for _ in range(2)]
+    lib.pfo2d_init_tiles(phi[0].ctypes.data, phi[1].ctypes.data, cells.ctypes.data,
+                         cls.ctypes.data, 9, 701, cx.ctypes.data, cy.ctypes.data,
+                         float(np.float32(p.init_radius())), float(np.float32(p.interface_k())))
+    rng = np.random.default_rng(9)
+    windows = [(144, 144, 64, 64), (176, 144, 32, 64), (144, 176, 64, 32), (160, 160, 32, 32),
+               (224, 224, 32, 32)]
+    inside = np.zeros((9, 288, 288), bool)
+    for n, c in enumerate(cls):
+        w, h, x0, y0 = windows[c]
+        inside[n, y0:y0 + h, x0:x0 + w] = True
+    tiles = phi[0].reshape(9, 288, 288)
+    tiles[inside] = (0.2 + 0.3 * rng.random(int(inside.sum()))).astype(np.float32)
+    lib.pfo2d_init_moments(cells.ctypes.data, cls.ctypes.data, phi[0].ctypes.data, 9, 0)
+    for lo, hi in (("bb_lo_x", "bb_hi_x"), ("bb_lo_y", "bb_hi_y")):
+        cells[lo], cells[hi] = 40, 90                       # the first step stays in its class
+    S = np.zeros(params.s_pitch_for(701) * 701, np.uint32)
+    flags = np.zeros(8, np.uint32)
+    lib.pfo2d_scatter_all(phi[0].ctypes.data, cells.ctypes.data, cls.ctypes.data, S.ctypes.data,
+                          9, 701, params.s_pitch_for(701), flags.ctypes.data)
+    say(f"fields up to the window's edge, 9 cells on {grid} compute units")
+    sim = sim_mod.Sim2D(wl)
+    sim.grid = grid
+    orc = oracle.OracleSim2D(wl, threads=8)
+    sim.load_state(phi[0], S, cells, cls, 98)
+    orc.load_state(phi[0], S, cells, cls, 98)
+    for k in range(3):
+        sim.step(1)
+        orc.step(1)
+        sim.sync()
+        if k == 0:
+            assert np.array_equal(sim.classes(), cls)
+            assert not sim.phi_now().reshape(9, 288, 288)[~inside].any()
+        assert_state_equal(sim, orc, f"grid {grid}, step {99 + k}")
+    assert not np.array_equal(sim.classes(), cls)
