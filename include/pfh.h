@@ -222,9 +222,9 @@ int pfh2d_configure_step(void);
  * LDS is static (sized for 16384 cells), so this only validates the size. */
 int pfh2d_configure_morton(int smem_bytes);
 /* Replaces k_step_grid(device) (include/kernels.cuh:221): the persistent
- * grid, the number of compute units (a step runs one 16-wave workgroup on each,
- * or two of 8 waves where it has more cells than that). Returns the grid size,
- * or a negative status. */
+ * grid, the number of compute units. A step runs one 16-wave workgroup on each
+ * where it has no more cells than that, or three rounds of them, and two of 8
+ * waves otherwise. Returns the grid size, or a negative status. */
 int pfh2d_step_grid(int device);
 
 /* Replaces launch_step (include/kernels.cuh:223-225, src/kernels.cu:1329-1363).

@@ -1,9 +1,9 @@
 // gfx950 kernels of the 2D per-cell phase-field update and their C ABI.
 //
 // The step is one persistent work-queue launch: two 8-wave workgroups per
-// compute unit (one of 16 waves when there are fewer cells) take cells from a
-// device cursor (reference step_body, src/kernels.cu:948-1024) and advance
-// one cell at a time through:
+// compute unit, or one of 16 waves where a cell would mostly be alone on its
+// unit (one_cell_per_unit), take cells from a device cursor (reference
+// step_body, src/kernels.cu:948-1024) and advance one cell at a time through:
 //   A  a column walk with a 3x3 register stencil over rows that each wave
 //      stages in LDS for itself; it gives the interaction integral terms and,
 //      for every pixel, the passive right-hand side, which stays in VGPRs;
@@ -16,8 +16,9 @@
 // Classes 0-3 take this walk; the rare classes 4 (224x224) and 5 (fallback)
 // read the tile from global memory.
 //
-// Arithmetic follows the reference's host semantics exactly: binary32
-// operations in source order with no multiply-add contraction (the build
+// Arithmetic: binary32 operations in the reference's order, each
+// product-and-add of the update fused by an explicit fmaf (passive_head_of,
+// with_repulsion, euler_update) and nothing contracted beyond that (the build
 // passes -ffp-contract=off), fp64 reductions, Q5.27 integer scatter.
 // Reference: process_cell src/kernels.cu:53-592, process_cell_fallback
 // :604-937, init/verify/pack/morton :1044-1302.
@@ -764,8 +765,9 @@ __device__ __forceinline__ float uni(float v) {
 }
 
 // Raw buffer descriptors: a byte offset at or past the end reads zeros and
-// stores nothing. One covers the rows of a tile that a window occupies, so
-// rows above and below the window need no test; kOffNone is past every one.
+// stores nothing; on gfx950 the scalar offset takes part in that test. One
+// covers the rows of a tile that a window occupies, so rows above and below the
+// window need no test; kOffNone is past every one.
 constexpr uint32_t kOffNone = 0x80000000u;
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc_of(const void* base, uint32_t bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, (int)bytes, 0x00020000);
@@ -2061,12 +2063,14 @@ int unsupported(const char* what) {
 using namespace pfh_host;
 
 namespace {
-// Both fields of the population (class-0 windows) against the 256 MB Infinity
-// Cache. While the step after this one finds the field there, its stores go
-// through the caches; larger populations store it non-temporally and leave the
-// cache to the aggregate. us per step, cached / non-temporal: 1024 cells (162
-// MiB) 80.7 / 82.1, 1536 (243 MiB) 115.9 / 114.4, 2048 161.4 / 155.6, 4096
-// 299.8 / 285.6; the line is where the two meet.
+// While the step after this one finds the field in the 256 MiB Infinity Cache,
+// its stores go through the caches; larger populations store it
+// non-temporally and leave the cache to the aggregate. us per step, cached /
+// non-temporal: 1024 cells (162 MiB for both fields) 80.7 / 82.1, 1536 (243 MiB)
+// 115.9 / 114.4, 2048 161.4 / 155.6, 4096 299.8 / 285.6. The line, 1314 cells, is
+// where the two differences interpolate to none. It counts class-0 windows for
+// every cell, and only class 0 has a body that streams: a population of larger
+// windows is stored through the caches whatever its size.
 constexpr size_t kStreamBytes = (size_t)208 << 20;
 constexpr size_t kCellFieldBytes =
     2u * sizeof(float) * (size_t)pfh::kShapes[0].wx * (size_t)pfh::kShapes[0].wy;
@@ -2074,11 +2078,19 @@ constexpr size_t kCellFieldBytes =
 // grid compute units: two 8-wave workgroups on each, or one of 16 waves where a
 // cell would mostly be alone on its unit: no more cells than units, or three
 // rounds of them, which pairs would take as two rounds of which the second is
-// half empty. us per step, pairs / 16 waves: 560 cells on 256 units 62.0 / 49.9,
-// 640 66.7 / 52.9, 768 69.3 / 58.4; 1024 cells 79.5 / 82.6, 1280 88.9 / 93.1,
-// 1792 122.4 / 129.2, 4096 296 / 320: with more rounds the workgroups drift
-// apart and none is empty. (Two full rounds, 512 cells, are 44.7 / 42.2; the
-// smaller populations of two rounds were not compared and stay pairs.)
+// half empty. us per step on 256 units, pairs / 16 waves, cells of radius 20 and
+// of radius 45 (larger classes among them):
+//    256  28.9 / 25.1   32.1 / 31.2      768  69.5 / 60.8   81.4 / 72.3
+//    288  38.5 / 36.4   40.7 / 41.6      896  74.6 / 71.1   86.6 / 84.4
+//    384  39.7 / 39.0   45.0 / 46.2     1024  75.9 / 76.5   90.6 / 96.2
+//    512  43.4 / 42.0   51.3 / 51.4     1280  94.5 / 101    113 / 119
+//    560  63.6 / 51.8   71.3 / 59.1     2048   149 / 159    174 / 189
+// Two rounds are pairs for the larger cells' sake; small ones lose 1 to 8% by
+// it, and four rounds of up to 900 cells 3 to 9%. The check step and the ensemble
+// behave as the plain step (check: 640 cells 51.0 / 42.5, 1024 57.3 / 58.4;
+// ensemble: 666 cells 72.0 / 59.6, 1155 91.1 / 97.3). The spatial observer does
+// not: its 8-wave build spills 49 registers where the other spills 10, and is
+// the slower one at every size (288 cells 72.3 / 58.4, 1024 141 / 120).
 bool one_cell_per_unit(int N, int grid) {
     const long long rounds = ((long long)N + grid - 1) / grid;
     return rounds <= 1 || rounds == 3;

@@ -353,7 +353,7 @@ __global__ __launch_bounds__(1024) void k3_measure(const pfh3d_step_args a,
     // memory, three. Bound by arithmetic and latency together: about 300
     // instructions a lane and plane, a third of them fp64, are 37 us of the
     // 64, and field, S words and clear, 224 MB, are 47 us at the rate of a
-    // copy.
+    // copy. 128 registers, the limit of a 16-wave workgroup, and 7 spilled.
     const uint32_t plane = 4u * (uint32_t)(B * B);
     const __amdgpu_buffer_rsrc_t bin =
         rsrc3(a.phi_in + (size_t)n * B * B * B, plane * (uint32_t)B);
@@ -1514,8 +1514,9 @@ size_t measure_lds(int B) {
 }
 // The update's y parts per slab: bricks from 32 split their rows in two, so
 // that a workgroup is at most 7 waves at B = 56 and two of them are resident
-// on a compute unit (one 13-wave workgroup otherwise): 208 against 212 us per
-// step at 256^3 / 128 cells.
+// on a compute unit (one 13-wave workgroup otherwise). us per step, two parts /
+// one, at the best number of slabs: 128 cells of 56 138.4 / 139.3, 224 of 64 332 /
+// 345, 8 of 48 43.6 / 45.5, 64 of 48 63.4 / 63.6, 128 of 40 65.9 / 65.2.
 int update_parts(int B) { return B >= 32 ? 2 : 1; }
 // a lane per 16 B group of a part's rows; the halo rows' groups are staged in a
 // second turn (as lanes of their own they made nine waves of eight at B = 64,
@@ -1570,9 +1571,10 @@ int pfh3d_update_slabs(int N, int B, int device) {
         "hipDeviceGetAttribute(multiProcessorCount)");
     if (st != PFH_OK) return st;
     // one full round of two resident workgroups per compute unit, counting
-    // the y parts of each slab: a partial round leaves part of the chip idle
-    // (at 128 cells, two parts: 2 slabs 208 us per step, 4 slabs 218, 8
-    // slabs 241); slabs of >= 4 planes
+    // the y parts of each slab: a partial round leaves part of the chip idle,
+    // and every slab reads two planes more (us per step, 1, 2, 4 and 8 slabs: 128
+    // cells of 56 163, 138, 148, 162, the rule 2; 64 of 48 105, 74, 63, 75, the rule
+    // 4; 224 of 64 346, 332, 343, 351, the rule 1); slabs of >= 4 planes
     int k = (2 * (cus > 0 ? cus : 1)) / (N * update_parts(B));
     if (k < 1) k = 1;
     if (k > B / 4) k = B / 4;
@@ -1629,7 +1631,7 @@ int pfh3d_update(const pfh3d_step_args* a, int slabs, void* stream) {
         if (k <= 0) return k;
     }
     if (k > a->B) return invalid("slabs must lie in [1, B]");
-    const size_t lds = update_lds(a->B);    // <= 46 KB: within the default 64 KB
+    const size_t lds = update_lds(a->B);    // 48,000 B at B = 64: within the default 64 KB
     const int H = update_parts(a->B);
     hipLaunchKernelGGL(pfh3::k3_update, dim3((unsigned)(a->N * k * H)),
                        dim3((unsigned)update_threads(a->B)), lds, as_stream(stream), *a, k, H);

@@ -893,7 +893,7 @@ __global__ __launch_bounds__(kLossNT) void k_sur_loss(const float* dphi, const f
 //   dW4[t][ci] += g[q - off(t)] h3[q][ci]        (36 sums in registers)
 // and the sums are added over the lanes (wave shuffles, then the 16 waves in
 // order). Bound by its 72 multiply-adds and the bf16 unpacking per four
-// channels: 128 crops 968 -> 58 us (before, a serial 96-term sum per entry and
+// channels: 128 crops 968 -> 52 us (before, a serial 96-term sum per entry and
 // row between two barriers, on 256 threads).
 constexpr int kBwdNT = 1024, kBwdWaves = kBwdNT / 64;
 __global__ __launch_bounds__(kBwdNT) void k_sur_out_bwd(const float* g, const bf16_t* H,
@@ -919,8 +919,8 @@ __global__ __launch_bounds__(kBwdNT) void k_sur_out_bwd(const float* g, const bf
         }
     // a weight that is not finite counts only where its tap lies in the crop
     // (times the ring's zeros it would be a NaN): such a workgroup sums again,
-    // with the taps tested. The branch costs nothing (128 crops back to back
-    // 62 -> 55 us: it keeps the compiler from moving the next pixel's work up).
+    // with the taps tested. The branch costs nothing (128 crops 58 -> 52 us: it
+    // keeps the compiler from moving the next pixel's work up).
     float z = 0.0f;
 #pragma unroll
     for (int t = 0; t < 9; ++t)
@@ -1009,9 +1009,10 @@ __global__ __launch_bounds__(kBwdNT) void k_sur_out_bwd(const float* g, const bf
 // 12 w .. 12 w + 11, one 32-pixel block after the other, with the next row's
 // loads in flight; db is the product with a fragment of ones. The waves' sums
 // are added in order through LDS. MFMA-bound by design (36 products a row and
-// block); measured for 128 crops: 32 channels 339 -> 44 us
-// (0.49 PFLOP/s on half the compute units), 8 channels 224 -> 34 us (before, every operand was transposed into LDS by 2 B stores
-// between two barriers a row).
+// block); measured for 128 crops: 32 channels 339 -> 41 us
+// (0.53 PFLOP/s on half the compute units), 8 channels 224 -> 35 us (before,
+// every operand was transposed into LDS by 2 B stores between two barriers a
+// row).
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 constexpr int kWgWaves = 8, kWgRows = kCrop / kWgWaves;
 
