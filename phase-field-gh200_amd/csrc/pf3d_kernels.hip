@@ -346,14 +346,14 @@ __global__ __launch_bounds__(1024) void k3_measure(const pfh3d_step_args a,
     // y + 1 and the words beside the group there. No wave waits for another:
     // with a ring of planes that all waves share, the barrier of every plane
     // left the arithmetic idle (128 bricks of 56, two shards: 90 -> 72 us a
-    // launch, and 64 with the reduction below; neighbours read from cache
+    // launch, and 61 with the reduction and the test below; neighbours read from cache
     // instead cost more L2 traffic than the halo, 118 us). A buffer descriptor
     // over the cube gives the zeros around it. The halo and the S words are
     // requested one plane ahead, the lane's own group, which comes from
     // memory, three. Bound by arithmetic and latency together: about 300
     // instructions a lane and plane, a third of them fp64, are 37 us of the
-    // 64, and field, S words and clear, 224 MB, are 47 us at the rate of a
-    // copy. 128 registers, the limit of a 16-wave workgroup, and 7 spilled.
+    // 61, and field, S words and clear, 224 MB, are 47 us at the rate of a
+    // copy. 119 registers of the 128 that a 16-wave workgroup may have, no spills.
     const uint32_t plane = 4u * (uint32_t)(B * B);
     const __amdgpu_buffer_rsrc_t bin =
         rsrc3(a.phi_in + (size_t)n * B * B * B, plane * (uint32_t)B);
@@ -421,7 +421,7 @@ __global__ __launch_bounds__(1024) void k3_measure(const pfh3d_step_args a,
     int lo2 = B, hi2 = -1;
 
     // Voxel j of plane z; every sum takes its terms in the reference's order.
-    // (An empty voxel adds zeros only: no test for it.)
+    // (An empty voxel adds zeros only: no test for it but the wave's below.)
     auto voxel = [&](double xd, double zd, float c, float gx, float gy, float gz,
                      uint32_t agg) {
         // other_field (src/pf3d/device_common.cuh:182-191), its S_NEGATIVE
@@ -468,41 +468,53 @@ __global__ __launch_bounds__(1024) void k3_measure(const pfh3d_step_args a,
             gy[j] = 0.5f * (Yp[j] - Ym[j]);
             gz[j] = 0.5f * (Ap[j] - Am[j]);
         }
-        // A value that is not finite is counted and adds nothing (zeros); one
-        // test per wave. (A neighbour's shows in the sums as it always did.)
-        f32x4 c = A0;
-        const float all = (A0[0] + A0[1]) + (A0[2] + A0[3]);
-        if (wave_any(!(fabsf(all) < INFINITY))) {
+        // A wave whose voxels are all empty, without a gradient, adds zeros only
+        // and is done (every bit zero, so that no -0 is taken for empty): 4096
+        // bricks of 16 with a field of 6 voxels' radius 45 -> 42 us. The branch
+        // also keeps the compiler from carrying a plane's values into the next
+        // (7 registers spilled without it): 128 bricks of 56 64 -> 61 us.
+        uint32_t bits = 0u;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const bool bad = !isfinite(c[j]);
-                n_nonfin += bad ? 1u : 0u;
-                c[j] = bad ? 0.0f : c[j];
-                gx[j] = bad ? 0.0f : gx[j];
-                gy[j] = bad ? 0.0f : gy[j];
-                gz[j] = bad ? 0.0f : gz[j];
+        for (int j = 0; j < 4; ++j)
+            bits |= __float_as_uint(A0[j]) | __float_as_uint(gx[j]) | __float_as_uint(gy[j]) |
+                    __float_as_uint(gz[j]);
+        if (wave_any(bits != 0u)) {
+            // A value that is not finite is counted and adds nothing (zeros); one
+            // test per wave. (A neighbour's shows in the sums as it always did.)
+            f32x4 c = A0;
+            const float all = (A0[0] + A0[1]) + (A0[2] + A0[3]);
+            if (wave_any(!(fabsf(all) < INFINITY))) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const bool bad = !isfinite(c[j]);
+                    n_nonfin += bad ? 1u : 0u;
+                    c[j] = bad ? 0.0f : c[j];
+                    gx[j] = bad ? 0.0f : gx[j];
+                    gy[j] = bad ? 0.0f : gy[j];
+                    gz[j] = bad ? 0.0f : gz[j];
+                }
             }
-        }
-        uint64_t hit = 0ull;
-        const double zd = (double)z;
-        double xd = xd0;      // x0 + j, not four registers pairs over the walk
-        asm volatile("" : "+v"(xd));
+            uint64_t hit = 0ull;
+            const double zd = (double)z;
+            double xd = xd0;      // x0 + j, not four registers pairs over the walk
+            asm volatile("" : "+v"(xd));
 #pragma unroll
-        for (int j = 0; j < 4; ++j, xd += 1.0) {
-            voxel(xd, zd, c[j], gx[j], gy[j], gz[j], Sz[j]);
-            const uint64_t in = __builtin_amdgcn_ballot_w64(fabsf(c[j]) > kEps);
-            sup[j] |= in;
-            hit |= in;
-        }
-        if (surface) {
+            for (int j = 0; j < 4; ++j, xd += 1.0) {
+                voxel(xd, zd, c[j], gx[j], gy[j], gz[j], Sz[j]);
+                const uint64_t in = __builtin_amdgcn_ballot_w64(fabsf(c[j]) > kEps);
+                sup[j] |= in;
+                hit |= in;
+            }
+            if (surface) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
-                aS += sqrt((double)gx[j] * (double)gx[j] + (double)gy[j] * (double)gy[j] +
-                           (double)gz[j] * (double)gz[j]);
-        }
-        if (hit) {
-            lo2 = min(lo2, z);
-            hi2 = z;
+                for (int j = 0; j < 4; ++j)
+                    aS += sqrt((double)gx[j] * (double)gx[j] + (double)gy[j] * (double)gy[j] +
+                               (double)gz[j] * (double)gz[j]);
+            }
+            if (hit) {
+                lo2 = min(lo2, z);
+                hi2 = z;
+            }
         }
         Am = A0;
         A0 = Ap;

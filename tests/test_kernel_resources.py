@@ -64,11 +64,12 @@ def test_measurement_of_small_bricks_fills_a_compute_unit(kernels):
     assert 16 * (measure[".group_segment_fixed_size"] + 2048) <= LDS_BYTES
 
 
-def test_update_keeps_its_planes_in_registers(kernels):
+@pytest.mark.parametrize("kernel", ["k3_measure", "k3_update"])
+def test_planes_stay_in_registers(kernels, kernel):
     """No spills: a reload waits for every plane in flight. (Scratch that is
     not a spill belongs to the out-of-line rare paths.)"""
-    update, = _matching(kernels, "k3_update")
-    assert update[".vgpr_spill_count"] == 0 and update[".sgpr_spill_count"] == 0
+    k, = _matching(kernels, kernel)
+    assert k[".vgpr_spill_count"] == 0 and k[".sgpr_spill_count"] == 0
 
 
 @pytest.mark.parametrize("kernel", ["k_sur_commitI", "k_sur_commit_cellsI"])
